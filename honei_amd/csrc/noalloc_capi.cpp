@@ -34,7 +34,7 @@ constexpr size_t kPartialBytes = sizeof(double) * (size_t)Workspace::kSlotCapaci
 constexpr size_t kCounterOff = kPartialBytes;
 constexpr size_t kScalarOff = kPartialBytes + 256;
 constexpr size_t kVectorOff = kPartialBytes + 4096;
-constexpr size_t kVectorBytes = (size_t)32 << 20;   // p, r and v together
+constexpr size_t kVectorBytes = (size_t)32 << 20;   // p, r and v together (small systems: two more)
 constexpr size_t kScratchBytes = kVectorOff + kVectorBytes;
 constexpr int kMaxDevices = 64;
 
@@ -106,7 +106,8 @@ int honei_hip_cg_solve_noalloc(int vtype, const void *Aj, const void *Ax, const 
     const EllView A = cg_view(vtype, Aj, Ax, Arl, rows, num_cols_per_row, stride, threads);
     char *v0 = base + kVectorOff;
     return cg_solve_on(A, b, x, max_iters, eps_relative, used_iters, final_defect, s, slots, v0, v0 + vbytes,
-                       v0 + 2 * vbytes, (CGScalars *)(base + kScalarOff));
+                       v0 + 2 * vbytes, cg_resident_fits(A) && 5 * vbytes <= kVectorBytes ? v0 + 3 * vbytes : nullptr,
+                       (CGScalars *)(base + kScalarOff));
 }
 
 }  // extern "C"

@@ -135,6 +135,7 @@ __global__ void k_cg_init(CGScalars *sc, double eps_rel, int max_iters) {
         sc->iters = 0;
         sc->max_iters = max_iters;
         sc->done = max_iters <= 0 ? 1 : 0;
+        sc->aborted = 0;
     }
 }
 
@@ -176,6 +177,7 @@ __global__ void k_pcg_init(const double *partials, int64_t nparts, CGScalars *sc
         sc->max_iters = max_iters;
         sc->done = max_iters <= 0 ? 1 : 0;
         sc->converged = 0;
+        sc->aborted = 0;
     }
 }
 

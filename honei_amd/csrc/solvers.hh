@@ -27,6 +27,7 @@ struct CGScalars {
     // block 0 writes the next one)
     double carry[2];
     int done, iters, max_iters, converged;   // converged: set by the PCG-Jacobi test only
+    int aborted;                             // a resident launch gave up waiting (cg_resident)
 };
 
 hipError_t cg_init(ValueType vt, CGScalars *sc, double eps_rel, int max_iters, hipStream_t s);
@@ -59,7 +60,8 @@ hipError_t mgpcg_pupdate(double *p, const double *z, int64_t n, const MgPcgScala
 // Host side of CGSolver (solvers_capi.cpp), shared by honei_hip_cg_solve and
 // its allocation-free variant: argument checks (HONEI status code), the
 // bytes of one CG vector (256-byte multiple), the matrix view, and the solve
-// on caller-provided vectors p, r, v, scalars and reduction slots.
+// on caller-provided vectors p, r, v, two vectors at pub (or null: no
+// resident launches), scalars and reduction slots.
 int cg_check_args(int vtype, const void *Aj, const void *Ax, const void *Arl, size_t rows, size_t stride,
                   size_t threads, const void *b, const void *x);
 size_t cg_vector_bytes(ValueType vt, size_t rows);
@@ -67,7 +69,7 @@ EllView cg_view(int vtype, const void *Aj, const void *Ax, const void *Arl, size
                 size_t stride, size_t threads);
 int cg_solve_on(const EllView &A, const void *b, void *x, size_t max_iters, double eps_relative, size_t *used_iters,
                 double *final_defect, hipStream_t s, const ReduceSlots &slots, void *p, void *r, void *v,
-                CGScalars *sc);
+                void *pub, CGScalars *sc);
 // Device address of the allocation-free variant's fixed scratch on the
 // current device (looked up once per device); HONEI status code.
 int noalloc_setup(void **out);
@@ -82,6 +84,30 @@ hipError_t pcg_start(ValueType vt, void *d, const void *r, const void *dinv, int
                      double eps_rel, int max_iters, const ReduceSlots &sl, hipStream_t s);
 hipError_t pcg_iteration(const EllView &A, void *x, void *d, void *r, void *t0, const void *dinv, CGScalars *sc,
                          const ReduceSlots &sl, int it, hipStream_t s);
+// Iterations it_begin .. it_end - 1 (or until the solve is over) in one
+// launch (cg_resident.hip); dinv null: CG, else PCG-Jacobi.  Expects what the
+// first iteration above expects in p, r and sc; xin is x (first launch) or
+// xs, pub0 and pub1 vectors of scratch.  x receives the result once the
+// solve is over.  sc->aborted set: x is untouched and the launches above have
+// to run, from the start.  Same bits as cg_iteration / pcg_iteration.
+// The lease (held while its launches run) says whether A fits and bounds the
+// resident work-groups per device; without one the launches above run.
+constexpr int kResidentIters = 4096;   // iterations per launch at most
+bool cg_resident_fits(const EllView &A);   // by layout and size
+class ResidentLease {
+  public:
+    ResidentLease(const EllView &A, const ReduceSlots &slots);
+    ~ResidentLease();
+    ResidentLease(const ResidentLease &) = delete;
+    ResidentLease &operator=(const ResidentLease &) = delete;
+    explicit operator bool() const { return count_ > 0; }
+
+  private:
+    int dev_ = 0, count_ = 0;
+};
+hipError_t cg_resident(const EllView &A, const void *dinv, const void *xin, void *x, void *xs, void *p, void *r,
+                       void *pub0, void *pub1, CGScalars *sc, const ReduceSlots &sl, int it_begin, int it_end,
+                       hipStream_t s);
 hipError_t coarse_cg(const EllView &A, const void *rhs, void *x, void *g, void *u, void *en, double konv,
                      int max_iters, int *iters_dev, hipStream_t s);
 hipError_t boundary_guess(double *guess, const double *b, int64_t n, int64_t side, hipStream_t s);

@@ -2,6 +2,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -54,6 +55,42 @@ int upload_ell(DevEll &M, ValueType vt, size_t rows, size_t cols, size_t stride,
     return check(hipMemcpy(M.Ax, Ax, size * vt_size(vt), hipMemcpyHostToDevice), "ELL value upload");
 }
 
+// The iteration loop of CG and PCG-Jacobi: resident launches where the
+// system fits and the device has room for them, else (or when one gave up
+// waiting) single iterations enqueued in chunks with one flag read per chunk.
+template <class Start, class Iterate, class Resident>
+int run_iterations(const EllView &A, bool may_stay, const ReduceSlots &slots, CGScalars *sc, size_t max_iters, hipStream_t s,
+                   Start &&start, Iterate &&iterate, Resident &&resident, CGScalars &h) {
+    auto read_back = [&]() -> int {
+        if (int st = check(hipMemcpyAsync(&h, sc, sizeof(CGScalars), hipMemcpyDeviceToHost, s), "cg readback"))
+            return st;
+        return check(hipStreamSynchronize(s), "cg sync");
+    };
+    if (int st = start()) return st;
+    if (may_stay && max_iters > 0) {
+        const ResidentLease lease(A, slots);
+        if (lease) {
+            for (size_t it = 0; it < max_iters; it += kResidentIters) {
+                const size_t end = std::min(max_iters, it + (size_t)kResidentIters);
+                if (int st = resident((int)it, (int)end)) return st;
+                if (int st = read_back()) return st;
+                if (h.done || h.aborted) break;
+            }
+            if (!h.aborted) return HONEI_HIP_SUCCESS;
+            if (int st = start()) return st;
+        }
+    }
+    size_t chunk = A.rows < 100000 ? 16 : 4, enqueued = 0;
+    while (true) {
+        for (size_t k = 0; k < chunk && enqueued < max_iters; ++k, ++enqueued)
+            if (int st = iterate((int)enqueued)) return st;
+        if (int st = read_back()) return st;
+        if (h.done || enqueued >= max_iters) break;
+        if (chunk < 64) chunk *= 2;
+    }
+    return HONEI_HIP_SUCCESS;
+}
+
 }  // namespace
 
 namespace honei {
@@ -87,40 +124,38 @@ EllView cg_view(int vtype, const void *Aj, const void *Ax, const void *Arl, size
     return A;
 }
 
-// CGSolver<Tag, NONE> (math/cg.hh:63-133) with p, r, v and the scalars in
-// caller-provided device memory and the reductions in `slots`.
+// CGSolver<Tag, NONE> (math/cg.hh:63-133) with p, r, v, the published vectors
+// and the scalars in caller-provided device memory, the reductions in `slots`.
 int cg_solve_on(const EllView &A, const void *b, void *x, size_t max_iters, double eps_relative, size_t *used_iters,
                 double *final_defect, hipStream_t s, const ReduceSlots &slots, void *p, void *r, void *v,
-                CGScalars *sc) {
+                void *pub, CGScalars *sc) {
     if (max_iters > 0x7fffffff) max_iters = 0x7fffffff;
     const size_t rows = (size_t)A.rows;
     const ValueType vv = A.vtype == VT_F64 ? VT_F64 : VT_F32;
     // r = b - A x ; p = r ; alpha = ||r||^2 (math/cg.hh:90-95)
-    EllArgs a;
-    a.mode = ELL_DEFECT;
-    a.out = r;
-    a.x = x;
-    a.rhs = b;
-    a.norm2 = &sc->alpha;
-    a.row_start = 0;
-    a.row_end = (int64_t)rows;
-    int st = check(ell_apply(A, a, slots, s), "cg defect");
-    if (st) return st;
-    if ((st = check(vcopy(p, r, (int64_t)rows, vv, s), "cg copy"))) return st;
-    if ((st = check(cg_init(vv, sc, eps_relative, (int)max_iters, s), "cg init"))) return st;
-    // enqueue iterations in chunks; one flag read per chunk
+    auto start = [&]() -> int {
+        EllArgs a;
+        a.mode = ELL_DEFECT;
+        a.out = r;
+        a.x = x;
+        a.rhs = b;
+        a.norm2 = &sc->alpha;
+        a.row_start = 0;
+        a.row_end = (int64_t)rows;
+        if (int st = check(ell_apply(A, a, slots, s), "cg defect")) return st;
+        if (int st = check(vcopy(p, r, (int64_t)rows, vv, s), "cg copy")) return st;
+        return check(cg_init(vv, sc, eps_relative, (int)max_iters, s), "cg init");
+    };
     CGScalars h{};
-    size_t chunk = rows < 100000 ? 16 : 4;
-    size_t enqueued = 0;
-    while (true) {
-        for (size_t k = 0; k < chunk && enqueued < max_iters; ++k, ++enqueued)
-            if ((st = check(cg_iteration(A, x, p, r, v, sc, slots, (int)enqueued, s), "cg iteration"))) return st;
-        if ((st = check(hipMemcpyAsync(&h, sc, sizeof(CGScalars), hipMemcpyDeviceToHost, s), "cg readback")))
-            return st;
-        if ((st = check(hipStreamSynchronize(s), "cg sync"))) return st;
-        if (h.done || enqueued >= max_iters) break;
-        if (chunk < 64) chunk *= 2;
-    }
+    auto iterate = [&](int it) {
+        return check(cg_iteration(A, x, p, r, v, sc, slots, it, s), "cg iteration");
+    };
+    auto resident = [&](int begin, int end) {
+        return check(cg_resident(A, nullptr, begin ? v : x, x, v, p, r, pub, (char *)pub + cg_vector_bytes(A.vtype, rows),
+                                 sc, slots, begin, end, s),
+                     "cg resident");
+    };
+    if (int st = run_iterations(A, pub != nullptr, slots, sc, max_iters, s, start, iterate, resident, h)) return st;
     if (used_iters) *used_iters = (size_t)h.iters;
     if (final_defect) *final_defect = h.current;
     if (!h.done && max_iters > 0) return fail(HONEI_HIP_ERROR_NOT_CONVERGED, "CG did not converge");
@@ -144,11 +179,14 @@ int honei_hip_cg_solve(int vtype, const void *Aj, const void *Ax, const void *Ar
     Workspace *w = workspace_for(S(stream));
     if (!w) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
     const size_t vbytes = cg_vector_bytes((ValueType)vtype, rows);
-    char *base = (char *)w->ensure_scratch(3 * vbytes + 256);
-    if (!base) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
     const EllView A = cg_view(vtype, Aj, Ax, Arl, rows, num_cols_per_row, stride, threads);
+    const bool fits = cg_resident_fits(A);
+    const size_t vectors = fits ? 5 : 3;
+    char *base = (char *)w->ensure_scratch(vectors * vbytes + 256);
+    if (!base) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
     return cg_solve_on(A, b, x, max_iters, eps_relative, used_iters, final_defect, S(stream), w->slots, base,
-                       base + vbytes, base + 2 * vbytes, (CGScalars *)(base + 3 * vbytes));
+                       base + vbytes, base + 2 * vbytes, fits ? base + 3 * vbytes : nullptr,
+                       (CGScalars *)(base + vectors * vbytes));
 }
 
 int honei_hip_pcg_jacobi(int vtype, const void *Aj, const void *Ax, const void *Arl, size_t rows,
@@ -166,50 +204,40 @@ int honei_hip_pcg_jacobi(int vtype, const void *Aj, const void *Ax, const void *
     const ValueType vt = (ValueType)vtype;
     const size_t es = vec_size(vt);
     const size_t vbytes = ((rows * es + 255) / 256) * 256;
-    char *base = (char *)w->ensure_scratch(3 * vbytes + 256);
+    const EllView A = cg_view(vtype, Aj, Ax, Arl, rows, num_cols_per_row, stride, threads);
+    const bool fits = cg_resident_fits(A);
+    const size_t vectors = fits ? 5 : 3;
+    char *base = (char *)w->ensure_scratch(vectors * vbytes + 256);
     if (!base) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
     void *d = base, *r = base + vbytes, *t0 = base + 2 * vbytes;
-    CGScalars *sc = (CGScalars *)(base + 3 * vbytes);
-    EllView A;
-    A.rows = (int64_t)rows;
-    A.cols = (int64_t)rows;
-    A.stride = (int64_t)stride;
-    A.ncpr = (int64_t)num_cols_per_row;
-    A.threads = (int)threads;
-    A.Aj = (const int32_t *)Aj;
-    A.Ax = Ax;
-    A.Arl = (const uint32_t *)Arl;
-    A.vtype = vt;
+    char *pub = base + 3 * vbytes;
+    CGScalars *sc = (CGScalars *)(base + vectors * vbytes);
     hipStream_t s = S(stream);
     // r = b - A x ; ||r||^2 ; d = z = dinv .* r ; r.z
     // (math/conjugate_gradients.hh:1125-1134)
-    EllArgs a;
-    a.mode = ELL_DEFECT;
-    a.out = r;
-    a.x = x;
-    a.rhs = b;
-    a.norm2 = &sc->current;
-    a.row_start = 0;
-    a.row_end = (int64_t)rows;
-    int st = check(ell_apply(A, a, w->slots, s), "pcg defect");
-    if (st) return st;
-    if ((st = check(pcg_start(vt, d, r, dd_inverted, (int64_t)rows, sc, eps_relative, (int)max_iters, w->slots, s),
-                    "pcg start")))
-        return st;
-    // enqueue iterations in chunks; one flag read per chunk
+    auto start = [&]() -> int {
+        EllArgs a;
+        a.mode = ELL_DEFECT;
+        a.out = r;
+        a.x = x;
+        a.rhs = b;
+        a.norm2 = &sc->current;
+        a.row_start = 0;
+        a.row_end = (int64_t)rows;
+        if (int st = check(ell_apply(A, a, w->slots, s), "pcg defect")) return st;
+        return check(pcg_start(vt, d, r, dd_inverted, (int64_t)rows, sc, eps_relative, (int)max_iters, w->slots, s),
+                     "pcg start");
+    };
     CGScalars h{};
-    size_t chunk = rows < 100000 ? 16 : 4;
-    size_t enqueued = 0;
-    while (true) {
-        for (size_t k = 0; k < chunk && enqueued < max_iters; ++k, ++enqueued)
-            if ((st = check(pcg_iteration(A, x, d, r, t0, dd_inverted, sc, w->slots, (int)enqueued, s), "pcg iteration")))
-                return st;
-        if ((st = check(hipMemcpyAsync(&h, sc, sizeof(CGScalars), hipMemcpyDeviceToHost, s), "pcg readback")))
-            return st;
-        if ((st = check(hipStreamSynchronize(s), "pcg sync"))) return st;
-        if (h.done || enqueued >= max_iters) break;
-        if (chunk < 64) chunk *= 2;
-    }
+    auto iterate = [&](int it) {
+        return check(pcg_iteration(A, x, d, r, t0, dd_inverted, sc, w->slots, it, s), "pcg iteration");
+    };
+    auto resident = [&](int begin, int end) {
+        return check(cg_resident(A, dd_inverted, begin ? t0 : x, x, t0, d, r, pub, pub + vbytes, sc, w->slots, begin,
+                                 end, s),
+                     "pcg resident");
+    };
+    if (int st = run_iterations(A, fits, w->slots, sc, max_iters, s, start, iterate, resident, h)) return st;
     if (used_iters) *used_iters = (size_t)h.iters;
     if (final_defect) *final_defect = h.current;
     if (max_iters > 0 && !h.converged) return fail(HONEI_HIP_ERROR_NOT_CONVERGED, "PCG-Jacobi reached max_iters");
