@@ -145,6 +145,7 @@ hipError_t BatchMG::tune_level(BLevel &lv) {
     hipError_t err = hipSuccess;
     const size_t vs = vt_size(vt), es = inner_vector_bytes();
     for (int T : {1, 2, 4}) {
+        if (T > 1 && lv.level <= kMaxCoarseTop) break;   // the coarse launch sums rows as T = 1
         const Level0 g = level_geometry(lv.level, T, 256);
         void *Aj = nullptr, *Arl = nullptr, *Ax = nullptr, *vec = nullptr, *scd = nullptr, *lst = nullptr;
         const size_t vbytes = (size_t)(ns * g.vld) * es;
@@ -428,7 +429,7 @@ hipError_t BatchMG::enqueue_vcycle(hipStream_t s) {
         return BMat{lv.Aj, lv.Arl, lv.Ax, lv.stride, lv.ax_ld, lv.n, lv.vld, (lv.n * lv.T + lv.block - 1) / lv.block};
     };
     // levels 1..lf as one launch (one work-group per slot), the rest level by level
-    const int64_t lf = cfg_.fused_levels >= 2 ? std::min<int64_t>(cfg_.fused_levels, max_level_) : 1;
+    const int64_t lf = std::max<int64_t>(1, fused_top());
     for (int64_t l = max_level_; l > lf; --l) {
         BLevel &lv = L_[(size_t)l];
         const BMat m = mat(lv);
@@ -452,36 +453,17 @@ hipError_t BatchMG::enqueue_vcycle(hipStream_t s) {
         HX(b_restrict(vt, lv, L_[(size_t)l - 1], w, s));
     }
     if (lf >= 2) {
-        FusedCycle fc{};
-        fc.top = (int)lf;
-        fc.n_pre = cfg_.n_pre;
-        fc.n_post = cfg_.n_post;
+        CoarseCycle cc{};
+        cc.top = (int)lf;
+        cc.n_pre = cfg_.n_pre;
+        cc.n_post = cfg_.n_post;
         for (int64_t l = 1; l <= lf; ++l) {
             const BLevel &lv = L_[(size_t)l];
-            FusedLevel &f = fc.lv[l];
-            f.Aj = lv.Aj;
-            f.Arl = lv.Arl;
-            f.Ax = lv.Ax;
-            f.stride = lv.stride;
-            f.ax_ld = lv.ax_ld;
-            f.n = lv.n;
-            f.vld = lv.vld;
-            f.side = lv.side;
-            f.cap = lv.cap;
-            f.ncpr = lv.ncpr;
-            f.T = lv.T;
-            f.dinv = lv.dinv;
-            f.rhs = lv.rhs;
-            f.x = lv.x;
-            f.d = lv.d;
-            f.t = lv.t;
+            cc.lv[l] = CoarseLevel{lv.kappa, lv.dinv, lv.rhs, lv.x, lv.kld, lv.vld, lv.cap, 0, 0};
         }
-        fc.g = L_[1].g;
-        fc.u = L_[1].u;
-        fc.en = L_[1].en;
-        fc.konv = coarse_konv();
-        fc.max_iters = (int)(4 * L_[1].n + 64);
-        HX(b_coarse_vcycle(vt, fc, level_work(1), L_[1].cap, s));
+        cc.konv = coarse_konv();
+        cc.max_iters = (int)(4 * L_[1].n + 64);
+        HX(b_coarse_cycle(vt, cc, level_work(1), L_[1].cap, s));
     } else {
         HX(b_coarse_cg(vt, L_[1], level_work(1), s));
     }

@@ -93,8 +93,9 @@ struct BatchConfig {
     // MIXED driver), 1 conjugate gradients in FP64 preconditioned by the
     // V-cycle (robust where the rediscretised hierarchy over-corrects).
     int32_t outer = 1;
-    // Levels 1..fused_levels of every V-cycle in one launch (one work-group
-    // per slot); 0 or 1: level by level.
+    // >= 2: the coarse levels of every V-cycle in one launch (one work-group
+    // per slot), as many as the launch takes (coarse_top); 0 or 1: level by
+    // level.
     int32_t fused_levels = 4;
     // 1: each step is one graph launch; 0: the same kernels enqueued on the
     // stream at every step (for tools that cannot follow graph launches).
@@ -251,6 +252,10 @@ struct BuildParams {
     int32_t T[kMaxLevel + 1];
 };
 
+// Finest level the coarse launch (b_coarse_cycle) takes.
+int64_t coarse_top(ValueType vt);
+constexpr int kMaxFusedLevels = 6;   // range of BatchConfig::fused_levels
+
 class BatchMG {
   public:
     BatchMG() = default;
@@ -325,27 +330,32 @@ class BatchMG {
     bool paired(const BLevel &lv) const {
         return cfg_.pair_sweeps && lv.side >= kPairMinSide && (cfg_.n_pre == 2 || cfg_.n_post == 2);
     }
-    // Some kernel reads level l's stored values: every level except those
-    // whose smoothing passes all run as matrix-free paired launches outside
-    // the fused coarse launch.
+    // Some kernel reads level l's stored values: every level except those of
+    // the coarse launch and those whose smoothing passes all run as
+    // matrix-free paired launches.
     bool stores_values(const BLevel &lv) const {
-        const int64_t lf = cfg_.fused_levels >= 2 ? std::min<int64_t>(cfg_.fused_levels, max_level_) : 1;
+        if (lv.level <= fused_top()) return false;
         const bool all_paired = paired(lv) && cfg_.n_pre == 2 && (cfg_.n_post == 2 || cfg_.n_post == 0);
-        return !(cfg_.matrix_free && all_paired && lv.level > lf);
+        return !(cfg_.matrix_free && all_paired);
+    }
+    // finest level of the coarse launch, 0: none
+    int64_t fused_top() const {
+        return cfg_.fused_levels >= 2 ? std::min(coarse_top((ValueType)cfg_.inner_vtype), max_level_) : 0;
     }
     // the up-leg of the level is one paired post-smoothing launch with the
     // prolongation from the level below fused in (b_pair with xc); it leaves
     // the level's result in t, every other level's in x
     bool fused_post(const BLevel &lv) const {
-        const int64_t lf = cfg_.fused_levels >= 2 ? std::min<int64_t>(cfg_.fused_levels, max_level_) : 1;
-        return paired(lv) && cfg_.n_post == 2 && lv.level > lf;
+        return paired(lv) && cfg_.n_post == 2 && lv.level > fused_top();
     }
     void *level_result(const BLevel &lv) const { return fused_post(lv) ? lv.t : lv.x; }
     // the level's paired launches gather the weights from the stencil arrays
-    bool stores_stencil(const BLevel &lv) const { return cfg_.matrix_free == 2 && !stores_values(lv); }
+    bool stores_stencil(const BLevel &lv) const {
+        return cfg_.matrix_free == 2 && !stores_values(lv) && lv.level > fused_top();
+    }
     // weight source of the level's paired launches (b_pair's wmode)
     int pair_weights(const BLevel &lv) const {
-        return cfg_.matrix_free == 0 ? 0 : (stores_stencil(lv) ? 2 : 1);
+        return cfg_.matrix_free == 0 && stores_values(lv) ? 0 : (stores_stencil(lv) ? 2 : 1);
     }
     // the FP64 outer values are read only when the outer row sums do not
     // form them from the cell coefficients
@@ -444,7 +454,8 @@ hipError_t b_prolong_axpy(ValueType vt, const BLevel &fine, const BLevel &coarse
 // writes two Jacobi sweeps of xin to out0 (xin != out0).  Bit-identical to
 // the separate b_ell launches.
 // wmode: the weights from the stored values (0), from lv.kappa (1), from the
-// distinct-weight arrays lv.st (2): the same bits in every form.
+// distinct-weight arrays lv.st (2): the same bits in every form.  3: the
+// constant operator (q1_constant_weights), for a level assembled as such.
 // xc (PAIR_POST, with `coarse`): the prolongation fused in, out0 =
 // J(J(xin + P xc)), the same bits as b_prolong_axpy into a third vector
 // followed by the unfused pair (xc: the coarse level's result).
@@ -463,34 +474,27 @@ struct SlotIds {
     int32_t n;
     int32_t id[kMaxSlotIds];
 };
-// The coarse end of the V-cycle in one launch: levels 1..top of every
-// listed slot by one work-group per slot (top = the slot's finest level if
-// that is below `top`), the same sweeps, transfers and coarse CG as the
-// level-by-level launches, in the same order and arithmetic.
-constexpr int kMaxFusedLevels = 6;
-struct FusedLevel {
-    const int32_t *Aj;
-    const uint32_t *Arl;
-    const void *Ax;
-    int64_t stride, ax_ld, n, vld, side, cap, ncpr;
-    int T;
-    void *dinv, *rhs, *x, *d, *t;   // inner vector type
+// The coarse end of the V-cycle in one launch (coarse_kernels.hip): levels
+// 1..top of every listed slot by one work-group per slot (from the slot's
+// finest level if that is below `top`): n_pre sweeps from zero, the transfers
+// and the coarse CG, n_post sweeps, the result in the finest one's x -- the
+// bits of the level-by-level launches at threads-per-row 1.  kappa null on
+// every level: the constant operator.
+constexpr int kMaxCoarseTop = 6;
+struct CoarseLevel {
+    const double *kappa;      // cell coefficients [slot][kld]
+    const void *dinv, *rhs;   // inner vector type, [slot][vld]
+    void *x;
+    int64_t kld, vld, cap;
+    int32_t n, at;            // set by b_coarse_cycle
 };
-// Byte offsets of a level's arrays in the LDS form of the fused cycle.
-struct FusedLds {
-    int32_t aj, arl, ax, dinv, rhs, x, d, t;
-};
-struct FusedCycle {
+struct CoarseCycle {
     int top, n_pre, n_post;
-    FusedLevel lv[kMaxFusedLevels + 1];   // index = level (1..top)
-    void *g, *u, *en;                     // level-1 CG scratch
+    CoarseLevel lv[kMaxCoarseTop + 1];   // index = level (1..top)
     double konv;
     int max_iters;
-    // LDS form (set by b_coarse_vcycle): per level, and the CG scratch
-    FusedLds lo[kMaxFusedLevels + 1];
-    int32_t og, ou, oen;
 };
-hipError_t b_coarse_vcycle(ValueType vt, const FusedCycle &fc, const BWork &w, int64_t max_slots, hipStream_t s);
+hipError_t b_coarse_cycle(ValueType vt, const CoarseCycle &cc, const BWork &w, int64_t max_slots, hipStream_t s);
 
 // Fresh scalars in `state` for slots[0..n), one launch per 256 ids.
 hipError_t b_set_states(SlotScalars *sc, const int64_t *slots, int64_t n, int32_t state, hipStream_t s);

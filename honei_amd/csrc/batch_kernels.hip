@@ -201,12 +201,11 @@ struct PairGeom {
 // Tiled launches stage the slots of a work-group's tiles in LDS at the
 // start; their grids give no work-group more than kTileSlots tiles.
 constexpr int kTileSlots = 1024;
+// Fewer tall tiles than this (one per CU) leave CUs without one: short tiles then.
+constexpr int64_t kMinTallTiles = 256;
 // The element-wise outer launches stage at most kElemSlots logical blocks'
 // slots and scalars per work-group.
 constexpr int kElemSlots = 64;
-// The fused coarse cycle's work-group: one per slot, five wavefronts, so a
-// sweep of the largest fused level (17^2 = 289 nodes) is one round.
-constexpr int kFusedThreads = 320;
 inline int tiled_grid(int64_t units, int threads) {
     const int64_t g = batch_grid(units, threads), need = (units + kTileSlots - 1) / kTileSlots;
     return (int)(g > need ? g : need);
@@ -271,7 +270,9 @@ __device__ inline void load_weights4(const double *p, double (&o)[4]) {
 // V: the vector and arithmetic type (float for float / bf16 values, double
 // for double values)
 // WM: weights from the stored values (0), formed from the cell coefficients
-// (1), gathered from the distinct-weight arrays (2).
+// (1), gathered from the distinct-weight arrays (2), the constant operator's
+// (3: no loads for the weights, and dinv, which has one interior and one
+// boundary value, loaded once).
 // FP (PAIR_POST only): xc = the coarse level's result (vld_c per slot).
 // NR: grid rows per thread; thread (i, lane) takes tile rows i + u *
 // kPairTileRows (u < NR), so a tile is kPairTileRows * NR - 2 rows and every
@@ -320,6 +321,12 @@ __global__ __launch_bounds__(kPairTileRows * kWave, 8) void k_b_pair(BMat m, BWo
             eb = ((t - 2 * kWave) % 2) ? kWave + 1 : 0;
         }
     }
+    V di_in = V(0), di_bnd = V(0);
+    if constexpr (WM == 3) {
+        di_in = dinv[S + 1];
+        di_bnd = dinv[0];
+    }
+    auto on_border = [&](int a, int b) { return a == 0 || a == S - 1 || b == 0 || b == S - 1; };
     int64_t k = 0;
     for (int64_t lb = lb0; lb < total; lb += gridDim.x, ++k) {
         int64_t e, rem, strip, seg;
@@ -348,7 +355,7 @@ __global__ __launch_bounds__(kPairTileRows * kWave, 8) void k_b_pair(BMat m, BWo
             r[u] = r0 - 1 + i + u * kPairTileRows;
             rc[u] = r[u] < 0 ? 0 : (r[u] > S - 1 ? S - 1 : r[u]);
             node[u] = (int64_t)rc[u] * S + colc;
-            bnd[u] = rc[u] == 0 || rc[u] == S - 1 || colc == 0 || colc == S - 1;
+            bnd[u] = on_border(rc[u], colc);
         }
         const int egr = min(max(r0 - 2 + ea, 0), S - 1), egc = min(max(c0 - 2 + eb, 0), S - 1);
         const int64_t ej = (int64_t)egr * S + egc;
@@ -358,14 +365,20 @@ __global__ __launch_bounds__(kPairTileRows * kWave, 8) void k_b_pair(BMat m, BWo
 #pragma unroll
         for (int u = 0; u < NR; ++u) {
             rh[u] = rs[node[u]];
-            di[u] = ds[node[u]];
+            if constexpr (WM == 3)
+                di[u] = bnd[u] ? di_bnd : di_in;
+            else
+                di[u] = ds[node[u]];
             xn[u] = (PAIR == PAIR_PRE) ? V(0) : xs[node[u]];
             if constexpr (FP) prolong_taps(xc + ls * vld_c, (S >> 1) + 1, rc[u], colc, tn[u]);
         }
         // the extra entry's loads only where there is one (the first waves)
         V e1 = V(0), e2 = V(0);
         if (threadIdx.x < kExtra) {
-            e1 = (PAIR == PAIR_PRE) ? ds[ej] : xs[ej];
+            if constexpr (PAIR == PAIR_PRE && WM == 3)
+                e1 = on_border(egr, egc) ? di_bnd : di_in;
+            else
+                e1 = (PAIR == PAIR_PRE) ? ds[ej] : xs[ej];
             if (PAIR == PAIR_PRE) e2 = rs[ej];
             if constexpr (FP) prolong_taps(xc + ls * vld_c, (S >> 1) + 1, egr, egc, te);
         }
@@ -404,6 +417,8 @@ __global__ __launch_bounds__(kPairTileRows * kWave, 8) void k_b_pair(BMat m, BWo
                 av[u][6] = q1[0];
                 av[u][7] = q0[1];
                 av[u][8] = q0[0];
+            } else if constexpr (WM == 3) {
+                q1_constant_weights<VT, V>(av[u]);
             } else {
 #pragma unroll
                 for (int q = 0; q < 9; ++q) av[u][q] = load_value_cached(ax + node[u] + (int64_t)q * m.stride);
@@ -1125,192 +1140,6 @@ __global__ __launch_bounds__(256) void k_b_coarse_cg(EllView A, BWork w, int64_t
     }
 }
 
-// ---- the coarse end of the V-cycle, one work-group per slot -------------------------
-// One sweep of level L of slot `ls` by the whole work-group (T lanes per row;
-// the loop bound is a multiple of blockDim so every lane of a row joins its
-// lane reduction).  Same row sum and epilogue as k_b_ell.
-template <typename VT, int T, int MODE, typename V = typename VecOf<VT>::type>
-__device__ inline void fused_sweep(const FusedLevel &L, int64_t ls, V *out, const V *x, const V *rhs, const V *dinv) {
-    const VT *Ax = (const VT *)L.Ax + ls * L.ax_ld;
-    const int64_t vo = ls * L.vld;
-    const V *xs = x + vo, *rs = rhs + vo, *ds = dinv + vo;
-    V *os = out + vo;
-    const int64_t total = ((L.n * T + blockDim.x - 1) / blockDim.x) * blockDim.x;
-    for (int64_t gid = threadIdx.x; gid < total; gid += blockDim.x) {
-        const int lane = (int)(gid & (T - 1));
-        const int64_t row = gid / T;
-        const bool active = row < L.n;
-        V s = V(0);
-        if (active) {
-            if constexpr (MODE == ELL_JACOBI0)
-                s = ell_lane_sum<VT, T, true, true>(L.Aj, Ax, row, lane, L.Arl[row], L.stride, rs, ds);
-            else
-                s = ell_lane_sum<VT, T, false, true>(L.Aj, Ax, row, lane, L.Arl[row], L.stride, xs);
-        }
-        s = lane_group_sum<T>(s);
-        if (active && lane == 0) {
-            if constexpr (MODE == ELL_DEFECT) {
-                os[row] = rs[row] - s;
-            } else {
-                const V xin = (MODE == ELL_JACOBI0) ? ds[row] * rs[row] : xs[row];
-                const V t = rs[row] - s;
-                os[row] = xin + t * ds[row];
-            }
-        }
-    }
-}
-
-template <typename VT, int MODE, typename V = typename VecOf<VT>::type>
-__device__ inline void fused_sweep_t(const FusedLevel &L, int64_t ls, V *out, const V *x, const V *rhs,
-                                     const V *dinv) {
-    switch (L.T) {
-        case 1: fused_sweep<VT, 1, MODE>(L, ls, out, x, rhs, dinv); break;
-        case 2: fused_sweep<VT, 2, MODE>(L, ls, out, x, rhs, dinv); break;
-        case 4: fused_sweep<VT, 4, MODE>(L, ls, out, x, rhs, dinv); break;
-        default: fused_sweep<VT, 8, MODE>(L, ls, out, x, rhs, dinv); break;
-    }
-    __syncthreads();
-}
-
-// Level l of the cycle: fc's arrays, or (lds non-null) the LDS copies at
-// the offsets fc.lo[l] (a copy of one level, so no runtime-indexed local array).
-template <bool LDSM>
-__device__ inline FusedLevel level_view(const FusedCycle &fc, int l, char *lds) {
-    FusedLevel L = fc.lv[l];
-    if constexpr (LDSM) {
-        const FusedLds &o = fc.lo[l];
-        L.Aj = (const int32_t *)(lds + o.aj);
-        L.Arl = (const uint32_t *)(lds + o.arl);
-        L.Ax = lds + o.ax;
-        L.dinv = lds + o.dinv;
-        L.rhs = lds + o.rhs;
-        L.x = lds + o.x;
-        L.d = lds + o.d;
-        L.t = lds + o.t;
-    }
-    return L;
-}
-
-// One V-cycle of slot g from level `top` down to the coarse CG and back
-// (fc's arrays indexed by slot g, or with LDSM the LDS copies at lds, g = 0;
-// a compile-time choice, so the LDS form's accesses are LDS instructions).
-template <typename VT, bool LDSM>
-__device__ inline void fused_cycle_body(const FusedCycle &fc, int64_t g, int top, char *lds) {
-    typedef typename VecOf<VT>::type V;
-    const Mask8 mk{0xffu};   // all Dirichlet, as the level-by-level transfers
-    // down: n_pre sweeps from zero (first two fused), defect, restriction
-    for (int l = top; l >= 2; --l) {
-        const FusedLevel L = level_view<LDSM>(fc, l, lds);
-        V *Lx = (V *)L.x, *Lt = (V *)L.t, *Ld = (V *)L.d;
-        const V *Lr = (const V *)L.rhs, *Ldi = (const V *)L.dinv;
-        const int rest = fc.n_pre - 2;
-        V *src = (rest % 2 == 0) ? Lx : Lt;
-        fused_sweep_t<VT, ELL_JACOBI0>(L, g, src, (const V *)nullptr, Lr, Ldi);
-        for (int k = 0; k < rest; ++k) {
-            V *dst = (src == Lx) ? Lt : Lx;
-            fused_sweep_t<VT, ELL_JACOBI>(L, g, dst, src, Lr, Ldi);
-            src = dst;
-        }
-        fused_sweep_t<VT, ELL_DEFECT>(L, g, Ld, Lx, Lr, (const V *)nullptr);
-        const FusedLevel C = level_view<LDSM>(fc, l - 1, lds);
-        const int64_t m = C.side - 1;
-        for (int64_t i = threadIdx.x; i < C.n; i += blockDim.x)
-            restrict_node<V>((V *)C.rhs + g * C.vld, Ld + g * L.vld, m, mk, i);
-        __syncthreads();
-    }
-    {   // coarse CG on level 1
-        const FusedLevel L = level_view<LDSM>(fc, 1, lds);
-        EllView A{};
-        A.rows = L.n;
-        A.cols = L.n;
-        A.stride = L.stride;
-        A.ncpr = L.ncpr;
-        A.threads = L.T;
-        A.Aj = L.Aj;
-        A.Ax = (const VT *)L.Ax + g * L.ax_ld;
-        A.Arl = L.Arl;
-        const int64_t o = g * L.vld;
-        V *cg = (V *)(LDSM ? lds + fc.og : fc.g), *cu = (V *)(LDSM ? lds + fc.ou : fc.u);
-        V *cen = (V *)(LDSM ? lds + fc.oen : fc.en);
-        (void)coarse_cg_block<VT>(A, (const V *)L.rhs + o, (V *)L.x + o, cg + o, cu + o, cen + o, fc.konv,
-                                  fc.max_iters);
-        __syncthreads();
-    }
-    // up: x += P x_coarse, n_post sweeps (result in x)
-    for (int l = 2; l <= top; ++l) {
-        const FusedLevel L = level_view<LDSM>(fc, l, lds);
-        const FusedLevel C = level_view<LDSM>(fc, l - 1, lds);
-        V *Lx = (V *)L.x, *Lt = (V *)L.t;
-        const V *Lr = (const V *)L.rhs, *Ldi = (const V *)L.dinv;
-        const int64_t m = C.side - 1;
-        for (int64_t i = threadIdx.x; i < L.n; i += blockDim.x)
-            prolong_node<V, true>(nullptr, (const V *)C.x + g * C.vld, m, mk, Lx + g * L.vld, V(1), i);
-        __syncthreads();
-        V *src = Lx, *dst = Lt;
-        for (int k = 0; k < fc.n_post; ++k) {
-            fused_sweep_t<VT, ELL_JACOBI>(L, g, dst, src, Lr, Ldi);
-            V *tmp = src;
-            src = dst;
-            dst = tmp;
-        }
-        if (src != Lx) {
-            for (int64_t i = threadIdx.x; i < L.n; i += blockDim.x) Lx[g * L.vld + i] = src[g * L.vld + i];
-            __syncthreads();
-        }
-    }
-}
-
-template <typename VT>
-__global__ __launch_bounds__(kFusedThreads) void k_b_coarse_vcycle(FusedCycle fc, BWork w) {
-    const int64_t a0 = active_first(w), na = active_count(w);
-    for (int64_t a = blockIdx.x; a < na; a += gridDim.x) {
-        const int64_t g = w.list[a0 + a];
-        int top = fc.top;
-        while (top > 1 && g >= fc.lv[top].cap) --top;   // slots whose finest level is lower
-        fused_cycle_body<VT, false>(fc, g, top, nullptr);
-    }
-}
-
-// The same cycle with the slot's levels in LDS (dynamic LDS, offsets
-// fc.lo, fc.og/ou/oen): the index arrays once per launch, then per slot its
-// values, dinv and finest right-hand side in, the cycle on the LDS copies
-// (slot index 0, the same code and arithmetic, so the same bits), and the
-// finest level's x back out.  Every phase then waits on LDS instead of an L2
-// round trip.
-__device__ inline void lds_copy_words(void *dst, const void *src, int64_t bytes) {
-    uint32_t *d = (uint32_t *)dst;
-    const uint32_t *s = (const uint32_t *)src;
-    for (int64_t i = threadIdx.x; i < bytes / 4; i += blockDim.x) d[i] = s[i];
-}
-template <typename VT>
-__global__ __launch_bounds__(kFusedThreads) void k_b_coarse_vcycle_lds(FusedCycle fc, BWork w) {
-    typedef typename VecOf<VT>::type V;
-    extern __shared__ __align__(16) char lds[];
-    const int64_t a0 = active_first(w), na = active_count(w);
-    if ((int64_t)blockIdx.x >= na) return;   // uniform per work-group
-    for (int l = 1; l <= fc.top; ++l) {
-        const FusedLevel &L = fc.lv[l];
-        lds_copy_words(lds + fc.lo[l].aj, L.Aj, 4 * L.ncpr * L.stride);
-        lds_copy_words(lds + fc.lo[l].arl, L.Arl, 4 * L.n);
-    }
-    for (int64_t a = blockIdx.x; a < na; a += gridDim.x) {
-        const int64_t g = w.list[a0 + a];
-        int top = fc.top;
-        while (top > 1 && g >= fc.lv[top].cap) --top;   // slots whose finest level is lower
-        for (int l = 1; l <= top; ++l) {
-            const FusedLevel &L = fc.lv[l];
-            lds_copy_words(lds + fc.lo[l].ax, (const VT *)L.Ax + g * L.ax_ld, (int64_t)sizeof(VT) * L.ax_ld);
-            lds_copy_words(lds + fc.lo[l].dinv, (const V *)L.dinv + g * L.vld, (int64_t)sizeof(V) * L.n);
-        }
-        lds_copy_words(lds + fc.lo[top].rhs, (const V *)fc.lv[top].rhs + g * fc.lv[top].vld,
-                       (int64_t)sizeof(V) * fc.lv[top].n);
-        __syncthreads();
-        fused_cycle_body<VT, true>(fc, 0, top, lds);
-        lds_copy_words((V *)fc.lv[top].x + g * fc.lv[top].vld, lds + fc.lo[top].x, (int64_t)sizeof(V) * fc.lv[top].n);
-        __syncthreads();
-    }
-}
-
 // Fresh scalars in `state` for the slots of one id list (passed by value).
 __global__ void k_b_set_states(SlotScalars *sc, SlotIds ids, int32_t state) {
     const int k = (int)threadIdx.x;
@@ -1635,7 +1464,7 @@ hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void
                lv.side > kMaxTransferSide || xc == out0))
         return hipErrorInvalidValue;
     const int64_t vld_c = fp ? coarse->vld : 0;
-    if (wmode < 0 || wmode > 2) return hipErrorInvalidValue;
+    if (wmode < 0 || wmode > 3) return hipErrorInvalidValue;
     if (wmode == 1 && (!lv.kappa || lv.kld < (lv.side - 1) * (lv.side - 1))) return hipErrorInvalidValue;
     if (wmode == 2 && !lv.st) return hipErrorInvalidValue;
     if (wmode == 0 && (!lv.Ax || !lv.Aj)) return hipErrorInvalidValue;
@@ -1645,7 +1474,9 @@ hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void
     pg.width = (int32_t)((lv.side + pg.strips - 1) / pg.strips);
     // two grid rows per thread on the larger levels (taller tiles: half the
     // halo rows per node, twice the loads in flight per thread)
-    const int nr = lv.side >= kPairTallMinSide && vt != VT_F64 ? 2 : 1;
+    int nr = lv.side >= kPairTallMinSide && vt != VT_F64 ? 2 : 1;
+    if (nr == 2 && lv.cap * pg.strips * ((lv.side + 2 * kPairTileRows - 3) / (2 * kPairTileRows - 2)) < kMinTallTiles)
+        nr = 1;
     const int64_t rows = (int64_t)kPairTileRows * nr - 2;
     pg.segs = (int32_t)((lv.side + rows - 1) / rows);
     if (lv.cap <= 0) return hipSuccess;
@@ -1659,7 +1490,9 @@ hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void
     pair_launch<VT, P, MFV>(grid, block, s, m, w, pg, out0, out1, x, lv.rhs, lv.dinv, xc, vld_c, nr)
 #define PAIR_WM(VT, P)                                                        \
     do {                                                                      \
-        if (wmode == 2)                                                       \
+        if (wmode == 3)                                                       \
+            PAIR_LAUNCH(VT, P, 3);                                            \
+        else if (wmode == 2)                                                  \
             PAIR_LAUNCH(VT, P, 2);                                            \
         else if (wmode == 1)                                                  \
             PAIR_LAUNCH(VT, P, 1);                                            \
@@ -1726,61 +1559,6 @@ hipError_t b_coarse_cg(ValueType vt, const BLevel &lv, const BWork &w, hipStream
                            (const double *)dr, dx, dg, du, de, konv, max_iters);
     else
         return hipErrorInvalidValue;
-    return hipGetLastError();
-}
-
-hipError_t b_coarse_vcycle(ValueType vt, const FusedCycle &fc, const BWork &w, int64_t max_slots, hipStream_t s) {
-    if (max_slots <= 0) return hipSuccess;
-    if (fc.top < 1 || fc.top > kMaxFusedLevels || fc.n_pre < 2 || fc.n_post < 0) return hipErrorInvalidValue;
-    for (int l = 1; l <= fc.top; ++l) {
-        const int T = fc.lv[l].T;
-        if (T != 1 && T != 2 && T != 4 && T != 8) return hipErrorInvalidValue;
-        if (l > 1 && (fc.lv[l].side != 2 * (fc.lv[l - 1].side - 1) + 1 || fc.lv[l].cap > fc.lv[l - 1].cap))
-            return hipErrorInvalidValue;
-    }
-    const int grid = (int)(max_slots < 2048 ? max_slots : 2048);
-    // the LDS form when every level of the cycle fits in 60 KiB (with the
-    // kernel's static LDS, within a work-group's 64 KiB)
-    FusedCycle f = fc;
-    const size_t vs = vt_size(vt), es = vt == VT_F64 ? 8 : 4;
-    int64_t at = 0;
-    auto take = [&](int64_t bytes) {
-        const int64_t o = at;
-        at += (bytes + 15) / 16 * 16;
-        return (int32_t)o;
-    };
-    for (int l = 1; l <= f.top; ++l) {
-        const FusedLevel &L = f.lv[l];
-        FusedLds &o = f.lo[l];
-        o.aj = take(4 * L.ncpr * L.stride);
-        o.arl = take(4 * L.n);
-        o.ax = take((int64_t)vs * L.ax_ld);
-        o.dinv = take((int64_t)es * L.n);
-        o.rhs = take((int64_t)es * L.n);
-        o.x = take((int64_t)es * L.n);
-        o.d = take((int64_t)es * L.n);
-        o.t = take((int64_t)es * L.n);
-    }
-    f.og = take((int64_t)es * f.lv[1].n);
-    f.ou = take((int64_t)es * f.lv[1].n);
-    f.oen = take((int64_t)es * f.lv[1].n);
-    const bool lds = at <= 60 * 1024;
-#define CYCLE_LAUNCH(VT)                                                                                  \
-    do {                                                                                                  \
-        if (lds)                                                                                          \
-            hipLaunchKernelGGL(k_b_coarse_vcycle_lds<VT>, dim3(grid), dim3(kFusedThreads), (size_t)at, s, f, w); \
-        else                                                                                              \
-            hipLaunchKernelGGL(k_b_coarse_vcycle<VT>, dim3(grid), dim3(kFusedThreads), 0, s, f, w);      \
-    } while (0)
-    if (vt == VT_F32)
-        CYCLE_LAUNCH(float);
-    else if (vt == VT_BF16)
-        CYCLE_LAUNCH(bf16);
-    else if (vt == VT_F64)
-        CYCLE_LAUNCH(double);
-    else
-        return hipErrorInvalidValue;
-#undef CYCLE_LAUNCH
     return hipGetLastError();
 }
 

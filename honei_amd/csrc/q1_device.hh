@@ -62,6 +62,19 @@ __device__ inline float bf16_round(float v) {
     return __uint_as_float((u >> 16) << 16);
 }
 
+// The nine weights of an interior row of the constant operator as a kernel
+// reading the stored matrix of value type VT sees them.
+template <typename VT, typename A>
+__device__ inline void q1_constant_weights(A (&w)[9]) {
+    A off = A(-1.0 / 3.0), mid = A(8.0 / 3.0);
+    if constexpr (sizeof(VT) == 2) {
+        off = bf16_round(off);
+        mid = bf16_round(mid);
+    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) w[k] = k == 4 ? mid : off;
+}
+
 // The weights of node (i, j) as a kernel reading the stored matrix of value
 // type VT sees them (arithmetic type A: float for float / bf16 values,
 // double for double): interior nodes from the cell coefficients, boundary

@@ -458,8 +458,9 @@ typedef struct {
     int32_t outer_method;      /* 0 defect correction x += V(b - A x) (the reference's MIXED
                                   driver); 1 FP64 conjugate gradients preconditioned by the V-cycle,
                                   converged residual confirmed by a recomputed b - A x (default) */
-    int32_t fused_levels;      /* levels 1..fused_levels (0..6, default 4) of every V-cycle run
-                                  as one launch, one work-group per slot (same arithmetic) */
+    int32_t fused_levels;      /* 0..6, default 4; 2 and up: the coarse levels of every V-cycle
+                                  (up to 65^2 nodes, FP64 33^2) run as one launch, one work-group
+                                  per slot (same arithmetic); 0, 1: level by level */
     int32_t use_graphs;        /* 1 (default): a step is one hipGraph launch; 0: the same kernels
                                   enqueued directly at every step (same results; for profilers
                                   that cannot follow graph launches) */
