@@ -13,10 +13,22 @@
 // Kernel fusion: the first two Jacobi sweeps from zero are one pass
 // (ELL_JACOBI0) and the correction x += c is folded into the last sweep;
 // prolongation and the coarse-grid correction x += alpha*c are one pass.
+//
+// Hierarchies that were assembled here (build_q1*) run their cycles as the
+// batch solver's launches over one slot (q1_vcycle): Jacobi0 + defect, and
+// prolongation + two sweeps, as one matrix-free launch each, the levels up to
+// 65^2 (FP64: 33^2) as one launch; with the FP64 outer iteration matrix-free too and its
+// scalars on the device (mg_kernels.hip).  Same operands, sums and roundings.
+// A V(2,2) cycle of 11 levels was 74 launches reading nine stored values and
+// columns per node in each; it is 16 that read 12-16 bytes a node (constant
+// operator) or 8 more per cell.
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <utility>
 
+#include "batch.hh"
 #include "runtime.hh"
 #include "solvers.hh"
 
@@ -68,7 +80,7 @@ MGHierarchy::~MGHierarchy() {
         l.A.release();
         l.P.release();
         l.R.release();
-        for (void *p : {l.dinv, l.c, l.d, l.rhs, l.x, l.t})
+        for (void *p : {l.dinv, l.c, l.d, l.rhs, l.x, l.t, (void *)l.kappa})
             if (p) (void)hipFree(p);
     }
     A_outer.release();
@@ -105,6 +117,9 @@ hipError_t MGHierarchy::alloc_coarse_scratch() {
     if (!scal_) {
         HX(hipMalloc((void **)&scal_, 64 * sizeof(double)));
         HX(fill_bytes_zero(scal_, 64 * sizeof(double), nullptr));
+        always_ = (OneSlot *)(scal_ + 60);
+        const OneSlot one{0, 0, 1};
+        HX(hipMemcpy(always_, &one, sizeof(one), hipMemcpyHostToDevice));
     }
     if (!slots_.partials) {
         slots_.capacity = 1 << 17;
@@ -116,10 +131,13 @@ hipError_t MGHierarchy::alloc_coarse_scratch() {
 }
 
 hipError_t MGHierarchy::build_q1(double omega, hipStream_t s) {
+    q1_ = false;
     for (int64_t l = min_level; l <= max_level; ++l) {
         const int64_t side = (1ll << l) + 1, n = side * side;
         const int64_t stride = 32 * ((n + 31) / 32);
         HX(alloc_level_vectors(l, n));
+        if (L[(size_t)l].kappa) (void)hipFree(L[(size_t)l].kappa);
+        L[(size_t)l].kappa = nullptr;
         HX(dev_ell_alloc(L[(size_t)l].A, inner, n, n, stride, side > 2 ? 9 : 1, 1));
         HX(q1_assemble(inner, side, L[(size_t)l].A.Aj, L[(size_t)l].A.Ax, L[(size_t)l].A.Arl, stride, nullptr,
                        L[(size_t)l].dinv, omega, s));
@@ -131,21 +149,25 @@ hipError_t MGHierarchy::build_q1(double omega, hipStream_t s) {
         HX(q1_assemble(VT_F64, side, A_outer.Aj, A_outer.Ax, A_outer.Arl, stride, nullptr, nullptr, 0.0, s));
     }
     HX(alloc_coarse_scratch());
+    q1_ = true;
     return hipStreamSynchronize(s);
 }
 
 hipError_t MGHierarchy::build_q1_coeff(double omega, const double *coeff, int averaging, hipStream_t s) {
-    // per-level coefficient arrays, finest first
-    std::vector<double *> kap((size_t)max_level + 1, nullptr);
+    q1_ = false;
+    // per-level coefficient arrays, finest first, kept with the levels
     hipError_t err = hipSuccess;
     for (int64_t l = max_level; l >= min_level && err == hipSuccess; --l) {
         const int64_t cells = (1ll << l);
-        if (l == max_level) {
-            kap[(size_t)l] = (double *)coeff;
-            continue;
-        }
-        err = hipMalloc((void **)&kap[(size_t)l], sizeof(double) * (size_t)(cells * cells));
-        if (err == hipSuccess) err = coarsen_coeff(kap[(size_t)l + 1], 2 * cells, kap[(size_t)l], cells, averaging, s);
+        double *&k = L[(size_t)l].kappa;
+        if (k) (void)hipFree(k);
+        k = nullptr;
+        err = hipMalloc((void **)&k, sizeof(double) * (size_t)(cells * cells));
+        if (err != hipSuccess) break;
+        if (l == max_level)
+            err = vcopy(k, coeff, cells * cells, VT_F64, s);
+        else
+            err = coarsen_coeff(L[(size_t)l + 1].kappa, 2 * cells, k, cells, averaging, s);
     }
     for (int64_t l = min_level; l <= max_level && err == hipSuccess; ++l) {
         const int64_t side = (1ll << l) + 1, n = side * side;
@@ -154,7 +176,7 @@ hipError_t MGHierarchy::build_q1_coeff(double omega, const double *coeff, int av
         if (err == hipSuccess) err = dev_ell_alloc(L[(size_t)l].A, inner, n, n, stride, side > 2 ? 9 : 1, 1);
         if (err == hipSuccess)
             err = q1_assemble(inner, side, L[(size_t)l].A.Aj, L[(size_t)l].A.Ax, L[(size_t)l].A.Arl, stride,
-                              kap[(size_t)l], L[(size_t)l].dinv, omega, s);
+                              L[(size_t)l].kappa, L[(size_t)l].dinv, omega, s);
     }
     if (err == hipSuccess) {
         const int64_t side = (1ll << max_level) + 1, n = side * side;
@@ -165,9 +187,83 @@ hipError_t MGHierarchy::build_q1_coeff(double omega, const double *coeff, int av
     }
     if (err == hipSuccess) err = alloc_coarse_scratch();
     (void)hipStreamSynchronize(s);
-    for (int64_t l = min_level; l < max_level; ++l)
-        if (kap[(size_t)l]) (void)hipFree(kap[(size_t)l]);
+    q1_ = err == hipSuccess;
     return err;
+}
+
+bool MGHierarchy::q1_cycle() const {
+    if (!q1_ || min_level != 1 || max_level < 2 || cfg.n_pre_smooth != 2 || cfg.prolmat ||
+        cfg.adapt_correction_factor != 1.0 || (!cfg.post_smooth_uses_pre && cfg.n_post_smooth != 2))
+        return false;
+    for (uint64_t m : cfg.mask)
+        if (m != 2) return false;
+    return true;
+}
+
+Q1Outer MGHierarchy::q1_outer() const {
+    const MGLevel &top = L[(size_t)max_level];
+    return Q1Outer{(int32_t)top.side, top.n, top.kappa};
+}
+
+namespace {
+
+// level lv as a batch level of one slot
+BLevel one_slot(const MGLevel &lv, int64_t level) {
+    BLevel b;
+    b.level = level;
+    b.side = lv.side;
+    b.n = lv.n;
+    b.cap = 1;
+    b.vld = lv.n;
+    b.stride = lv.A.v.stride;
+    b.ncpr = lv.A.v.ncpr;
+    b.ax_ld = b.ncpr * b.stride;
+    b.Aj = lv.A.Aj;
+    b.Arl = lv.A.Arl;
+    b.Ax = lv.A.Ax;
+    b.dinv = lv.dinv;
+    b.rhs = lv.rhs;
+    b.x = lv.x;
+    b.d = lv.d;
+    b.t = lv.t;
+    b.kappa = lv.kappa;
+    b.kld = (lv.side - 1) * (lv.side - 1);
+    return b;
+}
+BWork one_system(const OneSlot *w) { return BWork{&w->slot, &w->first, 0, 1, 0}; }
+int weights(const MGLevel &lv) { return lv.kappa ? 1 : 3; }
+
+}  // namespace
+
+hipError_t MGHierarchy::q1_up(int64_t l, const OneSlot *work, hipStream_t s) {
+    MGLevel &lv = L[(size_t)l];
+    const BLevel f = one_slot(lv, l), c = one_slot(L[(size_t)l - 1], l - 1);
+    HX(b_pair(inner, PAIR_POST, f, one_system(work), lv.t, nullptr, lv.x, s, weights(lv), &c, c.x));
+    std::swap(lv.x, lv.t);
+    return hipSuccess;
+}
+
+hipError_t MGHierarchy::q1_vcycle(int64_t top, const OneSlot *work, hipStream_t s) {
+    const BWork w = one_system(work);
+    const int64_t lf = std::min(coarse_top(inner), top);
+    for (int64_t l = top; l > lf; --l) {
+        MGLevel &lv = L[(size_t)l];
+        const BLevel f = one_slot(lv, l);
+        HX(b_pair(inner, PAIR_PRE, f, w, lv.x, lv.d, nullptr, s, weights(lv)));
+        HX(b_restrict(inner, f, one_slot(L[(size_t)l - 1], l - 1), w, s));
+    }
+    CoarseCycle cc{};
+    cc.top = (int)lf;
+    cc.n_pre = cc.n_post = 2;
+    for (int64_t l = 1; l <= lf; ++l) {
+        const BLevel b = one_slot(L[(size_t)l], l);
+        cc.lv[l] = CoarseLevel{b.kappa, b.dinv, b.rhs, b.x, b.kld, b.vld, 1, 0, 0};
+    }
+    cc.konv = inner == VT_F64 ? 2.220446049250313e-16 : 1.1920928955078125e-07;
+    cc.max_iters = (int)(4 * L[1].n + 64);
+    HX(b_coarse_cycle(inner, cc, w, 1, s));
+    for (int64_t l = lf + 1; l <= top; ++l) HX(q1_up(l, work, s));
+    return hipSuccess;
 }
 
 hipError_t MGHierarchy::read_scalar(double *dst, const double *src, hipStream_t s) {
@@ -265,6 +361,7 @@ hipError_t MGHierarchy::run_kernel(hipStream_t s, int64_t *inner_iters, double *
     // and no convergence test the initial norm is not needed either.  The
     // iterate x and the cycle count are unchanged by these omissions.
     const bool lean = mixed_inner_ && !cfg.convergence_check;
+    const bool q1 = q1_cycle();
     const bool need_initial = !(lean && cfg.n_max_iter == 1);
     // d[max] = rhs when the start vector is zero (no matvec), else rhs - A x
     const void *top_d = top.d;
@@ -285,6 +382,21 @@ hipError_t MGHierarchy::run_kernel(hipStream_t s, int64_t *inner_iters, double *
         for (iter = 1; iter <= cfg.n_max_iter; ++iter) {
             const bool skip_final = lean && iter == cfg.n_max_iter;
             int64_t l = maxl;
+            if (q1 && maxl > coarse_top(inner)) {
+                // the top level's down-leg on x, the rest as one-slot launches
+                HX(smooth_from_zero(maxl, top_d, top.c, top.x, s));
+                HX(defect(maxl, top.d, top.rhs, top.x, nullptr, s));
+                HX(b_restrict(inner, one_slot(top, maxl), one_slot(L[(size_t)maxl - 1], maxl - 1), one_system(always_),
+                              s));
+                HX(q1_vcycle(maxl - 1, always_, s));
+                HX(q1_up(maxl, always_, s));
+                if (skip_final) continue;
+                HX(defect(maxl, top.d, top.rhs, top.x, nrm, s));
+                HX(read_scalar(&h, nrm, s));
+                defn = (inner == VT_F64) ? std::sqrt(h) : (double)std::sqrt((float)h);
+                if (defn <= initial * cfg.tolerance) break;
+                continue;
+            }
             if (minl != maxl) {
                 bool started = true;
                 while (true) {
@@ -403,6 +515,100 @@ hipError_t MGHierarchy::solve_fixed(const void *b, void *x, hipStream_t s, int64
     return hipStreamSynchronize(s);
 }
 
+hipError_t MGHierarchy::alloc_outer_vectors(int64_t n) {
+    if (n64_ == n) return hipSuccess;
+    n64_ = 0;
+    for (double **p : {&guess_, &d64_, &res64_, &p64_, &q64_}) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+        HX(hipMalloc((void **)p, (size_t)n * sizeof(double)));
+    }
+    n64_ = n;
+    return hipSuccess;
+}
+
+namespace {
+
+// iterations (or outer steps) still needed at the convergence rate seen so
+// far, 1..8 per chunk
+int64_t chunk_needed(double rel, int64_t done, double tol) {
+    if (!(done > 0 && rel > 0.0 && rel < 1.0 && std::isfinite(rel))) return 1;
+    const double need = std::ceil(std::log(tol / rel) / (std::log(rel) / (double)done));
+    return need >= 8.0 ? 8 : (need > 1.0 ? (int64_t)need : 1);
+}
+
+}  // namespace
+
+// solve_pcg on a Q1 hierarchy: the same iteration, the confirmation of a
+// residual that met the tolerance once per chunk (the launches enqueued
+// behind it do nothing until then).
+hipError_t MGHierarchy::solve_pcg_q1(const double *b, double *x, hipStream_t s, int64_t *iters_out,
+                                     double *rel_defect) {
+    MGLevel &top = L[(size_t)max_level];
+    const Q1Outer o = q1_outer();
+    double *r = d64_, *p[2] = {p64_, res64_};
+    MgPcgScalars *sc = (MgPcgScalars *)(scal_ + 32);
+    const int cap = (int)(cfg.max_outer > 0 ? std::min<int64_t>(cfg.max_outer, 1 << 30) : 10000);
+    HX(boundary_guess(x, b, o.n, top.side, s));
+    HX(mg_pcg_defect(true, o, b, x, r, sc, slots_, cfg.tolerance, cap, s));
+    MgPcgScalars h{};
+    auto read_back = [&]() -> hipError_t {
+        HX(hipMemcpyAsync(&h, sc, sizeof(h), hipMemcpyDeviceToHost, s));
+        return hipStreamSynchronize(s);
+    };
+    int64_t chunk = 4;
+    for (int64_t k = 0;;) {
+        for (int64_t e = k + chunk; k < e; ++k) {
+            HX(mg_pcg_rhs(inner, top.rhs, r, o.n, sc, s));
+            HX(q1_vcycle(max_level, &sc->work, s));
+            HX(mg_pcg_outer(inner, o, top.x, x, r, p[k & 1], p[(k + 1) & 1], q64_, sc, slots_, s));
+        }
+        HX(mg_pcg_defect(false, o, b, x, r, sc, slots_, cfg.tolerance, cap, s));
+        HX(read_back());
+        if (h.done) break;
+        chunk = chunk_needed(h.initial > 0.0 ? h.nrm / h.initial : 1.0, h.iters, cfg.tolerance);
+    }
+    if (iters_out) *iters_out = h.iters;
+    if (rel_defect) *rel_defect = h.initial > 0 ? h.nrm / h.initial : 0.0;
+    return (h.initial > 0.0 && !(h.nrm < cfg.tolerance * h.initial)) ? hipErrorNotReady : hipSuccess;
+}
+
+// solve_mixed with one zero-start cycle per outer step on a Q1 hierarchy.
+hipError_t MGHierarchy::solve_mixed_q1(const double *b, double *x, hipStream_t s, int64_t *outer_out,
+                                       int64_t *inner_out, double *rel_defect) {
+    MGLevel &top = L[(size_t)max_level];
+    const Q1Outer o = q1_outer();
+    MgMixedScalars *sc = (MgMixedScalars *)(scal_ + 16);
+    static_assert(sizeof(MgMixedScalars) <= 16 * sizeof(double), "scalar record fits scal_[16..31]");
+    const int64_t cap = cfg.max_outer > 0 ? cfg.max_outer : 10000;
+    double *res[2] = {res64_, p64_};
+    HX(vcopy(guess_, x, o.n, VT_F64, s));
+    HX(boundary_guess(guess_, b, o.n, top.side, s));
+    HX(mg_defect(o, b, guess_, nullptr, nullptr, nullptr, d64_, slots_, nullptr, nullptr, s));
+    HX(mg_mixed_check(true, sc, o.n, slots_, cfg.tolerance, cap, s));
+    MgMixedScalars h{};
+    int64_t chunk = 4;
+    for (int64_t k = 0;;) {
+        for (int64_t e = k + chunk; k < e; ++k) {
+            HX(mg_mixed_rhs((float *)top.rhs, d64_, o.n, sc, s));
+            HX(q1_vcycle(max_level, &sc->work, s));
+            HX(mg_defect(o, b, k ? res[(k + 1) & 1] : nullptr, (const float *)top.x, &sc->scale, res[k & 1], d64_,
+                         slots_, &sc->done, nullptr, s));
+            HX(mg_mixed_check(false, sc, o.n, slots_, cfg.tolerance, cap, s));
+        }
+        HX(hipMemcpyAsync(&h, sc, sizeof(h), hipMemcpyDeviceToHost, s));
+        HX(hipStreamSynchronize(s));
+        if (h.done) break;
+        chunk = chunk_needed(h.initial > 0.0 ? h.norm / h.initial : 1.0, h.outer, cfg.tolerance);
+    }
+    HX(vcopy(x, res[(h.outer + 1) & 1], o.n, VT_F64, s));
+    HX(hipStreamSynchronize(s));
+    if (outer_out) *outer_out = h.outer;
+    if (inner_out) *inner_out = h.outer;
+    if (rel_defect) *rel_defect = h.initial > 0 ? h.norm / h.initial : 0.0;
+    return hipSuccess;
+}
+
 // FP64 conjugate gradients preconditioned by one V-cycle of the inner
 // hierarchy per iteration (z = |r| V(r / |r|), the cycle lean: from zero, no
 // inner norms).  Every scalar stays on the device (MgPcgScalars): the host
@@ -415,16 +621,10 @@ hipError_t MGHierarchy::solve_pcg(const double *b, double *x, hipStream_t s, int
     MGLevel &top = L[(size_t)max_level];
     if (!A_outer.Aj) return hipErrorInvalidValue;
     const int64_t n = top.n;
-    if (n64_ != n) {
-        for (double **p : {&guess_, &d64_, &res64_, &p64_, &q64_}) {
-            if (*p) (void)hipFree(*p);
-            *p = nullptr;
-            HX(hipMalloc((void **)p, (size_t)n * sizeof(double)));
-        }
-        n64_ = n;
-    }
+    HX(alloc_outer_vectors(n));
+    if (q1_cycle()) return solve_pcg_q1(b, x, s, iters_out, rel_defect);
     double *r = d64_, *z = res64_, *p = p64_, *q = q64_;
-    static_assert(sizeof(MgPcgScalars) <= 32 * sizeof(double), "scalar record fits scal_[32..63]");
+    static_assert(sizeof(MgPcgScalars) <= 28 * sizeof(double), "scalar record fits scal_[32..59]");
     MgPcgScalars *sc = (MgPcgScalars *)(scal_ + 32);
     const int cap = (int)(cfg.max_outer > 0 ? std::min<int64_t>(cfg.max_outer, 1 << 30) : 10000);
     // x0 with Dirichlet boundary values; r = b - A x0
@@ -508,14 +708,10 @@ hipError_t MGHierarchy::solve_mixed(const double *b, double *x, hipStream_t s, i
     MGLevel &top = L[(size_t)max_level];
     if (inner == VT_F64 || !A_outer.Aj) return hipErrorInvalidValue;
     const int64_t n = top.n;
-    if (n64_ != n) {
-        for (double **p : {&guess_, &d64_, &res64_, &p64_, &q64_}) {
-            if (*p) (void)hipFree(*p);
-            *p = nullptr;
-            HX(hipMalloc((void **)p, (size_t)n * sizeof(double)));
-        }
-        n64_ = n;
-    }
+    HX(alloc_outer_vectors(n));
+    if (q1_cycle() && cfg.n_max_iter == 1 && cfg.initial_zero && cfg.zero_inner_start && !cfg.convergence_check &&
+        !history)
+        return solve_mixed_q1(b, x, s, outer_out, inner_out, rel_defect);
     // x0 with Dirichlet boundary values, converted into the inner start vector
     HX(vcopy(guess_, x, n, VT_F64, s));
     HX(boundary_guess(guess_, b, n, top.side, s));

@@ -32,6 +32,10 @@ struct CGScalars {
 
 hipError_t cg_init(ValueType vt, CGScalars *sc, double eps_rel, int max_iters, hipStream_t s);
 
+// A batch work list (BWork) of one slot: slot 0 while end is 1, none at 0.
+struct OneSlot {
+    int32_t slot, first, end;
+};
 // Scalars of the multigrid-preconditioned CG of MGHierarchy::solve_pcg, kept
 // on the device: the host enqueues iterations in chunks and reads this
 // record once per chunk.  Once `done` is set no kernel of an iteration
@@ -45,6 +49,10 @@ struct MgPcgScalars {
     int32_t done;     // converged, broken down, non-finite or out of iterations
     int32_t verify;   // the recursive residual met the tolerance: the true defect decides
     int32_t iters, cap;
+    // solve_pcg on Q1 hierarchies: done or verify, no launch of an iteration
+    // does anything; the cycle's work list says the same
+    int32_t halt;
+    OneSlot work;
 };
 // Steps of one iteration (see MGHierarchy::solve_pcg): init after the first
 // defect; scale (rhs = r / |r|, FP32 or FP64 inner right-hand side); z =
@@ -56,6 +64,38 @@ hipError_t mgpcg_scale(ValueType inner, void *rhs, const double *r, int64_t n, c
                        hipStream_t s);
 hipError_t mgpcg_z(ValueType inner, double *z, const void *x, int64_t n, const MgPcgScalars *sc, hipStream_t s);
 hipError_t mgpcg_pupdate(double *p, const double *z, int64_t n, const MgPcgScalars *sc, hipStream_t s);
+
+// FP64 outer iterations on device-assembled Q1 hierarchies (mg_kernels.hip),
+// matrix-free: kappa null the constant operator, else the finest cells.
+struct Q1Outer {
+    int32_t side;
+    int64_t n;
+    const double *kappa;
+};
+// Scalars of MGHierarchy::solve_mixed kept on the device; once `done` is set
+// no launch of an outer iteration does anything.
+struct MgMixedScalars {
+    double initial, norm, scale, inv;
+    int32_t done, outer;
+    OneSlot work;   // of the cycle: empty once done
+};
+// d = b - A x and the partials of ||d||^2 (sl.partials); e non-null: x = (x
+// null: 0, else x) + e * *scale, also stored to xnew.  Nothing happens while
+// *skip is set or *gate is not.
+hipError_t mg_defect(const Q1Outer &o, const double *b, const double *x, const float *e, const double *scale,
+                     double *xnew, double *d, const ReduceSlots &sl, const int *skip, const int *gate, hipStream_t s);
+hipError_t mg_mixed_check(bool init, MgMixedScalars *sc, int64_t n, const ReduceSlots &sl, double tol, int64_t cap,
+                          hipStream_t s);
+hipError_t mg_mixed_rhs(float *rhs, const double *d, int64_t n, const MgMixedScalars *sc, hipStream_t s);
+// r = b - A x and its norm's decision: the start of the solve (init), or the
+// confirmation of a residual that met the tolerance (gated on sc->verify).
+hipError_t mg_pcg_defect(bool init, const Q1Outer &o, const double *b, const double *x, double *r, MgPcgScalars *sc,
+                         const ReduceSlots &sl, double tol, int cap, hipStream_t s);
+hipError_t mg_pcg_rhs(ValueType inner, void *rhs, const double *r, int64_t n, const MgPcgScalars *sc, hipStream_t s);
+// One iteration after its V-cycle (result x_top): r.z, direction and q = A p,
+// update, check.
+hipError_t mg_pcg_outer(ValueType inner, const Q1Outer &o, const void *x_top, double *x, double *r, const double *pold,
+                        double *pnew, double *q, MgPcgScalars *sc, const ReduceSlots &sl, hipStream_t s);
 
 // Host side of CGSolver (solvers_capi.cpp), shared by honei_hip_cg_solve and
 // its allocation-free variant: argument checks (HONEI status code), the
@@ -170,6 +210,7 @@ struct MGLevel {
     DevEll A, P, R;                 // P: prolongation into this level; R: restriction from it
     void *dinv = nullptr;           // omega / diag(A)
     void *c = nullptr, *d = nullptr, *rhs = nullptr, *x = nullptr, *t = nullptr;
+    double *kappa = nullptr;        // cell coefficients of a build_q1_coeff level
 };
 
 class MGHierarchy {
@@ -193,6 +234,10 @@ class MGHierarchy {
     // cells they cover (rediscretisation).
     hipError_t build_q1_coeff(double omega, const double *coeff_dev, int averaging, hipStream_t s);
 
+    // The levels and the outer system are no longer all as a build_q1* left
+    // them (a caller replaced one): no Q1 structure is assumed any more.
+    void forget_q1() { q1_ = false; }
+
     // One _multigrid_kernel call on the inner levels; returns the number of
     // V-cycles through *inner_iters.  rhs[max] and x[max] are inputs.
     hipError_t run_kernel(hipStream_t s, int64_t *inner_iters, double *final_defect);
@@ -211,9 +256,25 @@ class MGHierarchy {
     void *g_ = nullptr, *u_ = nullptr, *en_ = nullptr;   // coarse CG scratch
     int *iters_dev_ = nullptr;
     double *scal_ = nullptr;                            // device scalars
+    OneSlot *always_ = nullptr;     // device record, set for good (in scal_)
     double *guess_ = nullptr, *d64_ = nullptr, *res64_ = nullptr, *p64_ = nullptr, *q64_ = nullptr;
     int64_t n64_ = 0;
     bool mixed_inner_ = false;      // run_kernel called by the MIXED driver
+    bool q1_ = false;               // every level assembled on the device (build_q1*)
+    // The cycle can run as the batch solver's launches (q1_vcycle): Q1 levels
+    // from 1 up, two sweeps each way, bilinear transfers, unit correction,
+    // every border Dirichlet.
+    bool q1_cycle() const;
+    Q1Outer q1_outer() const;
+    // One V-cycle of levels 1..top from zero on L[top].rhs, result in
+    // L[top].x; work: a device record.
+    hipError_t q1_vcycle(int64_t top, const OneSlot *work, hipStream_t s);
+    // The up-leg of level l: L[l].x = J(J(x + P x_coarse)).
+    hipError_t q1_up(int64_t l, const OneSlot *work, hipStream_t s);
+    hipError_t alloc_outer_vectors(int64_t n);
+    hipError_t solve_pcg_q1(const double *b, double *x, hipStream_t s, int64_t *iters, double *rel_defect);
+    hipError_t solve_mixed_q1(const double *b, double *x, hipStream_t s, int64_t *outer, int64_t *inner,
+                              double *rel_defect);
     ReduceSlots slots_{};
     hipError_t smooth_from_zero(int64_t l, const void *rhs, void *out, void *acc, hipStream_t s);
     hipError_t sweeps(int64_t l, void *x, const void *rhs, int64_t count, hipStream_t s);

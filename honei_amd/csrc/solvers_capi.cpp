@@ -353,6 +353,7 @@ int honei_hip_mg_set_level(void *mg, size_t level, size_t rows, size_t stride, s
     MGHierarchy *h = (MGHierarchy *)mg;
     if ((int64_t)level < h->min_level || (int64_t)level > h->max_level)
         return fail(HONEI_HIP_ERROR_INVALID_ARGUMENT, "level out of range");
+    h->forget_q1();
     int st = upload_ell(h->L[level].A, h->inner, rows, rows, stride, ncpr, threads, Aj, Ax, Arl);
     if (st) return st;
     if ((st = check(h->alloc_level_vectors((int64_t)level, (int64_t)rows), "level vectors"))) return st;
@@ -368,7 +369,7 @@ int honei_hip_mg_set_transfer(void *mg, size_t level, int kind, size_t rows, siz
     MGHierarchy *h = (MGHierarchy *)mg;
     if ((int64_t)level <= h->min_level || (int64_t)level > h->max_level)
         return fail(HONEI_HIP_ERROR_INVALID_ARGUMENT, "transfer level out of range");
-    DevEll &M = kind == 0 ? h->L[level].P : h->L[level].R;
+    DevEll &M = kind == 0 ? h->L[level].P : h->L[level].R;   // used with prolmat only
     return upload_ell(M, h->inner, rows, cols, stride, ncpr, threads, Aj, Ax, Arl);
 }
 
@@ -376,6 +377,7 @@ int honei_hip_mg_set_outer(void *mg, size_t rows, size_t stride, size_t ncpr, si
                            const double *Ax, const uint64_t *Arl) {
     if (!mg) return fail(HONEI_HIP_ERROR_INVALID_ARGUMENT, "null argument");
     MGHierarchy *h = (MGHierarchy *)mg;
+    h->forget_q1();
     return upload_ell(h->A_outer, VT_F64, rows, rows, stride, ncpr, threads, Aj, Ax, Arl);
 }
 
