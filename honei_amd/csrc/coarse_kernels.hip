@@ -4,20 +4,24 @@
 // system's own right-hand side) to the correction it prolongs.
 //
 // Launch by launch these levels cost three launches each of 3-5 us in which
-// almost nothing runs.  Here vectors live in LDS and a node's weights with
-// the thread that owns the node: in registers from 33^2 nodes up (five nodes
-// a thread at 65^2), in LDS below.  Weights come from the cell coefficients
-// (or are the constant stencil), so no matrix is read.  Levels up to 9^2 and
-// the 3^2 CG run in one wavefront, without barriers; the CG's four sums and
-// two products per iteration are register moves between its nine lanes.  What
-// bounds it is the chain of phases (six per level, each an LDS round trip
-// and 18 dependent roundings per node) and the CG.
+// almost nothing runs.  Here vectors live in LDS, and each interior node's
+// weights, dinv and rhs with the thread that owns it, in registers (of the
+// levels that one wavefront runs: in LDS between their phases).  Weights come
+// from the cell coefficients (or are the constant stencil), so no matrix is
+// read; every global load of a system is issued before the first use.  Nodes
+// go row by row over the lanes, so a stencil is one LDS address and fixed
+// offsets, without a test for the boundary: below the finest level the
+// boundary's right-hand side and correction are 0 and it stays 0 in LDS; the
+// finest level's is a node of its own for a few threads.  Levels up to 9^2 and
+// the 3^2 CG run in one wavefront, without barriers; the CG's sums and products
+// are register moves between its nine lanes.
 //
-// 18 systems, levels 1..6: 23 us against 28-30 us for levels 1..4 in the
-// earlier one-launch form and six launches for levels 5 and 6; one system of
-// 257^2 nodes 26 us against 32 us and six launches.  256 systems of up to
-// 513^2 nodes: 26 us against 38 us and six launches.  Five nodes a thread with
-// positions kept across phases spilled 170 registers (45 us): `fresh`.
+// What bounds it: FP64 arithmetic of the weights (a quarter), VALU issue of
+// the 65^2 phases (a third), and the chain of short phases below.  One system
+// of 257^2 nodes 20.9 us; 18 systems, levels 1..6, 17.8 us; 256 systems of up
+// to 513^2 nodes 20.6 us.  (With flat node numbers, five a thread, and weights
+// in LDS below 33^2: 26.5, 22.8, 26.4; an earlier launch for levels 1..4 alone:
+// 32, 28, 38.)  Distinct weights read instead of formed: 21.8, 16.1, 22.2.
 //
 // Sums and roundings are those of the level-by-level launches: rows in column
 // order, boundary rows 0 + 1 x, transfers as k_b_restrict_rows /
@@ -35,54 +39,54 @@ namespace honei {
 namespace hipx {
 namespace {
 
-constexpr int kThreads = 1024;
+constexpr int kThreads = 1024, kWaves = kThreads / kWave;
 constexpr int kWaveTop = 3;    // levels up to here run in wavefront 0
-constexpr int kRegFrom = 5;    // levels from here keep weights, dinv and rhs in registers
 
 __host__ __device__ constexpr int side_at(int l) { return (1 << l) + 1; }
 __host__ __device__ constexpr int nodes_at(int l) { return side_at(l) * side_at(l); }
-// LDS, in elements: two vectors per level, then nine weights, dinv and rhs of
-// the levels below kRegFrom
+// LDS, in elements: the coarsest solution, then two vectors per level; behind
+// them what lanes without a node may read (never used)
 __host__ __device__ constexpr int vec_at(int l) {
-    int o = 0;
-    for (int k = 1; k < l; ++k) o += 2 * nodes_at(k);
+    int o = nodes_at(1);
+    for (int k = 2; k < l; ++k) o += 2 * nodes_at(k);
     return o;
 }
-__host__ __device__ constexpr int low_at(int l, int top) {
-    int o = vec_at(top + 1);
-    for (int k = 1; k < l; ++k) o += 11 * nodes_at(k);
-    return o;
-}
-__host__ __device__ constexpr int lds_elements(int top) { return low_at(kRegFrom < top + 1 ? kRegFrom : top + 1, top); }
+constexpr int kTail = 160;
+__host__ __device__ constexpr int lds_elements(int top) { return (vec_at(top + 1) + kTail + 3) / 4 * 4; }
 
+// Interior nodes over threads: a wavefront takes `rows` grid rows of `cols`
+// columns (a power of two, one more than the level's interior), the
+// work-group np times `step` rows.  So a node's stencil is one address and
+// fixed offsets.
 template <int L> struct Lv {
     static constexpr int side = side_at(L), n = nodes_at(L);
-    static constexpr bool wave = L <= kWaveTop, regs = L >= kRegFrom;
-    static constexpr int threads = wave ? kWave : kThreads;
-    static constexpr int np = (n + threads - 1) / threads;   // nodes per thread
+    static constexpr bool wave = L <= kWaveTop;
+    static constexpr int cols = 1 << L < kWave ? 1 << L : kWave, rows = kWave / cols;
+    static constexpr int waves = (1 << L) / rows < 1 ? 1 : ((1 << L) / rows < kWaves ? (1 << L) / rows : kWaves);
+    static constexpr int step = waves * rows, np = ((1 << L) + step - 1) / step;
+    static_assert((1 << L) <= cols, "one lane per column");
 };
 
-// what a thread keeps of its nodes of a register level
-template <typename V, int L> struct Regs {
-    V w[Lv<L>::np][9], di[Lv<L>::np], rh[Lv<L>::np];
+// what a thread keeps of its interior nodes: in registers; of the wavefront's
+// levels in LDS, in registers only while the level runs
+template <typename V, int NP> struct Regs {
+    V w[NP][9], di[NP], rh[NP];
 };
+// ... and what that is made from, as loaded (rhs used on the finest level only)
+template <typename V, int NP> struct Raw {
+    double c[NP][4];
+    V di[NP], rh[NP];
+};
+constexpr int kKeep = 11 * kWave;   // LDS elements of one of the wavefront's levels
 
-// Node q of this thread on level L (clamped to the last one) and the interior
-// node whose stencil fits its position.
-template <int L> struct Node {
-    int id, base;
-    bool live, bnd;
-    __device__ inline Node(int t, int q) {
-        constexpr int S = Lv<L>::side;
-        const int i = t + q * Lv<L>::threads;
-        live = i < Lv<L>::n;
-        id = live ? i : Lv<L>::n - 1;
-        const int r = id / S, c = id - r * S;
-        bnd = r == 0 || c == 0 || r == S - 1 || c == S - 1;
-        const int ir = r < 1 ? 1 : (r > S - 2 ? S - 2 : r), ic = c < 1 ? 1 : (c > S - 2 ? S - 2 : c);
-        base = ir * S + ic;
-    }
-};
+
+// The lane as a phase sees it: positions, masks and addresses formed from it
+// are formed in the phase again (a few instructions) instead of being kept in
+// registers from one phase to the others.
+__device__ inline int fresh(int t) {
+    asm volatile("" : "+v"(t));
+    return t;
+}
 
 template <int L> __device__ inline void level_sync() {
     if constexpr (Lv<L>::wave) {
@@ -106,117 +110,139 @@ template <typename V> __device__ inline V lane_value(V v, int lane) {
     }
 }
 
-// The thread index as a phase sees it: positions, masks and addresses formed
-// from it are formed in the phase again (a few instructions) instead of being
-// kept in registers from one phase to the others.
-__device__ inline int fresh(int t) {
-    asm volatile("" : "+v"(t));
-    return t;
-}
+// Node 0 of this thread on level L: grid position and LDS index; node q is
+// q * Lv<L>::step rows further.
+template <int L> struct Pos {
+    int r, c, id;
+    bool mine;   // the wavefront takes part
+    __device__ inline Pos(int lane_, int wv) {
+        const int lane = fresh(lane_);
+        r = 1 + wv * Lv<L>::rows + lane / Lv<L>::cols;
+        c = 1 + lane % Lv<L>::cols;
+        id = r * Lv<L>::side + c;
+        mine = wv < Lv<L>::waves;
+    }
+    __device__ inline bool live(int q) const {
+        return c < Lv<L>::side - 1 && r + q * Lv<L>::step < Lv<L>::side - 1;
+    }
+};
 
 template <typename VT, bool COEF, int TOP> struct Cycle {
     typedef typename VecOf<VT>::type V;
     V *mem;
-    int t;           // thread of the work-group
+    int lane, wv;    // of this thread
     bool odd_pre;    // an odd number of sweeps follows the first two: the iterate ends in the second vector
     const CoarseCycle &cc;
+    // the finest level's boundary node of this thread (id < 0: none); on the
+    // other levels the boundary stays 0: right-hand side and correction are
+    int bid;
+    V bdi, brh;
 
     template <int L> __device__ inline V *iterate() const { return mem + vec_at(L) + (odd_pre ? Lv<L>::n : 0); }
     template <int L> __device__ inline V *other() const { return mem + vec_at(L) + (odd_pre ? 0 : Lv<L>::n); }
-    template <int L> __device__ inline V *low() const { return mem + low_at(L, TOP); }
     // where the level's result is after the up-leg
     template <int L> __device__ inline const V *result() const {
-        if constexpr (L == 1) return mem + vec_at(1);
+        if constexpr (L == 1) return mem;
         return (cc.n_post & 1) ? iterate<L>() : other<L>();
     }
 
-    // weights and dinv of the level's nodes; top: its right-hand side too
-    template <int L, typename R> __device__ inline void load(R &reg, int64_t g, bool top) const {
+    // cells, dinv and rhs of the thread's nodes as wavefront v of the level's
+    template <int L> __device__ inline void fetch(Raw<V, Lv<L>::np> &raw, int64_t g, int v) const {
+        constexpr int S = Lv<L>::side;
         const CoarseLevel &cl = cc.lv[L];
+        const Pos<L> p(lane, v);
+        if (!p.mine) return;
         const V *dinv = (const V *)cl.dinv + g * cl.vld, *rhs = (const V *)cl.rhs + g * cl.vld;
-        constexpr int S = Lv<L>::side, NP = Lv<L>::regs ? Lv<L>::np : 1;
-        const int t = fresh(this->t);
+        const double *kap = cl.kappa + g * cl.kld;
 #pragma unroll
-        for (int q = 0; q < NP; ++q) {
-            const int i = t + q * kThreads;
-            if (!Lv<L>::regs && i >= Lv<L>::n) break;
-            const int id = i < Lv<L>::n ? i : Lv<L>::n - 1, r = id / S, c = id - r * S;
-            V w[9];
+        for (int q = 0; q < Lv<L>::np; ++q) {
+            // a lane without a node: the last interior one's
+            const int r = min(p.r + q * Lv<L>::step, S - 2), c = min(p.c, S - 2);
             if constexpr (COEF) {
-                const int ir = r < 1 ? 1 : (r > S - 2 ? S - 2 : r), ic = c < 1 ? 1 : (c > S - 2 ? S - 2 : c);
-                const double *cs = cl.kappa + g * cl.kld + ((ir - 1) * (S - 1) + ic - 1), *cs2 = cs + (S - 1);
-                q1_interior_weights_cells<VT, V>(cs[0], cs[1], cs2[0], cs2[1], w);
-            } else {
-                q1_constant_weights<VT, V>(w);
+                const double *cs = kap + ((r - 1) * (S - 1) + c - 1), *cs2 = cs + (S - 1);
+                raw.c[q][0] = cs[0];
+                raw.c[q][1] = cs[1];
+                raw.c[q][2] = cs2[0];
+                raw.c[q][3] = cs2[1];
             }
-            const V di = dinv[id], rh = top ? rhs[id] : V(0);
-            if constexpr (Lv<L>::regs) {
-#pragma unroll
-                for (int k = 0; k < 9; ++k) reg.w[q][k] = w[k];
-                reg.di[q] = di;
-                reg.rh[q] = rh;
-            } else {
-                V *lo = low<L>();
-#pragma unroll
-                for (int k = 0; k < 9; ++k) lo[k * Lv<L>::n + id] = w[k];
-                lo[9 * Lv<L>::n + id] = di;
-                lo[10 * Lv<L>::n + id] = rh;
-            }
-            if (L > 1 && top && i < Lv<L>::n) (mem + vec_at(L) + Lv<L>::n)[id] = di * rh;
+            raw.di[q] = dinv[r * S + c];
+            raw.rh[q] = rhs[r * S + c];
         }
+    }
+    // weights; on the finest level the first operand dinv .* rhs
+    template <int L>
+    __device__ inline void settle(Regs<V, Lv<L>::np> &reg, const Raw<V, Lv<L>::np> &raw, bool top, int v) const {
+        const Pos<L> p(lane, v);
+        if (!p.mine) return;
+#pragma unroll
+        for (int q = 0; q < Lv<L>::np; ++q) {
+            if constexpr (COEF)
+                q1_interior_weights_cells<VT, V>(raw.c[q][0], raw.c[q][1], raw.c[q][2], raw.c[q][3], reg.w[q]);
+            reg.di[q] = raw.di[q];
+            reg.rh[q] = raw.rh[q];
+            if (top && p.live(q))
+                (mem + vec_at(L) + Lv<L>::n)[p.id + q * Lv<L>::step * Lv<L>::side] = raw.di[q] * raw.rh[q];
+        }
+    }
+
+    // the wavefront's levels: put away and taken back by their lanes
+    template <int L> __device__ inline V *kept() const { return mem + lds_elements(TOP) + (L - 2) * kKeep + lane; }
+    template <int L> __device__ inline void put(const Regs<V, Lv<L>::np> &reg) const {
+        V *k = kept<L>();
+        if constexpr (COEF) {
+#pragma unroll
+            for (int i = 0; i < 9; ++i) k[i * kWave] = reg.w[0][i];
+        }
+        k[9 * kWave] = reg.di[0];
+        k[10 * kWave] = reg.rh[0];
+    }
+    template <int L> __device__ inline void get(Regs<V, Lv<L>::np> &reg) const {
+        const V *k = kept<L>();
+        if constexpr (COEF) {
+#pragma unroll
+            for (int i = 0; i < 9; ++i) reg.w[0][i] = k[i * kWave];
+        }
+        reg.di[0] = k[9 * kWave];
+        reg.rh[0] = k[10 * kWave];
     }
 
     // DEFECT: dst = rhs - A src; else a Jacobi sweep (from zero: src = dinv .* rhs)
-    template <int L, bool DEFECT, typename R>
-    __device__ inline void sweep(const V *src, V *dst, const R &reg) const {
+    template <int L, bool DEFECT> __device__ inline void sweep(const V *src, V *dst, const Regs<V, Lv<L>::np> &reg, bool top) const {
         constexpr int S = Lv<L>::side;
-        const int t = fresh(this->t);
+        const Pos<L> p(lane, wv);
+        if (p.mine) {
+            src += p.id;
 #pragma unroll
-        for (int q = 0; q < Lv<L>::np; ++q) {
-            const Node<L> nd(t, q);
-            V x[9], s = V(0), di, rh;
+            for (int q = 0; q < Lv<L>::np; ++q) {
+                constexpr int Q = Lv<L>::step * S;
+                V x[9], w[9], s = V(0);
 #pragma unroll
-            for (int k = 0; k < 9; ++k) x[k] = src[k == 4 ? nd.id : nd.base + (k / 3 - 1) * S + (k % 3 - 1)];
-            if constexpr (Lv<L>::regs) {
-                if constexpr (COEF) {
+                for (int k = 0; k < 9; ++k) x[k] = src[q * Q + (k / 3 - 1) * S + (k % 3 - 1)];
+                if constexpr (!COEF) q1_constant_weights<VT, V>(w);
 #pragma unroll
-                    for (int k = 0; k < 9; ++k) s = s + reg.w[q][k] * x[k];
-                }
-                di = reg.di[q];
-                rh = reg.rh[q];
-            } else {
-                const V *lo = low<L>() + nd.id;
-                if constexpr (COEF) {
-#pragma unroll
-                    for (int k = 0; k < 9; ++k) s = s + lo[k * Lv<L>::n] * x[k];
-                }
-                di = lo[9 * Lv<L>::n];
-                rh = lo[10 * Lv<L>::n];
+                for (int k = 0; k < 9; ++k) s = s + (COEF ? reg.w[q][k] : w[k]) * x[k];
+                const V d = reg.rh[q] - s;
+                if (p.live(q)) dst[p.id + q * Q] = DEFECT ? d : x[4] + d * reg.di[q];
             }
-            if constexpr (!COEF) {
-                V w[9];
-                q1_constant_weights<VT, V>(w);
-#pragma unroll
-                for (int k = 0; k < 9; ++k) s = s + w[k] * x[k];
-            }
-            s = nd.bnd ? V(0) + V(1) * x[4] : s;
-            const V d = rh - s;
-            if (nd.live) dst[nd.id] = DEFECT ? d : x[4] + d * di;
+            src -= p.id;
+        }
+        if (top && bid >= 0) {
+            const V x = src[bid], d = brh - (V(0) + V(1) * x);
+            dst[bid] = DEFECT ? d : x + d * bdi;
         }
     }
 
-    // the right-hand side of level L - 1 from the defect of level L, and its
-    // first operand dinv .* rhs
-    template <int L, typename R> __device__ inline void restrict_to_coarser(R &reg) const {
-        constexpr int C = L - 1, S = Lv<L>::side, m = Lv<C>::side - 1;
-        const V *f = other<L>();
-        const int t = fresh(this->t);
+    // the right-hand side of level C from the defect of the finer one (its
+    // border is Dirichlet: 0), value(q, s) taking node q's
+    template <int C, typename F> __device__ inline void restrict_to(F &&value) const {
+        constexpr int SF = Lv<C + 1>::side;
+        const Pos<C> p(lane, wv);
+        if (!p.mine) return;
+        const V *f = other<C + 1>() + 2 * p.r * SF + 2 * p.c;
 #pragma unroll
         for (int q = 0; q < Lv<C>::np; ++q) {
-            const Node<C> nd(t, q);
-            const int ir = nd.base / Lv<C>::side, ic = nd.base - ir * Lv<C>::side;
-            const int d = ic - ir;
-            const V *f0 = f + 2 * ir * S + 2 * ic, *fm = f0 - S, *fp = f0 + S;
+            const V *f0 = f + q * 2 * Lv<C>::step * SF, *fm = f0 - SF, *fp = f0 + SF;
+            const int d = p.c - (p.r + q * Lv<C>::step);
             const V h = V(0.5), qq = V(0.25);
             const V A_ = h * fm[0], B_ = h * fp[0], C_ = h * f0[1], D_ = h * f0[-1];
             const V E_ = qq * fp[1], F_ = qq * fp[-1], G_ = qq * fm[1], H_ = qq * fm[-1];
@@ -235,72 +261,64 @@ template <typename VT, bool COEF, int TOP> struct Cycle {
             s = s + F_;
             s = d >= 2 ? s + D_ : s;
             s = d >= 1 ? s + C_ : s;
-            s = nd.bnd ? V(0) : s;
-            static_assert(m >= 2, "coarse grids have an interior");
-            V di;
-            if constexpr (Lv<C>::regs) {
-                reg.rh[q] = s;
-                di = reg.di[q];
-            } else {
-                V *lo = low<C>() + nd.id;
-                if (nd.live) lo[10 * Lv<C>::n] = s;
-                di = lo[9 * Lv<C>::n];
-            }
-            if (C > 1 && nd.live) (mem + vec_at(C) + Lv<C>::n)[nd.id] = di * s;
+            value(q, s);
         }
     }
+    template <int C> __device__ inline void restrict_to_level(Regs<V, Lv<C>::np> &reg) const {
+        const Pos<C> p(lane, wv);
+        restrict_to<C>([&](int q, V s) {
+            reg.rh[q] = s;
+            if (p.live(q)) (mem + vec_at(C) + Lv<C>::n)[p.id + q * Lv<C>::step * Lv<C>::side] = reg.di[q] * s;
+        });
+    }
 
-    // from the level's rhs and first operand to the coarser level's
-    template <int L, typename R, typename RC> __device__ inline void down(const R &reg, RC &rc) const {
+    // from the level's rhs and first operand to its defect
+    template <int L> __device__ inline void down(const Regs<V, Lv<L>::np> &reg, bool top) const {
         V *x = mem + vec_at(L), *y = x + Lv<L>::n;
-        sweep<L, false>(y, x, reg);
+        sweep<L, false>(y, x, reg, top);
         level_sync<L>();
         for (int k = 2; k < cc.n_pre; ++k) {
-            sweep<L, false>((k & 1) ? y : x, (k & 1) ? x : y, reg);
+            sweep<L, false>((k & 1) ? y : x, (k & 1) ? x : y, reg, top);
             level_sync<L>();
         }
-        sweep<L, true>(iterate<L>(), other<L>(), reg);
+        sweep<L, true>(iterate<L>(), other<L>(), reg, top);
         level_sync<L>();
-        if constexpr (Lv<L - 1>::wave == Lv<L>::wave) {
-            restrict_to_coarser<L>(rc);
-            level_sync<L>();
-        }
     }
 
-    template <int L, typename R> __device__ inline void up(const R &reg) const {
-        constexpr int S = Lv<L>::side, nc = Lv<L - 1>::side;
+    template <int L> __device__ inline void up(const Regs<V, Lv<L>::np> &reg, bool top) const {
+        constexpr int nc = Lv<L - 1>::side;
         V *a = other<L>(), *b = iterate<L>();
         const V *xc = result<L - 1>();
-        const int t = fresh(this->t);
+        const Pos<L> p(lane, wv);
+        if (p.mine) {
 #pragma unroll
-        for (int q = 0; q < Lv<L>::np; ++q) {
-            const Node<L> nd(t, q);
-            const int r = nd.id / S, c = nd.id - r * S;
-            const int rlo = r >> 1, rhi = (r + 1) >> 1, clo = c >> 1, chi = (c + 1) >> 1;
-            const V t0 = xc[rlo * nc + clo], t1 = xc[rlo * nc + chi], t2 = xc[rhi * nc + clo], t3 = xc[rhi * nc + chi];
-            const V h = V(0.5), qq = V(0.25);
-            const V f_rc = ((V(0) + t0 * qq + t1 * qq) + t2 * qq) + t3 * qq;
-            const V f_c = (V(0) + t0 * h) + t1 * h, f_r = (V(0) + t0 * h) + t2 * h;
-            V f = (r & 1) ? ((c & 1) ? f_rc : f_r) : ((c & 1) ? f_c : t0);
-            f = nd.bnd ? V(0) : f;
-            const V v = b[nd.id] + f * V(1);
-            if (nd.live) a[nd.id] = v;
+            for (int q = 0; q < Lv<L>::np; ++q) {
+                const int r = p.r + q * Lv<L>::step, c = p.c, id = p.id + q * Lv<L>::step * Lv<L>::side;
+                const V *c0 = xc + (r >> 1) * nc + (c >> 1), *c1 = xc + ((r + 1) >> 1) * nc + (c >> 1);
+                const int dc = c & 1;
+                const V t0 = c0[0], t1 = c0[dc], t2 = c1[0], t3 = c1[dc];
+                const V h = V(0.5), qq = V(0.25);
+                const V f_rc = ((V(0) + t0 * qq + t1 * qq) + t2 * qq) + t3 * qq;
+                const V f_c = (V(0) + t0 * h) + t1 * h, f_r = (V(0) + t0 * h) + t2 * h;
+                const V f = (r & 1) ? ((c & 1) ? f_rc : f_r) : ((c & 1) ? f_c : t0);
+                const V v = b[id] + f * V(1);
+                if (p.live(q)) a[id] = v;
+            }
         }
+        if (top && bid >= 0) a[bid] = b[bid] + V(0) * V(1);
         level_sync<L>();
         for (int k = 0; k < cc.n_post; ++k) {
-            sweep<L, false>((k & 1) ? b : a, (k & 1) ? a : b, reg);
+            sweep<L, false>((k & 1) ? b : a, (k & 1) ? a : b, reg, top);
             level_sync<L>();
         }
     }
 
-    // coarse_cg_block on the 3 x 3 grid by wavefront 0, lane = node
-    __device__ inline void coarse_cg() const {
+    // coarse_cg_block on the 3 x 3 grid by wavefront 0, lane = node; rhs: the
+    // centre's (the border's is 0), w: the centre row (the others are 0 + 1 x)
+    __device__ inline void coarse_cg(V centre, const V (&w)[9]) const {
+        const int t = lane;
         const bool in = t < 9;
-        const V *lo = low<1>();
-        V w[9];
-#pragma unroll
-        for (int k = 0; k < 9; ++k) w[k] = lo[k * 9 + 4];   // the centre row; the others are 0 + 1 x
-        const V rhs = in ? lo[90 + t] : V(0);
+        const V rhs = t == 4 ? centre : V(0);
         const V e = eps_of<V>();
         auto mul = [&](V v) {
             V s = V(0);
@@ -330,65 +348,138 @@ template <typename VT, bool COEF, int TOP> struct Cycle {
             norm_x_last = norm_x;
             norm_x = sum(x, x);
         }
-        if (in) (mem + vec_at(1))[t] = x;
+        if (in) mem[t] = x;
     }
 };
-
-struct None {};
 
 template <typename VT, bool COEF, int TOP>
 __global__ __launch_bounds__(kThreads) void k_coarse_cycle(CoarseCycle cc, BWork w) {
     typedef typename VecOf<VT>::type V;
-    __shared__ V mem[lds_elements(TOP)];
+    __shared__ __attribute__((aligned(16))) V mem[lds_elements(TOP) + 2 * kKeep + 12];
     const int64_t a0 = w.bounds[w.lo], na = w.bounds[w.hi] - w.bounds[w.lo];
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t % kWave, wv = __builtin_amdgcn_readfirstlane(t / kWave);
     for (int64_t a = blockIdx.x; a < na; a += gridDim.x) {
         const int64_t g = w.list[a0 + a];
         int top = cc.top;
-        while (top > 1 && g >= cc.lv[top].cap) --top;   // systems whose finest level is lower
-        const Cycle<VT, COEF, TOP> c{mem, t, (cc.n_pre & 1) != 0, cc};
-        None no;
-        Regs<V, 5> r5;
-        Regs<V, TOP >= 6 ? 6 : 5> r6;
+        while (top > 2 && g >= cc.lv[top].cap) --top;   // systems whose finest level is lower
+        Cycle<VT, COEF, TOP> c{mem, lane, wv, (cc.n_pre & 1) != 0, cc, -1, V(0), V(0)};
+        const CoarseLevel &cl = cc.lv[top];
+        // every global load of the system before the first use (initialised:
+        // else what a branch leaves unset lives on from system to system)
+        Raw<V, Lv<TOP >= 6 ? 6 : 5>::np> f6{};
+        Raw<V, 1> f5{}, f4{}, fw{};
         if constexpr (TOP >= 6) {
-            if (top >= 6) c.template load<6>(r6, g, top == 6);
+            if (top >= 6) c.template fetch<6>(f6, g, wv);
         }
-        if (top >= 5) c.template load<5>(r5, g, top == 5);
-        if (top >= 4) c.template load<4>(no, g, top == 4);
-        if (top >= 3) c.template load<3>(no, g, top == 3);
-        if (top >= 2) c.template load<2>(no, g, top == 2);
-        c.template load<1>(no, g, top == 1);
-        __syncthreads();
-        if constexpr (TOP >= 6) {
-            if (top >= 6) c.template down<6>(r6, r5);
-        }
-        if (top >= 5) c.template down<5>(r5, no);
-        if (top >= 4) c.template down<4>(no, no);
-        if (t < kWave) {
-            if (top >= 4) {
-                c.template restrict_to_coarser<4>(no);
-                level_sync<3>();
+        if (top >= 5) c.template fetch<5>(f5, g, wv);
+        if (top >= 4) c.template fetch<4>(f4, g, wv);
+        // wavefronts 1 and 2 make wavefront 0's levels, 3 the centre row of level 1
+        if (wv == 1 && top >= 3) c.template fetch<3>(fw, g, 0);
+        if (wv == 2) c.template fetch<2>(fw, g, 0);
+        if constexpr (COEF) {
+            if (wv == 3) {
+                const double *k = cc.lv[1].kappa + g * cc.lv[1].kld;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) fw.c[0][i] = k[i];
             }
-            if (top >= 3) c.template down<3>(no, no);
-            if (top >= 2) c.template down<2>(no, no);
-            c.coarse_cg();
-            level_sync<1>();
-            if (top >= 2) c.template up<2>(no);
-            if (top >= 3) c.template up<3>(no);
+        }
+        // the finest level's boundary: bottom, top, left, right without corners twice
+        const int e = (1 << top), side = e + 1;
+        if (t < 4 * e) {
+            const int k = t & (e - 1), part = t >> top;
+            c.bid = part == 0 ? k : (part == 1 ? e * side + k + 1 : (part == 2 ? (k + 1) * side : k * side + e));
+            c.bdi = ((const V *)cl.dinv + g * cl.vld)[c.bid];
+            c.brh = ((const V *)cl.rhs + g * cl.vld)[c.bid];
+        }
+        for (int i = t; i < lds_elements(TOP) / 4; i += kThreads) {
+            V *m = mem + 4 * i;
+            m[0] = m[1] = m[2] = m[3] = V(0);
         }
         __syncthreads();
-        if (top >= 4) c.template up<4>(no);
-        if (top >= 5) c.template up<5>(r5);
+        if (wv >= 1 && wv <= 3) {
+            Regs<V, 1> rw{};
+            if (wv == 1 && top >= 3) {
+                c.template settle<3>(rw, fw, top == 3, 0);
+                c.template put<3>(rw);
+            }
+            if (wv == 2) {
+                c.template settle<2>(rw, fw, top == 2, 0);
+                c.template put<2>(rw);
+            }
+            if (wv == 3) {
+                if constexpr (COEF)
+                    q1_interior_weights_cells<VT, V>(fw.c[0][0], fw.c[0][1], fw.c[0][2], fw.c[0][3], rw.w[0]);
+                else
+                    q1_constant_weights<VT, V>(rw.w[0]);
+#pragma unroll
+                for (int k = 0; k < 9; ++k) mem[lds_elements(TOP) + 2 * kKeep + k] = rw.w[0][k];
+            }
+        }
+        Regs<V, Lv<TOP >= 6 ? 6 : 5>::np> r6{};
+        Regs<V, 1> r5{}, r4{};
+        if (top >= 4) c.template settle<4>(r4, f4, top == 4, wv);
+        if (top >= 5) c.template settle<5>(r5, f5, top == 5, wv);
         if constexpr (TOP >= 6) {
-            if (top >= 6) c.template up<6>(r6);
+            if (top >= 6) c.template settle<6>(r6, f6, top == 6, wv);
+        }
+        if (c.bid >= 0) mem[cl.at + cl.n + c.bid] = c.bdi * c.brh;
+        __syncthreads();
+        if constexpr (TOP >= 6) {
+            if (top >= 6) {
+                c.template down<6>(r6, top == 6);
+                c.template restrict_to_level<5>(r5);
+                __syncthreads();
+            }
+        }
+        if (top >= 5) {
+            c.template down<5>(r5, top == 5);
+            c.template restrict_to_level<4>(r4);
+            __syncthreads();
+        }
+        if (top >= 4) c.template down<4>(r4, top == 4);
+        if (wv == 0) {
+            if (top >= 3) {
+                Regs<V, 1> r3{};
+                c.template get<3>(r3);
+                if (top >= 4) {
+                    c.template restrict_to_level<3>(r3);
+                    c.template put<3>(r3);
+                    level_sync<3>();
+                }
+                c.template down<3>(r3, top == 3);
+            }
+            {
+                Regs<V, 1> r2{};
+                c.template get<2>(r2);
+                if (top >= 3) {
+                    c.template restrict_to_level<2>(r2);
+                    level_sync<2>();
+                }
+                c.template down<2>(r2, top == 2);
+                V centre = V(0), w1[9];
+                c.template restrict_to<1>([&](int, V s) { centre = s; });
+#pragma unroll
+                for (int k = 0; k < 9; ++k) w1[k] = mem[lds_elements(TOP) + 2 * kKeep + k];
+                c.coarse_cg(lane_value(centre, 0), w1);
+                level_sync<1>();
+                c.template up<2>(r2, top == 2);
+            }
+            if (top >= 3) {
+                Regs<V, 1> r3{};
+                c.template get<3>(r3);
+                c.template up<3>(r3, top == 3);
+            }
+        }
+        __syncthreads();
+        if (top >= 4) c.template up<4>(r4, top == 4);
+        if (top >= 5) c.template up<5>(r5, top == 5);
+        if constexpr (TOP >= 6) {
+            if (top >= 6) c.template up<6>(r6, top == 6);
         }
         // the finest level's result
-        const CoarseLevel &cl = cc.lv[top];
         V *out = (V *)cl.x + g * cl.vld;
-        const int n = cl.n, at = cc.lv[top].at;
-        const bool first = top == 1 || (((cc.n_pre ^ cc.n_post) & 1) != 0);
-        const V *src = mem + at + (first ? 0 : n);
-        for (int i = t; i < n; i += kThreads) out[i] = src[i];
+        const V *src = mem + cl.at + (((cc.n_pre ^ cc.n_post) & 1) ? 0 : cl.n);
+        for (int i = t; i < cl.n; i += kThreads) out[i] = src[i];
         __syncthreads();
     }
 }
@@ -399,7 +490,7 @@ int64_t coarse_top(ValueType vt) { return vt == VT_F64 ? 5 : 6; }
 
 hipError_t b_coarse_cycle(ValueType vt, const CoarseCycle &cc, const BWork &w, int64_t max_slots, hipStream_t s) {
     if (max_slots <= 0) return hipSuccess;
-    if (cc.top < 1 || cc.top > coarse_top(vt) || cc.n_pre < 2 || cc.n_post < 0) return hipErrorInvalidValue;
+    if (cc.top < 2 || cc.top > coarse_top(vt) || cc.n_pre < 2 || cc.n_post < 0) return hipErrorInvalidValue;
     CoarseCycle c = cc;
     const bool coef = cc.lv[1].kappa != nullptr;
     for (int l = 1; l <= cc.top; ++l) {
