@@ -68,8 +68,10 @@ constexpr int kMaxClasses = 16;
 // Paired row passes (b_pair): tiles of at most kPairWidth columns (62 + a
 // halo column each side fill a wavefront) and kPairRows rows (kPairTileRows
 // with the halo, one wavefront per row: 1024-thread work-groups), on levels
-// from kPairMinSide^2 nodes up; from kPairTallMinSide^2 nodes up every thread
-// takes two grid rows (tiles of 2 kPairTileRows - 2 rows).  The CG direction
+// from kPairMinSide^2 nodes up; launches with many tiles of systems from
+// kPairTallMinSide^2 nodes up march down columns (k_b_stream) or, with stored
+// weights, take two grid rows per thread (tiles of 2 kPairTileRows - 2 rows).
+// The CG direction
 // launch tiles the finest grids in the same column strips and bands of
 // kDirRows rows (kDirNodes grid rows per thread).
 enum PairKind { PAIR_PRE = 0, PAIR_POST = 1 };
@@ -462,6 +464,10 @@ hipError_t b_prolong_axpy(ValueType vt, const BLevel &fine, const BLevel &coarse
 hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void *out0, void *out1,
                   const void *xin, hipStream_t s, int wmode = 0, const BLevel *coarse = nullptr,
                   const void *xc = nullptr);
+// The same passes, one wavefront marching down a column strip (k_b_stream):
+// b_pair's launch for large levels, after its checks (wmode 1 or 3).
+hipError_t b_pair_stream(ValueType vt, int pair, const BLevel &lv, const BWork &w, void *out0, void *out1,
+                         const void *xin, hipStream_t s, int wmode, const void *xc, int64_t vld_c);
 // The distinct-weight arrays of `count` slots of a side x side level from
 // their cell coefficients (kappa + g kld, st + g 4 vld).
 hipError_t b_stencil_fill(ValueType vt, int64_t side, const double *kappa, int64_t kld, void *st, int64_t vld,

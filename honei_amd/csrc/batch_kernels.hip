@@ -1430,7 +1430,8 @@ void pair_launch_rows(dim3 grid, dim3 block, hipStream_t s, const BMat &m, const
                       void *out0, void *out1, const void *x, const void *rhs, const void *dinv, const void *xc,
                       int64_t vld_c, int nr) {
     typedef typename VecOf<VT>::type V;
-    if constexpr (sizeof(V) == 4) {   // FP64 vectors: two rows per thread would spill
+    // FP64 vectors: two rows per thread would spill; other weights: b_pair_stream
+    if constexpr (sizeof(V) == 4 && (WM == 0 || WM == 2)) {
         if (nr == 2) {
             hipLaunchKernelGGL((k_b_pair<VT, P, WM, FP, 2>), grid, block, 0, s, m, w, pg, (V *)out0, (V *)out1,
                                (const V *)x, (const V *)rhs, (const V *)dinv, (const V *)xc, vld_c);
@@ -1472,11 +1473,19 @@ hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void
     pg.side = (int32_t)lv.side;
     pg.strips = (int32_t)((lv.side + kPairWidth - 1) / kPairWidth);
     pg.width = (int32_t)((lv.side + pg.strips - 1) / pg.strips);
-    // two grid rows per thread on the larger levels (taller tiles: half the
-    // halo rows per node, twice the loads in flight per thread)
-    int nr = lv.side >= kPairTallMinSide && vt != VT_F64 ? 2 : 1;
-    if (nr == 2 && lv.cap * pg.strips * ((lv.side + 2 * kPairTileRows - 3) / (2 * kPairTileRows - 2)) < kMinTallTiles)
-        nr = 1;
+    // launches of at least kMinTallTiles tall tiles: with weights that come
+    // from the cells or the constant operator, the column march (by total
+    // nodes, 129^2 systems, FP32, PRE / POST, tile against march in us: 0.27 M
+    // 6.7 / 6.7 and 7.2 / 6.6, 0.53 M 10.8 / 9.1 and 8.5 / 8.4; FP64, 1.07 M
+    // 17.2 / 20.9 and 15.2 / 16.6); with stored weights two grid rows per
+    // thread (taller tiles: half the halo rows per node, twice the loads in
+    // flight per thread)
+    const int64_t tall_rows = 2 * kPairTileRows - 2;
+    const bool tall = lv.side >= kPairTallMinSide &&
+                      lv.cap * pg.strips * ((lv.side + tall_rows - 1) / tall_rows) >= kMinTallTiles;
+    if (tall && (wmode == 1 || wmode == 3))
+        return b_pair_stream(vt, pair, lv, w, out0, out1, xin, s, wmode, xc, vld_c);
+    const int nr = tall && vt != VT_F64 ? 2 : 1;
     const int64_t rows = (int64_t)kPairTileRows * nr - 2;
     pg.segs = (int32_t)((lv.side + rows - 1) / rows);
     if (lv.cap <= 0) return hipSuccess;

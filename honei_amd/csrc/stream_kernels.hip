@@ -1,0 +1,320 @@
+// stream_kernels.hip -- the paired row passes of large Q1 levels, one
+// wavefront marching down a column strip.
+#include "batch.hh"
+#include "q1_device.hh"
+
+namespace honei {
+namespace hipx {
+namespace {
+
+// The lane to the left's / right's value (lane 0 / lane 63: zero).
+template <int CTRL>
+__device__ inline float lane_shift(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ inline double lane_shift(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+template <typename T> __device__ inline T from_west(T v) { return lane_shift<0x138>(v); }
+template <typename T> __device__ inline T from_east(T v) { return lane_shift<0x130>(v); }
+
+// A strip is at most kStreamWidth columns (two halo columns each side fill a
+// wavefront), a segment kStreamRows rows; kStreamShortRows where the running
+// systems give fewer than kStreamFill long segments (four wavefronts a SIMD),
+// so that few systems still spread over the chip.  Both are 2 modulo 6: with
+// the four rows of the halo a segment is a whole number of rounds, and starts
+// on an even row.
+constexpr int64_t kStreamWidth = 60, kStreamFill = 4096, kStreamBlocks = 4096;
+constexpr int kStreamRows = 20, kStreamShortRows = 8;
+constexpr int kStreamDepth = 3;   // rows in flight
+
+struct StreamGeom {
+    int32_t side, width, strips;
+    int32_t rows[2], segs[2];   // long and short segments
+};
+
+// Weights of one row of cells (the cell east of the lane's node; the nodes'
+// corner and vertical neighbours) and of one row of nodes.
+template <typename V> struct CellRow { V corner, across; };
+template <typename V> struct NodeRow { V east, diag; };
+
+// The interior row sum of the lane's node: nine terms in column order, below
+// (b), own and above (a) rows of x.  A term whose weight and operand both
+// belong to the node to the west is formed there and shifted.
+template <typename V>
+__device__ inline V stencil(const CellRow<V> &b, const NodeRow<V> &n, const CellRow<V> &a, V xb, V x, V xa) {
+    V s = V(0);
+    s = s + from_west(b.corner * xb);
+    s = s + b.across * xb;
+    s = s + b.corner * from_east(xb);
+    s = s + from_west(n.east * x);
+    s = s + n.diag * x;
+    s = s + n.east * from_east(x);
+    s = s + from_west(a.corner * xa);
+    s = s + a.across * xa;
+    s = s + a.corner * from_east(xa);
+    return s;
+}
+
+// k_b_pair's two passes, the same terms in the same order.  A wavefront owns
+// `rows` rows by `width` (<= 60) columns of one slot's grid and marches down
+// them, one row a step: row r arrives (its operand x formed), row r - 1's
+// first-pass value, then row r - 2's second-pass value follow from the last
+// three rows, which stay in registers; a node's neighbours to the west and
+// east are in the next lanes.  So there is no LDS and no barrier, every
+// wavefront runs on its own with D rows' loads in flight, and a weight is
+// formed once per cell, edge and node (four divisions a node; nine where
+// every node forms its row alone).  Bound by memory: 24 bytes a node, and the
+// halo's rows and columns through L2.  With weights from the cells, 51 systems
+// of 513^2 in FP32, PRE / POST: 89 / 80 us (3.6 / 4.1 TB/s) where the tiles of
+// k_b_pair take 117 / 118; BF16, 32 systems: 53 / 51, tiles 74 / 80; FP64, 32
+// systems: 80 / 87, tiles 97 / 119.  Longer segments (32 to 68 rows: 95 / 86)
+// leave the chip less evenly filled, shorter ones (8: 92 / 85) load more halo;
+// six rows in flight instead of three took 93 / 86 (fewer wavefronts).  When
+// the last few systems run, short segments take 7 us where long ones take 13.
+// WM: 1 weights from the cells, 3 the constant operator's.
+template <typename VT, int PAIR, int WM, bool FP, int D, typename V = typename VecOf<VT>::type>
+__global__ __launch_bounds__(256) void k_b_stream(BWork w, StreamGeom g, int64_t vld, const double *kappa, int64_t kld,
+                                                  V *out0, V *out1, const V *xin, const V *rhs, const V *dinv,
+                                                  const V *xc, int64_t vld_c) {
+    constexpr int U = 6;   // steps per round: a multiple of D, of the three rows kept and of the coarse rows' two
+    static_assert(U % D == 0, "ring");
+    const int lane = threadIdx.x % kWave;
+    const int64_t a0 = w.bounds[w.lo], na = w.bounds[w.hi] - a0;
+    const bool brief = na * g.strips * g.segs[0] < kStreamFill;
+    const int rows = brief ? g.rows[1] : g.rows[0];
+    const uint32_t per = (uint32_t)g.strips * (uint32_t)(brief ? g.segs[1] : g.segs[0]);
+    const int S = g.side;
+    const int64_t total = na * per;
+    // every XCD takes one contiguous eighth of the segments, whatever their number
+    const int64_t quads = (total + 3) / 4, share = quads / kXcds, more = quads % kXcds;
+    const int64_t xcd = blockIdx.x % kXcds, step = (gridDim.x - 1 - xcd) / kXcds + 1;
+    const int64_t lo = xcd * share + (xcd < more ? xcd : more), hi = lo + share + (xcd < more ? 1 : 0);
+    for (int64_t quad = lo + blockIdx.x / kXcds; quad < hi; quad += step) {
+        const int64_t q = quad * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+        if (q >= total) break;
+        const uint32_t e = (uint32_t)q / per, rem = (uint32_t)q - e * per;
+        const uint32_t seg = rem / (uint32_t)g.strips, strip = rem - seg * (uint32_t)g.strips;
+        const int64_t ls = w.list[a0 + e] - w.base;
+        const int r0 = (int)seg * rows, r1 = min(S, r0 + rows);
+        const int c0 = (int)strip * g.width, c1 = min(S, c0 + g.width);
+        const int col = c0 - 2 + lane;
+        const int rlast = __builtin_amdgcn_readfirstlane(min(S - 1, r1 + 1));   // the last row a load asks for
+        const bool mine = lane >= 2 && col < c1;
+        const uint32_t cn = (uint32_t)min(max(col, 0), S - 1);    // the lane's node
+        const uint32_t cc = (uint32_t)min(max(col, 0), S - 2);    // and cell column (positions outside: never used)
+        const bool side_border = cn == 0 || (int)cn == S - 1;
+        const V *rs = rhs + ls * vld, *ds = dinv + ls * vld, *xs = xin + ls * vld;
+        const double *ks = WM == 1 ? kappa + ls * kld : nullptr;
+        V *o0 = out0 + ls * vld, *o1 = out1 + ls * vld;
+        // FP: the coarse values left and right of the node's column
+        const V *cs = FP ? xc + ls * vld_c : nullptr;
+        const int SC = (S >> 1) + 1;
+        const uint32_t clo = cn >> 1, chi = (cn + 1) >> 1;
+        const uint32_t ct = min(clo, (uint32_t)(SC - 2));
+
+        V di_in = V(0), di_bnd = V(0);
+        if constexpr (WM == 3) {
+            di_in = dinv[S + 1];
+            di_bnd = dinv[0];
+        }
+        // rows in flight
+        V prh[D], pdi[D], pxn[D], pt0[D], pt1[D];
+        double pk[D];
+        auto load = [&](int r, int i, bool odd) {
+            const int rc = min(max(r, 0), rlast);
+            const int64_t at = (int64_t)rc * S;
+            prh[i] = (rs + at)[cn];
+            if constexpr (WM != 3) pdi[i] = (ds + at)[cn];
+            if constexpr (PAIR == PAIR_POST) pxn[i] = (xs + at)[cn];
+            if constexpr (WM == 1) {
+                const int kr = min(max(r - 1, 0), S - 2);   // the cells below the row
+                pk[i] = (ks + (int64_t)kr * (S - 1))[cc];
+            }
+            if constexpr (FP) {
+                if (odd) {   // the coarse row above an odd row
+                    const V *p = cs + (int64_t)min((rc + 1) >> 1, SC - 1) * SC;
+                    pt0[i] = p[ct];
+                    pt1[i] = (p + 1)[ct];
+                }
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < D; ++i) load(r0 - 2 + i, i, (i & 1) != 0);
+        V t0 = V(0), t1 = V(0);   // the coarse row at or below the current row
+        if constexpr (FP) {
+            const V *p = cs + (int64_t)max((r0 - 2) >> 1, 0) * SC;
+            t0 = p[ct];
+            t1 = (p + 1)[ct];
+        }
+        // the last three rows: x, first pass v, rhs, dinv; cells b (one row
+        // below), bb (two below) and their weights
+        V x1 = V(0), x2 = V(0), v2 = V(0), v3 = V(0), h1 = V(0), h2 = V(0), d1 = V(0), d2 = V(0);
+        double k1 = 0.0, across1 = 0.0;
+        CellRow<V> cconst{};
+        NodeRow<V> nconst{};
+        if constexpr (WM == 3) {
+            V wv[9];
+            q1_constant_weights<VT, V>(wv);
+            cconst.corner = wv[0];
+            cconst.across = wv[1];
+            nconst.east = wv[3];
+            nconst.diag = wv[4];
+        }
+        CellRow<V> c2 = cconst, c3 = cconst;
+        NodeRow<V> n2 = nconst;
+        auto put = [](double v) {
+            V a = (V)v;
+            if constexpr (sizeof(VT) == 2) a = bf16_round(a);
+            return a;
+        };
+        for (int base = r0 - 2; base < r1 + 2; base += U) {
+#pragma unroll
+            for (int j = 0; j < U; ++j) {
+                const int r = base + j, i = j % D;
+                const bool odd = (j & 1) != 0;
+                // ---- row r arrives ----
+                const V h0 = prh[i];
+                V d0;
+                if constexpr (WM == 3)
+                    d0 = (side_border || r <= 0 || r >= S - 1) ? di_bnd : di_in;
+                else
+                    d0 = pdi[i];
+                V x0;
+                if constexpr (PAIR == PAIR_PRE) {
+                    x0 = d0 * h0;
+                } else {
+                    x0 = pxn[i];
+                    if constexpr (FP) {   // + P xc, as k_b_prolong_rows forms it
+                        const V half = V(0.5), q4 = V(0.25);
+                        const V tl = clo == ct ? t0 : t1, tr = chi == ct ? t0 : t1;
+                        V f;
+                        if (odd) {
+                            const V u0 = pt0[i], u1 = pt1[i];
+                            const V ul = clo == ct ? u0 : u1, ur = chi == ct ? u0 : u1;
+                            const V f_rc = ((V(0) + tl * q4 + tr * q4) + ul * q4) + ur * q4;
+                            const V f_r = (V(0) + tl * half) + ul * half;
+                            f = (cn & 1) ? f_rc : f_r;
+                            t0 = u0;
+                            t1 = u1;
+                        } else {
+                            const V f_c = (V(0) + tl * half) + tr * half;
+                            f = (cn & 1) ? f_c : tl;
+                        }
+                        if (side_border || r <= 0 || r >= S - 1) f = V(0);
+                        x0 = x0 + f * V(1);
+                    }
+                }
+                // ---- the weights of cell row r - 1 and node row r - 1 ----
+                CellRow<V> c1 = cconst;
+                NodeRow<V> n1 = nconst;
+                if constexpr (WM == 1) {
+                    const double k0 = pk[i], kw = from_west(k0);
+                    const double pair0 = kw + k0;
+                    c1.corner = put(-div3_rn(k0));
+                    c1.across = put(-0.5 * div3_rn(pair0));
+                    n1.east = put(-0.5 * div3_rn(k1 + k0));
+                    n1.diag = put(div3_rn(2.0 * ((across1 + kw) + k0)));
+                    k1 = k0;
+                    across1 = pair0;
+                }
+                load(r + D, i, ((j + D) & 1) != 0);
+                // ---- row r - 1, first pass ----
+                V v1;
+                {
+                    const int a = r - 1;
+                    V sm = stencil(c2, n1, c1, x2, x1, x0);
+                    if (side_border || a <= 0 || a >= S - 1) sm = V(0) + V(1) * x1;
+                    v1 = x1 + (h1 - sm) * d1;
+                    if (PAIR == PAIR_PRE && mine && a >= r0 && a < r1) (o0 + (int64_t)a * S)[cn] = v1;
+                }
+                // ---- row r - 2, second pass ----
+                {
+                    const int b = r - 2;
+                    V sm = stencil(c3, n2, c2, v3, v2, v1);
+                    if (side_border || b <= 0 || b >= S - 1) sm = V(0) + V(1) * v2;
+                    const V t = h2 - sm;
+                    if (mine && b >= r0 && b < r1) {
+                        if constexpr (PAIR == PAIR_PRE)
+                            (o1 + (int64_t)b * S)[cn] = t;
+                        else
+                            (o0 + (int64_t)b * S)[cn] = v2 + t * d2;
+                    }
+                }
+                x2 = x1;
+                x1 = x0;
+                v3 = v2;
+                v2 = v1;
+                h2 = h1;
+                h1 = h0;
+                d2 = d1;
+                d1 = d0;
+                c3 = c2;
+                c2 = c1;
+                n2 = n1;
+            }
+        }
+    }
+}
+
+template <typename VT, int PAIR, int WM, bool FP>
+void stream_launch(dim3 grid, hipStream_t s, const BWork &w, const StreamGeom &g, const BLevel &lv, void *out0,
+                   void *out1, const void *xin, const void *xc, int64_t vld_c) {
+    using V = typename VecOf<VT>::type;
+    hipLaunchKernelGGL((k_b_stream<VT, PAIR, WM, FP, kStreamDepth>), grid, dim3(256), 0, s, w, g, lv.vld, lv.kappa, lv.kld,
+                       (V *)out0, (V *)out1, (const V *)xin, (const V *)lv.rhs, (const V *)lv.dinv, (const V *)xc,
+                       vld_c);
+}
+
+template <typename VT, int WM>
+void stream_pair(int pair, dim3 grid, hipStream_t s, const BWork &w, const StreamGeom &g, const BLevel &lv, void *out0,
+                 void *out1, const void *xin, const void *xc, int64_t vld_c) {
+    if (pair == PAIR_PRE)
+        stream_launch<VT, PAIR_PRE, WM, false>(grid, s, w, g, lv, out0, out1, lv.rhs, nullptr, 0);
+    else if (xc)
+        stream_launch<VT, PAIR_POST, WM, true>(grid, s, w, g, lv, out0, out0, xin, xc, vld_c);
+    else
+        stream_launch<VT, PAIR_POST, WM, false>(grid, s, w, g, lv, out0, out0, xin, nullptr, 0);
+}
+
+}  // namespace
+
+hipError_t b_pair_stream(ValueType vt, int pair, const BLevel &lv, const BWork &w, void *out0, void *out1,
+                         const void *xin, hipStream_t s, int wmode, const void *xc, int64_t vld_c) {
+    StreamGeom g;
+    g.side = (int32_t)lv.side;
+    g.strips = (int32_t)((lv.side + kStreamWidth - 1) / kStreamWidth);
+    g.width = (int32_t)((lv.side + g.strips - 1) / g.strips);
+    const int rows[2] = {kStreamRows, kStreamShortRows};
+    for (int k = 0; k < 2; ++k) {
+        g.rows[k] = rows[k];
+        g.segs[k] = (int32_t)((lv.side + rows[k] - 1) / rows[k]);
+    }
+    const int64_t units = lv.cap * (int64_t)g.strips * g.segs[1], blocks = (units + 3) / 4;
+    if (units < 1) return hipSuccess;
+    if (units > INT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)(blocks < kStreamBlocks ? blocks : kStreamBlocks));
+#define STREAM(VT)                                                                    \
+    do {                                                                              \
+        if (wmode == 3)                                                               \
+            stream_pair<VT, 3>(pair, grid, s, w, g, lv, out0, out1, xin, xc, vld_c);  \
+        else                                                                          \
+            stream_pair<VT, 1>(pair, grid, s, w, g, lv, out0, out1, xin, xc, vld_c);  \
+    } while (0)
+    if (vt == VT_F32)
+        STREAM(float);
+    else if (vt == VT_BF16)
+        STREAM(bf16);
+    else if (vt == VT_F64)
+        STREAM(double);
+    else
+        return hipErrorInvalidValue;
+#undef STREAM
+    return hipGetLastError();
+}
+
+}  // namespace hipx
+}  // namespace honei

@@ -1,0 +1,51 @@
+"""The paired row passes that march down column strips (large levels) against
+one launch per pass, in a batch pool: the same bits while all systems run and
+when the last few do.
+"""
+import numpy as np
+import pytest
+
+import honei_amd as H
+from tests.patterns import lognormal_cells, poisson_system_seeds, uniform_pm1
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    H.init(0)
+    yield
+
+
+# launches of many tiles on one level, on each level, and with all levels'
+# systems together; one system short of the rule on its finest level
+@pytest.mark.parametrize("levels,counts", [([7], [18]), ([7], [17]), ([8], [6]), ([9, 8, 7], [2, 4, 14])])
+@pytest.mark.parametrize("inner", [H.F32, H.BF16, H.F64])
+def test_pairs(inner, levels, counts):
+    got = []
+    for pair in (0, 1):
+        B = H.Batch(levels, counts, H.batch_config(autotune=0, inner_vtype=inner, pair_sweeps=pair, iters_per_launch=4,
+                                                   max_outer=40))
+        keep, slots = [], []
+        for c, lv in enumerate(levels):
+            for j in range(counts[c]):
+                cs, bs = poisson_system_seeds(400 + c, j)
+                side = 2 ** lv + 1
+                # systems that need more iterations than the others: the last to run
+                cells = lognormal_cells(cs, (side - 1) ** 2) ** (1.5 if j == 0 else 1.0)
+                keep.append((H.DeviceArray.from_host(cells, np.float64),
+                             H.DeviceArray.from_host(uniform_pm1(bs, side * side))))
+                slots.append(B.slot(c, j))
+        B.load_many(slots, [k for k, _ in keep], [b for _, b in keep])
+        B.run()
+        info = B.poll()
+        xs = []
+        for g, (_, b) in zip(slots, keep):
+            x = H.DeviceArray(b.n, np.float64)
+            B.result(g, x)
+            xs.append(((info[g].iters, info[g].status, info[g].rel), x.get()))
+        got.append(xs)
+    for (ia, xa), (ib, xb) in zip(*got):
+        assert ia == ib
+        assert np.array_equal(xa, xb)
+        assert np.isfinite(xa).all() and xa.any()
