@@ -625,14 +625,17 @@ def level_launch_rates(B, levels, level, reps=20):
     cap = sum(1 for L in levels if L >= level)
     # the pool's default weight source (matrix_free 1): 8 bytes per cell
     # instead of the stored values
-    rows = {"paired_pre": (pre, cap * (8 * cells + 16 * n),
-                           "k_b_pair<float,PRE,weights from cells>: Jacobi0 then the defect"),
+    # levels that pair fuse the restriction into the pre-smoothing launch (rst
+    # = 0 there): the coarse right-hand side is written instead of the defect
+    rows = {"paired_pre": (pre, cap * (8 * cells + (16 * n if rst > 0 else 12 * n + 4 * nc)),
+                           "paired launch, weights from cells: Jacobi0 then the defect%s"
+                           % ("" if rst > 0 else ", restricted")),
             "restriction": (rst, cap * (4 * n + 4 * nc), "k_b_restrict_rows"),
             "prolongation": (pro, cap * (8 * n + 4 * nc), "k_b_prolong_rows: t = x + P e"),
             # levels that pair fuse the prolongation into the post-smoothing
             # launch (pro = 0 there): the coarse result is read once more
             "paired_post": (post, cap * (8 * cells + 16 * n + (4 * nc if pro == 0 else 0)),
-                            "k_b_pair<float,POST,weights from cells%s>: two Jacobi sweeps"
+                            "paired launch, weights from cells: two Jacobi sweeps%s"
                             % (", prolongation fused" if pro == 0 else ""))}
     out = {"level": level, "side": side, "slots": cap}
     for key, (us, nb, what) in rows.items():

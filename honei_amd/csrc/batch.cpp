@@ -220,12 +220,19 @@ hipError_t BatchMG::tune_level(BLevel &lv) {
             if (err == hipSuccess) err = vfill(tl.kappa, 1.0, ns * tl.kld, VT_F64, s_main_);
             if (err == hipSuccess) err = hipMalloc(&tl.st, (size_t)(ns * 4 * g.vld) * vs);
             if (err == hipSuccess) err = b_stencil_fill(vt, g.side, tl.kappa, tl.kld, tl.st, g.vld, ns, s_main_);
+            BLevel tc;   // the level below, its right-hand side in the output's buffer
+            tc.side = (g.side - 1) / 2 + 1;
+            tc.n = tc.side * tc.side;
+            tc.cap = ns;
+            tc.vld = g.vld;
+            tc.rhs = out;
             // every weight source: the stored values (0), the cell
             // coefficients (1), the distinct-weight arrays (2)
             for (int mf = 0; mf < 3; ++mf) {
                 for (int pass = 0; pass < 2 && err == hipSuccess; ++pass) {
                     auto launch = [&]() {
-                        return pass == 0 ? b_pair(vt, PAIR_PRE, tl, w, tl.x, out, nullptr, s_main_, mf)
+                        return pass == 0 ? (mf == 1 ? b_pre_restrict(vt, tl, tc, w, s_main_, mf)
+                                                    : b_pair(vt, PAIR_PRE, tl, w, tl.x, out, nullptr, s_main_, mf))
                                          : b_pair(vt, PAIR_POST, tl, w, out, nullptr, tl.x, s_main_, mf);
                     };
                     const int reps = n >= 65536 ? 10 : 30;
@@ -435,9 +442,8 @@ hipError_t BatchMG::enqueue_vcycle(hipStream_t s) {
         const BMat m = mat(lv);
         const BWork w = level_work(l);
         if (paired(lv) && cfg_.n_pre == 2) {
-            // x = Jacobi0, d = rhs - A x: one launch
-            HX(b_pair(vt, PAIR_PRE, lv, w, lv.x, lv.d, nullptr, s, pair_weights(lv)));
-            HX(b_restrict(vt, lv, L_[(size_t)l - 1], w, s));
+            // x = Jacobi0, rhs of the next level = R (rhs - A x)
+            HX(b_pre_restrict(vt, lv, L_[(size_t)l - 1], w, s, pair_weights(lv)));
             continue;
         }
         // x = n_pre Jacobi sweeps from zero (first two fused), ending in x
@@ -823,8 +829,12 @@ hipError_t BatchMG::time_level(int64_t level, int reps, double us[5]) {
     };
     const bool mf = cfg_.matrix_free != 0;
     const int wm = pair_weights(lv);
-    if (paired(lv)) timeit([&]() { return b_pair(vt, PAIR_PRE, lv, w, lv.x, lv.d, nullptr, s_main_, wm); }, &us[0]);
-    timeit([&]() { return b_restrict(vt, lv, lc, w, s_main_); }, &us[1]);
+    const bool one_pre = paired(lv) && wm == 1;   // the restriction in the paired launch
+    if (one_pre)
+        timeit([&]() { return b_pre_restrict(vt, lv, lc, w, s_main_, wm); }, &us[0]);
+    else if (paired(lv))
+        timeit([&]() { return b_pair(vt, PAIR_PRE, lv, w, lv.x, lv.d, nullptr, s_main_, wm); }, &us[0]);
+    if (!one_pre) timeit([&]() { return b_restrict(vt, lv, lc, w, s_main_); }, &us[1]);
     if (fused_post(lv))
         timeit([&]() { return b_pair(vt, PAIR_POST, lv, w, lv.t, nullptr, lv.x, s_main_, wm, &lc, lc.x); }, &us[3]);
     else

@@ -464,10 +464,16 @@ hipError_t b_prolong_axpy(ValueType vt, const BLevel &fine, const BLevel &coarse
 hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void *out0, void *out1,
                   const void *xin, hipStream_t s, int wmode = 0, const BLevel *coarse = nullptr,
                   const void *xc = nullptr);
-// The same passes, one wavefront marching down a column strip (k_b_stream):
-// b_pair's launch for large levels, after its checks (wmode 1 or 3).
-hipError_t b_pair_stream(ValueType vt, int pair, const BLevel &lv, const BWork &w, void *out0, void *out1,
-                         const void *xin, hipStream_t s, int wmode, const void *xc, int64_t vld_c);
+// Weights from the cells or the constant operator (wmode 1, 3): the passes by
+// one wavefront marching down a column strip (k_b_stream).  PAIR_POST for
+// b_pair (xin, xc as there), PAIR_PRE for b_pre_restrict (xc = the coarse
+// right-hand side), after their checks.
+hipError_t b_pair_stream(ValueType vt, int pair, const BLevel &lv, const BWork &w, void *out0, const void *xin,
+                         hipStream_t s, int wmode, void *xc, int64_t vld_c);
+// fine.x = Jacobi0, coarse.rhs = R (rhs - A x): one launch with wmode 1 or 3,
+// else PAIR_PRE (the defect in fine.d) and the restriction.
+hipError_t b_pre_restrict(ValueType vt, const BLevel &fine, const BLevel &coarse, const BWork &w, hipStream_t s,
+                          int wmode);
 // The distinct-weight arrays of `count` slots of a side x side level from
 // their cell coefficients (kappa + g kld, st + g 4 vld).
 hipError_t b_stencil_fill(ValueType vt, int64_t side, const double *kappa, int64_t kld, void *st, int64_t vld,

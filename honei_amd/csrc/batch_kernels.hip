@@ -375,10 +375,7 @@ __global__ __launch_bounds__(kPairTileRows * kWave, 8) void k_b_pair(BMat m, BWo
         // the extra entry's loads only where there is one (the first waves)
         V e1 = V(0), e2 = V(0);
         if (threadIdx.x < kExtra) {
-            if constexpr (PAIR == PAIR_PRE && WM == 3)
-                e1 = on_border(egr, egc) ? di_bnd : di_in;
-            else
-                e1 = (PAIR == PAIR_PRE) ? ds[ej] : xs[ej];
+            e1 = (PAIR == PAIR_PRE) ? ds[ej] : xs[ej];
             if (PAIR == PAIR_PRE) e2 = rs[ej];
             if constexpr (FP) prolong_taps(xc + ls * vld_c, (S >> 1) + 1, egr, egc, te);
         }
@@ -1465,7 +1462,7 @@ hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void
                lv.side > kMaxTransferSide || xc == out0))
         return hipErrorInvalidValue;
     const int64_t vld_c = fp ? coarse->vld : 0;
-    if (wmode < 0 || wmode > 3) return hipErrorInvalidValue;
+    if (wmode < 0 || wmode > 3 || (pair == PAIR_PRE && (wmode == 1 || wmode == 3))) return hipErrorInvalidValue;
     if (wmode == 1 && (!lv.kappa || lv.kld < (lv.side - 1) * (lv.side - 1))) return hipErrorInvalidValue;
     if (wmode == 2 && !lv.st) return hipErrorInvalidValue;
     if (wmode == 0 && (!lv.Ax || !lv.Aj)) return hipErrorInvalidValue;
@@ -1475,16 +1472,16 @@ hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void
     pg.width = (int32_t)((lv.side + pg.strips - 1) / pg.strips);
     // launches of at least kMinTallTiles tall tiles: with weights that come
     // from the cells or the constant operator, the column march (by total
-    // nodes, 129^2 systems, FP32, PRE / POST, tile against march in us: 0.27 M
-    // 6.7 / 6.7 and 7.2 / 6.6, 0.53 M 10.8 / 9.1 and 8.5 / 8.4; FP64, 1.07 M
-    // 17.2 / 20.9 and 15.2 / 16.6); with stored weights two grid rows per
+    // nodes, 129^2 systems, POST, tile against march in us: FP32 0.27 M 6.7 /
+    // 6.6, 0.53 M 9.1 / 8.4; FP64 1.07 M 20.9 / 16.6; below, the tiles'
+    // shorter chain: 0.13 M 4.5 / 6.6); with stored weights two grid rows per
     // thread (taller tiles: half the halo rows per node, twice the loads in
     // flight per thread)
     const int64_t tall_rows = 2 * kPairTileRows - 2;
     const bool tall = lv.side >= kPairTallMinSide &&
                       lv.cap * pg.strips * ((lv.side + tall_rows - 1) / tall_rows) >= kMinTallTiles;
     if (tall && (wmode == 1 || wmode == 3))
-        return b_pair_stream(vt, pair, lv, w, out0, out1, xin, s, wmode, xc, vld_c);
+        return b_pair_stream(vt, pair, lv, w, out0, xin, s, wmode, const_cast<void *>(xc), vld_c);
     const int nr = tall && vt != VT_F64 ? 2 : 1;
     const int64_t rows = (int64_t)kPairTileRows * nr - 2;
     pg.segs = (int32_t)((lv.side + rows - 1) / rows);
@@ -1499,12 +1496,8 @@ hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void
     pair_launch<VT, P, MFV>(grid, block, s, m, w, pg, out0, out1, x, lv.rhs, lv.dinv, xc, vld_c, nr)
 #define PAIR_WM(VT, P)                                                        \
     do {                                                                      \
-        if (wmode == 3)                                                       \
-            PAIR_LAUNCH(VT, P, 3);                                            \
-        else if (wmode == 2)                                                  \
+        if (wmode == 2)                                                       \
             PAIR_LAUNCH(VT, P, 2);                                            \
-        else if (wmode == 1)                                                  \
-            PAIR_LAUNCH(VT, P, 1);                                            \
         else                                                                  \
             PAIR_LAUNCH(VT, P, 0);                                            \
     } while (0)
@@ -1512,6 +1505,10 @@ hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void
     do {                                                                      \
         if (pair == PAIR_PRE)                                                 \
             PAIR_WM(VT, PAIR_PRE);                                            \
+        else if (wmode == 3)                                                  \
+            PAIR_LAUNCH(VT, PAIR_POST, 3);                                    \
+        else if (wmode == 1)                                                  \
+            PAIR_LAUNCH(VT, PAIR_POST, 1);                                    \
         else                                                                  \
             PAIR_WM(VT, PAIR_POST);                                           \
     } while (0)
@@ -1527,6 +1524,18 @@ hipError_t b_pair(ValueType vt, int pair, const BLevel &lv, const BWork &w, void
 #undef PAIR_WM
 #undef PAIR_LAUNCH
     return hipGetLastError();
+}
+
+hipError_t b_pre_restrict(ValueType vt, const BLevel &fine, const BLevel &coarse, const BWork &w, hipStream_t s,
+                          int wmode) {
+    if (wmode != 1 && wmode != 3) {
+        const hipError_t e = b_pair(vt, PAIR_PRE, fine, w, fine.x, fine.d, nullptr, s, wmode);
+        return e != hipSuccess ? e : b_restrict(vt, fine, coarse, w, s);
+    }
+    if (fine.side != 2 * (coarse.side - 1) + 1 || fine.cap > coarse.cap || fine.side > kMaxTransferSide ||
+        fine.T != 1 || fine.side < 5 || !fine.x || !coarse.rhs || (wmode == 1 && (!fine.kappa || fine.kld < (fine.side - 1) * (fine.side - 1))))
+        return hipErrorInvalidValue;
+    return b_pair_stream(vt, PAIR_PRE, fine, w, fine.x, nullptr, s, wmode, coarse.rhs, coarse.vld);
 }
 
 hipError_t b_copy(ValueType vt, const BLevel &lv, const BWork &w, void *dst, const void *src, hipStream_t s) {

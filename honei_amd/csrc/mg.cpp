@@ -249,8 +249,7 @@ hipError_t MGHierarchy::q1_vcycle(int64_t top, const OneSlot *work, hipStream_t 
     for (int64_t l = top; l > lf; --l) {
         MGLevel &lv = L[(size_t)l];
         const BLevel f = one_slot(lv, l);
-        HX(b_pair(inner, PAIR_PRE, f, w, lv.x, lv.d, nullptr, s, weights(lv)));
-        HX(b_restrict(inner, f, one_slot(L[(size_t)l - 1], l - 1), w, s));
+        HX(b_pre_restrict(inner, f, one_slot(L[(size_t)l - 1], l - 1), w, s, weights(lv)));
     }
     CoarseCycle cc{};
     cc.top = (int)lf;

@@ -22,18 +22,19 @@ template <typename T> __device__ inline T from_west(T v) { return lane_shift<0x1
 template <typename T> __device__ inline T from_east(T v) { return lane_shift<0x130>(v); }
 
 // A strip is at most kStreamWidth columns (two halo columns each side fill a
-// wavefront), a segment kStreamRows rows; kStreamShortRows where the running
-// systems give fewer than kStreamFill long segments (four wavefronts a SIMD),
-// so that few systems still spread over the chip.  Both are 2 modulo 6: with
-// the four rows of the halo a segment is a whole number of rounds, and starts
-// on an even row.
+// wavefront; the restriction takes one more to the west and ends on an even
+// one: two columns fewer).  Segments are long, medium or short: the longest
+// of which the running systems give kStreamFill (four wavefronts a SIMD), so
+// that a few systems still spread over the chip.  With the rows of the halo
+// (four, six with the restriction) a segment is a whole number of rounds of
+// six steps, and it starts on an even row.
 constexpr int64_t kStreamWidth = 60, kStreamFill = 4096, kStreamBlocks = 4096;
-constexpr int kStreamRows = 20, kStreamShortRows = 8;
 constexpr int kStreamDepth = 3;   // rows in flight
 
 struct StreamGeom {
     int32_t side, width, strips;
-    int32_t rows[2], segs[2];   // long and short segments
+    int32_t rows[3], segs[3];   // long, medium and short segments
+    int64_t from[2];            // running systems from which the long, the medium ones are taken
 };
 
 // Weights of one row of cells (the cell east of the lane's node; the nodes'
@@ -59,6 +60,32 @@ __device__ inline V stencil(const CellRow<V> &b, const NodeRow<V> &n, const Cell
     return s;
 }
 
+// k_b_restrict_rows' value of the lane's coarse node (its fine node in this
+// lane's column and the middle row), d = coarse column - row, from the defect
+// rows below (b), through (m) and above (a) it: the same terms in the same
+// order.
+template <typename V>
+__device__ inline V restrict_value(int d, V b, V m, V a) {
+    const V h = V(0.5), q = V(0.25);
+    const V C = h * from_east(m), D = h * from_west(m);
+    V s = m;
+    s = d <= -1 ? s + D : s;
+    s = d <= -2 ? s + C : s;
+    s = s + h * b;
+    s = d == -1 ? s + C : s;
+    s = d == 0 ? s + D : s;
+    s = s + q * from_east(b);
+    s = s + q * from_west(b);
+    s = s + h * a;
+    s = d == 0 ? s + C : s;
+    s = d == 1 ? s + D : s;
+    s = s + q * from_east(a);
+    s = s + q * from_west(a);
+    s = d >= 2 ? s + D : s;
+    s = d >= 1 ? s + C : s;
+    return s;
+}
+
 // k_b_pair's two passes, the same terms in the same order.  A wavefront owns
 // `rows` rows by `width` (<= 60) columns of one slot's grid and marches down
 // them, one row a step: row r arrives (its operand x formed), row r - 1's
@@ -67,26 +94,40 @@ __device__ inline V stencil(const CellRow<V> &b, const NodeRow<V> &n, const Cell
 // east are in the next lanes.  So there is no LDS and no barrier, every
 // wavefront runs on its own with D rows' loads in flight, and a weight is
 // formed once per cell, edge and node (four divisions a node; nine where
-// every node forms its row alone).  Bound by memory: 24 bytes a node, and the
-// halo's rows and columns through L2.  With weights from the cells, 51 systems
-// of 513^2 in FP32, PRE / POST: 89 / 80 us (3.6 / 4.1 TB/s) where the tiles of
-// k_b_pair take 117 / 118; BF16, 32 systems: 53 / 51, tiles 74 / 80; FP64, 32
-// systems: 80 / 87, tiles 97 / 119.  Longer segments (32 to 68 rows: 95 / 86)
-// leave the chip less evenly filled, shorter ones (8: 92 / 85) load more halo;
-// six rows in flight instead of three took 93 / 86 (fewer wavefronts).  When
-// the last few systems run, short segments take 7 us where long ones take 13.
+// every node forms its row alone).
+// PAIR_PRE writes no defect: when the three defect rows around a coarse row
+// are there, its restriction goes out instead (k_b_restrict_rows' terms and
+// order).  Only the coarse right-hand side ever reads the defect, so a write
+// and a read of it and a launch are saved.  FUSED (PAIR_POST only): with the
+// prolongation.
+// Bound by memory: 21 (PRE) and 25 bytes a node with weights from the cells,
+// and the halo's rows and columns through L2.  51 systems of 513^2 in FP32,
+// PRE with the restriction / POST with the prolongation: 89 / 80 us (3.2 /
+// 4.2 TB/s) where the tiles of k_b_pair take 117 and 20 for the restriction /
+// 118; all levels of 256 systems 159 / 143, tiles 212 and 43 / 223.  One
+// system of 1025^2, 513^2, 257^2, 129^2 with the constant operator, PRE: 9.1,
+// 5.6, 5.0, 5.5, tiles and restriction 13.8, 9.6, 8.7, 7.9.  Longer segments
+// (32 to 68 rows: POST 86) leave the chip less evenly filled, shorter ones
+// (8: 85) load more halo; six rows in flight instead of three took 86 (fewer
+// wavefronts).  When the last few systems run, short segments take 7 us where
+// long ones take 13.
 // WM: 1 weights from the cells, 3 the constant operator's.
-template <typename VT, int PAIR, int WM, bool FP, int D, typename V = typename VecOf<VT>::type>
+template <typename VT, int PAIR, int WM, bool FUSED, int D, typename V = typename VecOf<VT>::type>
 __global__ __launch_bounds__(256) void k_b_stream(BWork w, StreamGeom g, int64_t vld, const double *kappa, int64_t kld,
-                                                  V *out0, V *out1, const V *xin, const V *rhs, const V *dinv,
-                                                  const V *xc, int64_t vld_c) {
+                                                  V *out0, const V *xin, const V *rhs, const V *dinv,
+                                                  V *xc, int64_t vld_c) {
+    constexpr bool RS = PAIR == PAIR_PRE, FP = PAIR == PAIR_POST && FUSED;
+    static_assert(!RS || !FUSED, "the prolongation fuses into the post-smoothing pair");
+    constexpr int LEAD = RS ? 4 : 2;    // steps before a segment's first row (an even number)
+    constexpr int SIDE = RS ? 3 : 2;    // halo columns to the west
     constexpr int U = 6;   // steps per round: a multiple of D, of the three rows kept and of the coarse rows' two
     static_assert(U % D == 0, "ring");
+    static_assert(LEAD % 2 == 0, "row parity");
     const int lane = threadIdx.x % kWave;
     const int64_t a0 = w.bounds[w.lo], na = w.bounds[w.hi] - a0;
-    const bool brief = na * g.strips * g.segs[0] < kStreamFill;
-    const int rows = brief ? g.rows[1] : g.rows[0];
-    const uint32_t per = (uint32_t)g.strips * (uint32_t)(brief ? g.segs[1] : g.segs[0]);
+    const int pick = na >= g.from[0] ? 0 : (na >= g.from[1] ? 1 : 2);
+    const int rows = g.rows[pick];
+    const uint32_t per = (uint32_t)g.strips * (uint32_t)g.segs[pick];
     const int S = g.side;
     const int64_t total = na * per;
     // every XCD takes one contiguous eighth of the segments, whatever their number
@@ -101,15 +142,15 @@ __global__ __launch_bounds__(256) void k_b_stream(BWork w, StreamGeom g, int64_t
         const int64_t ls = w.list[a0 + e] - w.base;
         const int r0 = (int)seg * rows, r1 = min(S, r0 + rows);
         const int c0 = (int)strip * g.width, c1 = min(S, c0 + g.width);
-        const int col = c0 - 2 + lane;
+        const int col = c0 - SIDE + lane;
         const int rlast = __builtin_amdgcn_readfirstlane(min(S - 1, r1 + 1));   // the last row a load asks for
-        const bool mine = lane >= 2 && col < c1;
+        const bool mine = lane >= SIDE && col < c1;
         const uint32_t cn = (uint32_t)min(max(col, 0), S - 1);    // the lane's node
         const uint32_t cc = (uint32_t)min(max(col, 0), S - 2);    // and cell column (positions outside: never used)
         const bool side_border = cn == 0 || (int)cn == S - 1;
         const V *rs = rhs + ls * vld, *ds = dinv + ls * vld, *xs = xin + ls * vld;
         const double *ks = WM == 1 ? kappa + ls * kld : nullptr;
-        V *o0 = out0 + ls * vld, *o1 = out1 + ls * vld;
+        V *o0 = out0 + ls * vld;
         // FP: the coarse values left and right of the node's column
         const V *cs = FP ? xc + ls * vld_c : nullptr;
         const int SC = (S >> 1) + 1;
@@ -143,7 +184,12 @@ __global__ __launch_bounds__(256) void k_b_stream(BWork w, StreamGeom g, int64_t
             }
         };
 #pragma unroll
-        for (int i = 0; i < D; ++i) load(r0 - 2 + i, i, (i & 1) != 0);
+        for (int i = 0; i < D; ++i) load(r0 - LEAD + i, i, (i & 1) != 0);
+        // RS: the last coarse row, on the border, follows one step past the grid
+        const int rend = RS && r1 == S ? S + 3 : r1 + 2;
+        const int rcoarse = rend - 3;   // the last defect row that completes a coarse row
+        V *cr = RS ? xc + ls * vld_c : nullptr;
+        V e1 = V(0), e2 = V(0);   // defect rows r - 3, r - 4
         V t0 = V(0), t1 = V(0);   // the coarse row at or below the current row
         if constexpr (FP) {
             const V *p = cs + (int64_t)max((r0 - 2) >> 1, 0) * SC;
@@ -171,7 +217,7 @@ __global__ __launch_bounds__(256) void k_b_stream(BWork w, StreamGeom g, int64_t
             if constexpr (sizeof(VT) == 2) a = bf16_round(a);
             return a;
         };
-        for (int base = r0 - 2; base < r1 + 2; base += U) {
+        for (int base = r0 - LEAD; base < rend; base += U) {
 #pragma unroll
             for (int j = 0; j < U; ++j) {
                 const int r = base + j, i = j % D;
@@ -237,11 +283,18 @@ __global__ __launch_bounds__(256) void k_b_stream(BWork w, StreamGeom g, int64_t
                     V sm = stencil(c3, n2, c2, v3, v2, v1);
                     if (side_border || b <= 0 || b >= S - 1) sm = V(0) + V(1) * v2;
                     const V t = h2 - sm;
-                    if (mine && b >= r0 && b < r1) {
-                        if constexpr (PAIR == PAIR_PRE)
-                            (o1 + (int64_t)b * S)[cn] = t;
-                        else
-                            (o0 + (int64_t)b * S)[cn] = v2 + t * d2;
+                    if constexpr (RS) {
+                        if (odd) {   // rows b - 2 .. b around coarse row (b - 1) / 2
+                            const int I = (b - 1) / 2;
+                            const V f = restrict_value((int)(cn >> 1) - I, e2, e1, t);
+                            if (mine && !(cn & 1) && b > r0 && b <= rcoarse)
+                                (cr + (int64_t)I * SC)[cn >> 1] =
+                                    (side_border || I == 0 || I == SC - 1) ? V(0) : f;
+                        }
+                        e2 = e1;
+                        e1 = t;
+                    } else if (mine && b >= r0 && b < r1) {
+                        (o0 + (int64_t)b * S)[cn] = v2 + t * d2;
                     }
                 }
                 x2 = x1;
@@ -260,49 +313,53 @@ __global__ __launch_bounds__(256) void k_b_stream(BWork w, StreamGeom g, int64_t
     }
 }
 
-template <typename VT, int PAIR, int WM, bool FP>
+template <typename VT, int PAIR, int WM, bool FUSED>
 void stream_launch(dim3 grid, hipStream_t s, const BWork &w, const StreamGeom &g, const BLevel &lv, void *out0,
-                   void *out1, const void *xin, const void *xc, int64_t vld_c) {
+                   const void *xin, void *xc, int64_t vld_c) {
     using V = typename VecOf<VT>::type;
-    hipLaunchKernelGGL((k_b_stream<VT, PAIR, WM, FP, kStreamDepth>), grid, dim3(256), 0, s, w, g, lv.vld, lv.kappa, lv.kld,
-                       (V *)out0, (V *)out1, (const V *)xin, (const V *)lv.rhs, (const V *)lv.dinv, (const V *)xc,
-                       vld_c);
+    hipLaunchKernelGGL((k_b_stream<VT, PAIR, WM, FUSED, kStreamDepth>), grid, dim3(256), 0, s, w, g, lv.vld, lv.kappa,
+                       lv.kld, (V *)out0, (const V *)xin, (const V *)lv.rhs, (const V *)lv.dinv, (V *)xc, vld_c);
 }
 
 template <typename VT, int WM>
 void stream_pair(int pair, dim3 grid, hipStream_t s, const BWork &w, const StreamGeom &g, const BLevel &lv, void *out0,
-                 void *out1, const void *xin, const void *xc, int64_t vld_c) {
+                 const void *xin, void *xc, int64_t vld_c) {
     if (pair == PAIR_PRE)
-        stream_launch<VT, PAIR_PRE, WM, false>(grid, s, w, g, lv, out0, out1, lv.rhs, nullptr, 0);
+        stream_launch<VT, PAIR_PRE, WM, false>(grid, s, w, g, lv, out0, lv.rhs, xc, vld_c);
     else if (xc)
-        stream_launch<VT, PAIR_POST, WM, true>(grid, s, w, g, lv, out0, out0, xin, xc, vld_c);
+        stream_launch<VT, PAIR_POST, WM, true>(grid, s, w, g, lv, out0, xin, xc, vld_c);
     else
-        stream_launch<VT, PAIR_POST, WM, false>(grid, s, w, g, lv, out0, out0, xin, nullptr, 0);
+        stream_launch<VT, PAIR_POST, WM, false>(grid, s, w, g, lv, out0, xin, nullptr, 0);
 }
 
 }  // namespace
 
-hipError_t b_pair_stream(ValueType vt, int pair, const BLevel &lv, const BWork &w, void *out0, void *out1,
-                         const void *xin, hipStream_t s, int wmode, const void *xc, int64_t vld_c) {
+hipError_t b_pair_stream(ValueType vt, int pair, const BLevel &lv, const BWork &w, void *out0, const void *xin,
+                         hipStream_t s, int wmode, void *xc, int64_t vld_c) {
+    const bool rs = pair == PAIR_PRE;
     StreamGeom g;
     g.side = (int32_t)lv.side;
-    g.strips = (int32_t)((lv.side + kStreamWidth - 1) / kStreamWidth);
+    const int64_t most = rs ? kStreamWidth - 2 : kStreamWidth;
+    g.strips = (int32_t)((lv.side + most - 1) / most);
     g.width = (int32_t)((lv.side + g.strips - 1) / g.strips);
-    const int rows[2] = {kStreamRows, kStreamShortRows};
-    for (int k = 0; k < 2; ++k) {
+    if (rs) g.width += g.width & 1;
+    const int rows[3] = {rs ? 24 : 20, rs ? 12 : 14, rs ? 6 : 8};
+    for (int k = 0; k < 3; ++k) {
         g.rows[k] = rows[k];
         g.segs[k] = (int32_t)((lv.side + rows[k] - 1) / rows[k]);
+        const int64_t per = (int64_t)g.strips * g.segs[k];
+        if (k < 2) g.from[k] = (kStreamFill + per - 1) / per;
     }
-    const int64_t units = lv.cap * (int64_t)g.strips * g.segs[1], blocks = (units + 3) / 4;
+    const int64_t units = lv.cap * (int64_t)g.strips * g.segs[2], blocks = (units + 3) / 4;
     if (units < 1) return hipSuccess;
     if (units > INT32_MAX) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)(blocks < kStreamBlocks ? blocks : kStreamBlocks));
 #define STREAM(VT)                                                                    \
     do {                                                                              \
         if (wmode == 3)                                                               \
-            stream_pair<VT, 3>(pair, grid, s, w, g, lv, out0, out1, xin, xc, vld_c);  \
+            stream_pair<VT, 3>(pair, grid, s, w, g, lv, out0, xin, xc, vld_c);  \
         else                                                                          \
-            stream_pair<VT, 1>(pair, grid, s, w, g, lv, out0, out1, xin, xc, vld_c);  \
+            stream_pair<VT, 1>(pair, grid, s, w, g, lv, out0, xin, xc, vld_c);  \
     } while (0)
     if (vt == VT_F32)
         STREAM(float);

@@ -532,14 +532,16 @@ int honei_hip_batch_shape(void *batch, int32_t level, int32_t *threads, int32_t 
                           double *sweep_us, int64_t *tune_slots);
 /* Levels that run the paired launches (pair_sweeps, levels of 33^2 nodes and
  * up): the autotuner's measured time of one paired Jacobi0 + defect launch
- * and of one paired two-sweep launch over the same tuning batch
- * (microseconds; 0 when the level is not paired or not tuned).            */
+ * (matrix_free 1: with the restriction in it) and of one paired two-sweep
+ * launch over the same tuning batch (microseconds; 0 when the level is not
+ * paired or not tuned).                                                    */
 int honei_hip_batch_pair_timing(void *batch, int32_t level, double *pre_us, double *post_us);
 /* Measurement (no reference counterpart): one level's launches timed over
  * every slot present on that level -- the launch shape of a batched step at
  * full activity -- with HIP events on the pool's stream, `reps` launches
  * after one warm-up: us[0] paired Jacobi0 + defect, us[1] restriction to
- * level - 1, us[2] prolongation + correction from level - 1, us[3] paired
+ * level - 1 (where the level pairs with matrix_free 1 it runs inside us[0]'s
+ * launch and us[1] is 0), us[2] prolongation + correction from level - 1, us[3] paired
  * two-sweep launch (0 where the level does not pair; where it pairs, the
  * prolongation + correction runs inside it and us[2] is 0), us[4] the FP64
  * p = z + beta p with q = A p, p.q (one tiled launch) over every slot of

@@ -18,8 +18,10 @@ def _init():
 
 
 # launches of many tiles on one level, on each level, and with all levels'
-# systems together; one system short of the rule on its finest level
-@pytest.mark.parametrize("levels,counts", [([7], [18]), ([7], [17]), ([8], [6]), ([9, 8, 7], [2, 4, 14])])
+# systems together; one system short of the rule on its finest level; enough
+# systems for medium and for long segments (shorter ones as systems finish)
+@pytest.mark.parametrize("levels,counts", [([7], [18]), ([7], [17]), ([8], [6]), ([9, 8, 7], [2, 4, 14]),
+                                           ([7], [130]), ([7], [230])])
 @pytest.mark.parametrize("inner", [H.F32, H.BF16, H.F64])
 def test_pairs(inner, levels, counts):
     got = []
@@ -29,6 +31,10 @@ def test_pairs(inner, levels, counts):
         keep, slots = [], []
         for c, lv in enumerate(levels):
             for j in range(counts[c]):
+                if j >= 20:   # the earlier systems again
+                    keep.append(keep[-20])
+                    slots.append(B.slot(c, j))
+                    continue
                 cs, bs = poisson_system_seeds(400 + c, j)
                 side = 2 ** lv + 1
                 # systems that need more iterations than the others: the last to run
