@@ -281,6 +281,159 @@ __global__ __launch_bounds__(1024) void k_product_staged(const int32_t *__restri
     }
 }
 
+// ---- wide float rows, one lane per row ------------------------------------------
+// y = A x for rows of 17 to 28 entries of 4 bytes.  Where neighbouring rows'
+// columns are scattered, ell_row_kernel is bound by its gathers: each takes a
+// cache line of its own from L2, and four of them at a time wait for the
+// indices before them.  Here a work-group looks at the first entries of its
+// rows.  Scattered: the whole row's indices go to registers, the column window
+// of the work-group follows from them, x is copied into LDS once (coalesced)
+// and gathered from there; a window too wide for it is gathered from global
+// memory.  Not scattered: rows in steps of eight entries, the next step's
+// indices loaded ahead.  Entries past a row's end are asked for outside the
+// buffer (no memory access), so no load sits behind a branch.  The sum is
+// ell_lane_sum's, term for term.
+// Rows of 1 .. 27 entries within +-4096 columns: 10^6 rows 90 -> 50 us (216 MB
+// of padded streams, 4.3 TB/s), 120,000 12.1 -> 9.8.  27-point stencil of
+// 100^3: 37.5 -> 35.6; 25 points of 1000^2: 33.7 -> 34.0.
+// Doubles stay with ell_row_kernel: the window and the row leave four
+// wavefronts a SIMD, which took 121 -> 69 us on scattered rows but 62 -> 68 on
+// the 27-point stencil; so do rows of more than 28 entries (regular ones 14.0
+// -> 15.2 at 300,000 rows), of 16 and fewer (nothing gained where regular),
+// and fewer rows than kRowsMin (65,537: 4.6 -> 6.3, too few work-groups).
+constexpr int kRowsBlock = 512;
+constexpr int kRowsWindow = 9216;   // entries of x: 36 KiB, four work-groups a CU
+constexpr int64_t kRowsMin = 98304;
+
+template <int NC>
+__global__ __launch_bounds__(kRowsBlock, 6) void k_product_rows(KArgs a) {
+    constexpr int P = 8, U = 8;   // entries looked at first; entries a step
+    constexpr uint32_t kOutside = 0x80000000u;
+    __shared__ float win[kRowsWindow];
+    __shared__ int32_t red[4][kRowsBlock / kWave];
+    const float *__restrict__ x = (const float *)a.x;
+    const int64_t row = a.row_start + xcd_block(blockIdx.x, gridDim.x) * kRowsBlock + threadIdx.x;
+    const uint32_t len = row < a.row_end ? a.Arl[row] : 0u;
+    const auto rAj = buffer_rsrc(a.Aj, a.aj_bytes), rAx = buffer_rsrc(a.Ax, a.ax_bytes);
+    const uint32_t oj = (uint32_t)row * 4u, stride = (uint32_t)a.stride;
+    int32_t j[NC];
+    auto index = [&](int k) {
+        j[k] = BufLoad<int32_t>::template load<kBufNT>(rAj, (uint32_t)k < len ? oj : kOutside, (uint32_t)k * stride * 4u);
+    };
+    auto value = [&](int k) {
+        return BufLoad<float>::template load<kBufNT>(rAx, (uint32_t)k < len ? oj : kOutside,
+                                                  (uint32_t)k * stride * 4u);
+    };
+#pragma unroll
+    for (int k = 0; k < P; ++k) index(k);
+    // scattered: most entries of neighbouring rows (four of a row looked at)
+    // lie further apart than a cache line of 32 entries
+    const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
+    const uint32_t wlen = lane ? (uint32_t)__shfl_up((int)len, 1) : 0u;
+    int far = 0, pairs = 0;
+#pragma unroll
+    for (int k = 0; k < P; k += 2) {
+        const int32_t d = j[k] - __shfl_up(j[k], 1);
+        const bool both = (uint32_t)k < len && (uint32_t)k < wlen;
+        pairs += __popcll(__ballot(both));
+        far += __popcll(__ballot(both && (d > 32 || d < -32)));
+    }
+    if (lane == 0) {
+        red[0][wv] = far;
+        red[1][wv] = pairs;
+    }
+    __syncthreads();
+    far = pairs = 0;
+#pragma unroll
+    for (int w = 0; w < kRowsBlock / kWave; ++w) {
+        far += red[0][w];
+        pairs += red[1][w];
+    }
+    float s = 0.0f;
+    if (2 * far > pairs) {   // the same for the whole work-group
+#pragma unroll
+        for (int k = P; k < NC; ++k) index(k);
+        int32_t lo = INT32_MAX, hi = INT32_MIN;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            lo = (uint32_t)k < len && j[k] < lo ? j[k] : lo;
+            hi = (uint32_t)k < len && j[k] > hi ? j[k] : hi;
+        }
+        for (int off = kWave / 2; off > 0; off >>= 1) {
+            const int32_t ol = __shfl_xor(lo, off), oh = __shfl_xor(hi, off);
+            lo = ol < lo ? ol : lo;
+            hi = oh > hi ? oh : hi;
+        }
+        if (lane == 0) {
+            red[2][wv] = lo;
+            red[3][wv] = hi;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kRowsBlock / kWave; ++w) {
+            lo = red[2][w] < lo ? red[2][w] : lo;
+            hi = red[3][w] > hi ? red[3][w] : hi;
+        }
+        const int64_t width = (int64_t)hi - lo + 1;
+        const bool staged = width <= kRowsWindow;
+        if (staged) {
+            constexpr int C = 6;   // loads of the copy in flight
+            for (int i0 = 0; i0 < (int)width; i0 += C * kRowsBlock) {
+                float c[C];
+#pragma unroll
+                for (int i = 0; i < C; ++i) {
+                    const int at = i0 + i * kRowsBlock + (int)threadIdx.x;
+                    c[i] = x[lo + (at < (int)width ? at : 0)];
+                }
+#pragma unroll
+                for (int i = 0; i < C; ++i) {
+                    const int at = i0 + i * kRowsBlock + (int)threadIdx.x;
+                    if (at < (int)width) win[at] = c[i];
+                }
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int k0 = 0; k0 < NC; k0 += U) {
+            float av[U], xv[U];
+#pragma unroll
+            for (int u = 0; u < U && k0 + u < NC; ++u) av[u] = value(k0 + u);
+            if (staged) {
+#pragma unroll
+                for (int u = 0; u < U && k0 + u < NC; ++u)
+                    xv[u] = win[(uint32_t)(k0 + u) < len ? j[k0 + u] - lo : 0];
+            } else {
+#pragma unroll
+                for (int u = 0; u < U && k0 + u < NC; ++u)
+                    xv[u] = x[(uint32_t)(k0 + u) < len ? j[k0 + u] : lo];
+            }
+#pragma unroll
+            for (int u = 0; u < U && k0 + u < NC; ++u) s = (uint32_t)(k0 + u) < len ? s + av[u] * xv[u] : s;
+        }
+    } else {
+        int32_t jj[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) jj[u] = j[u];
+        const int32_t some = j[0];   // a column of the row
+        for (uint32_t k0 = 0; k0 < len; k0 += U) {
+            float av[U], xv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                av[u] = BufLoad<float>::template load<kBufNT>(
+                    rAx, k0 + u < len ? oj + (k0 + u) * stride * 4u : kOutside, 0u);
+#pragma unroll
+            for (int u = 0; u < U; ++u) xv[u] = x[k0 + u < len ? jj[u] : some];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                jj[u] = BufLoad<int32_t>::template load<kBufNT>(
+                    rAj, k0 + U + u < len ? oj + (k0 + U + u) * stride * 4u : kOutside, 0u);
+#pragma unroll
+            for (int u = 0; u < U; ++u) s = k0 + u < len ? s + av[u] * xv[u] : s;
+        }
+    }
+    if (row < a.row_end) ((float *)a.out)[row - a.row_start] = s;
+}
+
 typedef void (*StagedFn)(const int32_t *, const void *, const uint32_t *, int64_t, int64_t, const void *, void *,
                          const int32_t *, int64_t, int);
 
@@ -379,6 +532,12 @@ hipError_t ell_apply(const EllView &A, const EllArgs &e, const ReduceSlots &slot
     k.aj_bytes = (uint32_t)(slots_total * 4 * iw);
     k.gate = e.gate;
     k.ax_bytes = (uint32_t)(slots_total * vsz);
+    if (e.mode == ELL_PRODUCT && A.vtype == VT_F32 && T == 1 && iw == 1 && !e.gate && e.block <= 0 && A.ncpr > 16 &&
+        A.ncpr <= 28 && nrows >= kRowsMin && slots_total * 4 < (int64_t(1) << 31)) {
+        fn = A.ncpr <= 24 ? k_product_rows<24> : k_product_rows<28>;
+        hipLaunchKernelGGL(fn, dim3((unsigned)((nrows + kRowsBlock - 1) / kRowsBlock)), dim3(kRowsBlock), 0, s, k);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(block), 0, s, k);
     if (norm)
         hipLaunchKernelGGL(k_finish_norm, dim3(1), dim3(1024), 0, s, (const double *)slots.partials, grid, e.norm2,
