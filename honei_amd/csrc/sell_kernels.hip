@@ -18,6 +18,7 @@
 // widths).  perm maps positions to rows, len holds each position's length.
 
 #include "backend.hh"
+#include "ell_device.hh"
 #include "hip_common.hh"
 
 #pragma clang fp contract(off)
@@ -30,6 +31,7 @@ constexpr int kSellC = 64;          // rows per slice
 constexpr int kSellWindow = 2048;   // rows sorted together
 constexpr int kSellKeys = 64;       // sort keys: lengths 0..62 and 63+ (longer rows share the last key)
 constexpr int kSellChunks = kSellWindow / kSellC;
+constexpr int kSellStaged = 512;    // threads of the staged product
 
 // perm / len of window blockIdx.x: rows by key descending, ties by row index
 // (a counting sort; ranks from wavefront ballots, so the order is fixed).
@@ -207,72 +209,115 @@ __global__ __launch_bounds__(1024) void k_sell_ranges(const int32_t *__restrict_
     }
 }
 
-// y = A x with x staged in LDS: one 1024-thread work-group per sort window
-// (32 slices, two per wavefront).  The window's column range of x is copied
-// into LDS once (coalesced), then each slice streams its index and value
-// arrays and gathers x from LDS.  The terms and their order are k_sell_spmv's,
-// so y has the same bits; a window wider than `cap` entries, or a row with an
-// entry outside the recorded range, sums that row from global x instead.
+// y = A x with x staged in LDS: one 512-thread work-group per sort window (32
+// slices, four per wavefront: one of each eight, so that every wavefront has
+// long and short ones).  The window's column range of x is copied into LDS
+// once (coalesced); each wavefront streams its slices one after the other,
+// the next eight slots' index and value loads issued before this eight's sums
+// (into the next slice, too), and gathers x from LDS.  Slots past a slice's
+// width are asked for outside its buffer (no memory access).  The terms and
+// their order are k_sell_spmv's, so y has the same bits; a window wider than
+// `cap` entries, or a row with an entry outside the recorded range, sums that
+// row from global x instead.
+// Bound by memory once the loads run ahead: a work-group waits four times (its
+// slices' widths, x's range, x, the first slots) before it streams, so two of
+// them share a CU (2 x 80 KiB of doubles at +-4096 columns) and eight slots of
+// each lane are always on their way.  Rows of 1 .. 27 entries within +-4096
+// columns, 2 10^6: FP64 88 -> 77 us (4.8 TB/s), FP32 70 -> 50; 100,003: 23.8 ->
+// 15.9, 21.8 -> 12.8, where two slices per wavefront of 1024 threads waited
+// for every eight or four slots.  Both slices side by side with sixteen slots
+// on their way took 94 (one work-group a CU); twelve slots took 78.
 template <typename VT>
-__global__ __launch_bounds__(1024) void k_sell_spmv_staged(
+__global__ __launch_bounds__(kSellStaged, 4) void k_sell_spmv_staged(
     const int32_t *__restrict__ sAj, const VT *__restrict__ sAx, const int32_t *__restrict__ perm,
     const uint32_t *__restrict__ len, const int32_t *__restrict__ width, const int64_t *__restrict__ base,
     int64_t rows, int64_t slices, const VT *__restrict__ x, VT *__restrict__ y, const int32_t *__restrict__ ranges,
     int64_t cap) {
     extern __shared__ unsigned char sell_stage_raw[];
     VT *win = reinterpret_cast<VT *>(sell_stage_raw);
-    constexpr int U = sizeof(VT) == 8 ? 4 : 8;
-    constexpr int kSlicesPerWave = kSellChunks / (1024 / kWave);
-    const int64_t wdw = xcd_block(blockIdx.x, gridDim.x);   // neighbouring windows on one XCD
+    constexpr int W = kSellStaged / kWave, N = kSellChunks / W, U = 8;   // wavefronts, slices of each, slots a step
+    constexpr int kWidest = 1 << 20;                                     // 32-bit offsets into a slice
+    const int64_t wdw = xcd_block(blockIdx.x, gridDim.x);                // neighbouring windows on one XCD
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    int64_t sl[N], b[N];
+    int w[N];
+    uint32_t l[N];
+    int32_t dst[N];
+    bool narrow = true;
+#pragma unroll
+    for (int h = 0; h < N; ++h) {
+        sl[h] = wdw * kSellChunks + h * W + (h % 2 ? W - 1 - wave : wave);
+        const int64_t i = sl[h] * kSellC + lane;
+        const bool here = sl[h] < slices;
+        w[h] = here ? width[sl[h]] : 0;
+        b[h] = here ? base[sl[h]] : 0;
+        l[h] = i < rows ? len[i] : 0u;
+        dst[h] = i < rows ? perm[i] : -1;
+        narrow = narrow && w[h] <= kWidest;
+    }
+    auto load = [&](int h, int k0, int32_t (&jd)[U], VT (&vd)[U]) {
+        const uint32_t slots = (uint32_t)min(w[h], kWidest) * (uint32_t)kSellC;
+        const auto rj = buffer_rsrc(sAj + b[h], slots * 4u), rv = buffer_rsrc(sAx + b[h], slots * (uint32_t)sizeof(VT));
+        const uint32_t slot = (uint32_t)(k0 * kSellC + lane);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            jd[u] = BufLoad<int32_t>::template load<kBufNT>(rj, slot * 4u + (uint32_t)(u * kSellC * 4), 0u);
+            vd[u] = BufLoad<VT>::template load<kBufNT>(
+                rv, slot * (uint32_t)sizeof(VT) + (uint32_t)(u * kSellC * sizeof(VT)), 0u);
+        }
+    };
+    int32_t j[U], jn[U];
+    VT v[U], vn[U];
+    load(0, 0, j, v);
     const int32_t lo = ranges[2 * wdw], hi = ranges[2 * wdw + 1];
     const int64_t wn = (int64_t)hi - (int64_t)lo + 1;
     const bool staged = hi >= lo && wn <= cap;
-    if (staged)
-        for (int64_t i = threadIdx.x; i < wn; i += blockDim.x) win[i] = x[lo + i];
-    __syncthreads();
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    for (int h = 0; h < kSlicesPerWave; ++h) {
-        const int64_t sl = wdw * kSellChunks + wave * kSlicesPerWave + h;
-        if (sl >= slices) break;
-        const int64_t i = sl * kSellC + lane;
-        const bool valid = i < rows;
-        const uint32_t l = valid ? len[i] : 0u;
-        const int w = width[sl];
-        const int64_t b = base[sl] + lane;
-        VT acc = VT(0);
-        bool outside = !staged;
-        if (staged) {
-            int k = 0;
-            for (; k + U <= w; k += U) {
-                int32_t j[U];
-                VT v[U];
+    if (staged) {
+        constexpr int C = 10;   // loads of the copy in flight
+        for (int i0 = threadIdx.x; i0 < (int)wn; i0 += C * kSellStaged) {
+            VT c[C];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    j[u] = __builtin_nontemporal_load(sAj + b + (int64_t)(k + u) * kSellC);
-                    v[u] = __builtin_nontemporal_load(sAx + b + (int64_t)(k + u) * kSellC);
-                }
+            for (int i = 0; i < C; ++i) c[i] = x[lo + min(i0 + i * kSellStaged, (int)wn - 1)];
+#pragma unroll
+            for (int i = 0; i < C; ++i)
+                if (i0 + i * kSellStaged < (int)wn) win[i0 + i * kSellStaged] = c[i];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < N; ++h) {
+        VT acc = VT(0);
+        bool outside = !staged || !narrow;
+        if (staged && narrow) {
+            for (int k0 = 0;;) {
+                const bool last = k0 + U >= w[h];
+                if (!last)
+                    load(h, k0 + U, jn, vn);
+                else if (h + 1 < N)
+                    load(h + 1 < N ? h + 1 : h, 0, jn, vn);
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const uint32_t o = (uint32_t)(j[u] - lo);
-                    const bool in = o < (uint32_t)wn, use = (uint32_t)(k + u) < l;
+                    const bool in = o < (uint32_t)wn, use = (uint32_t)(k0 + u) < l[h];
                     outside |= use && !in;
                     acc = use ? acc + v[u] * win[in ? o : 0u] : acc;
                 }
-            }
-            for (; k < w; ++k) {
-                const int32_t j = __builtin_nontemporal_load(sAj + b + (int64_t)k * kSellC);
-                const VT v = __builtin_nontemporal_load(sAx + b + (int64_t)k * kSellC);
-                const uint32_t o = (uint32_t)(j - lo);
-                const bool in = o < (uint32_t)wn, use = (uint32_t)k < l;
-                outside |= use && !in;
-                acc = use ? acc + v * win[in ? o : 0u] : acc;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    j[u] = jn[u];
+                    v[u] = vn[u];
+                }
+                if (last) break;
+                k0 += U;
             }
         }
         if (outside) {   // the row from global x, the same terms in the same order
             acc = VT(0);
-            for (uint32_t k = 0; k < l; ++k) acc = acc + sAx[b + (int64_t)k * kSellC] * x[sAj[b + (int64_t)k * kSellC]];
+            const int64_t at = b[h] + lane;
+            for (uint32_t k = 0; k < l[h]; ++k)
+                acc = acc + sAx[at + (int64_t)k * kSellC] * x[sAj[at + (int64_t)k * kSellC]];
         }
-        if (valid) y[perm[i]] = acc;
+        if (dst[h] >= 0) y[dst[h]] = acc;
     }
 }
 
@@ -333,11 +378,11 @@ hipError_t sell_spmv_staged(ValueType vt, const int32_t *sAj, const void *sAx, c
     if (window < 1 || (size_t)window * vs > kMaxStageBytes || windows > 0x7fffffff) return hipErrorInvalidValue;
     const size_t lds = (size_t)window * vs;
     if (vt == VT_F32)
-        hipLaunchKernelGGL(k_sell_spmv_staged<float>, dim3((unsigned)windows), dim3(1024), lds, s, sAj,
+        hipLaunchKernelGGL(k_sell_spmv_staged<float>, dim3((unsigned)windows), dim3(kSellStaged), lds, s, sAj,
                            (const float *)sAx, perm, len, width, base, rows, slices, (const float *)x, (float *)y,
                            ranges, window);
     else if (vt == VT_F64)
-        hipLaunchKernelGGL(k_sell_spmv_staged<double>, dim3((unsigned)windows), dim3(1024), lds, s, sAj,
+        hipLaunchKernelGGL(k_sell_spmv_staged<double>, dim3((unsigned)windows), dim3(kSellStaged), lds, s, sAj,
                            (const double *)sAx, perm, len, width, base, rows, slices, (const double *)x, (double *)y,
                            ranges, window);
     else
