@@ -146,7 +146,8 @@ __global__ void k_zero_words(uint32_t *p, size_t n) {
 // MODE 0: sum x*y ; 1: sum x*x ; 2: x += a*y then sum x*x.  Each thread
 // walks its grid-stride elements four at a time into four accumulators
 // (the four loads in flight together), summed in a fixed order at the end;
-// the grid depends on n only, so the result is reproducible.
+// the grid depends on n only, so the result is reproducible.  A grid of one
+// work-group writes the result, others leave partials for k_finish_sum.
 template <typename V, int MODE>
 __global__ __launch_bounds__(kBlock) void k_reduce(V *x, const V *y, V a, const double *a_dev, int64_t n,
                                                    double *out, ReduceSlots slots, const int *skip) {
@@ -177,7 +178,12 @@ __global__ __launch_bounds__(kBlock) void k_reduce(V *x, const V *y, V a, const 
     for (int u = 0; u < 3; ++u)   // at most three left; compile-time accumulator index
         if (i + u * stride < n) acc[u] += term(i + u * stride);
     const double b = block_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
-    if (threadIdx.x == 0) slots.partials[blockIdx.x] = b;
+    if (threadIdx.x == 0) {
+        if (gridDim.x == 1)
+            *out = 0.0 + b;   // the sum of one partial
+        else
+            slots.partials[blockIdx.x] = b;
+    }
 }
 
 __global__ void k_finish_sum(const double *partials, int64_t nparts, double *out, const int *skip) {
@@ -202,8 +208,9 @@ hipError_t dot(const void *x, const void *y, int64_t n, ValueType vt, double *ou
         const int g = reduce_grid(n);
         hipLaunchKernelGGL((k_reduce<V, 0>), dim3(g), dim3(kBlock), 0, s, (V *)x, (const V *)y,
                            V(0), (const double *)nullptr, n, out, sl, (const int *)nullptr);
-        hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, (const double *)sl.partials, (int64_t)g, out,
-                           (const int *)nullptr);
+        if (g > 1)
+            hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, (const double *)sl.partials, (int64_t)g,
+                               out, (const int *)nullptr);
         return hipGetLastError();
     });
 }
@@ -213,8 +220,9 @@ hipError_t norm2(const void *x, int64_t n, ValueType vt, double *out, const Redu
         const int g = reduce_grid(n);
         hipLaunchKernelGGL((k_reduce<V, 1>), dim3(g), dim3(kBlock), 0, s, (V *)x, (const V *)x,
                            V(0), (const double *)nullptr, n, out, sl, (const int *)nullptr);
-        hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, (const double *)sl.partials, (int64_t)g, out,
-                           (const int *)nullptr);
+        if (g > 1)
+            hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, (const double *)sl.partials, (int64_t)g,
+                               out, (const int *)nullptr);
         return hipGetLastError();
     });
 }
@@ -225,8 +233,9 @@ hipError_t axpy_norm2(void *x, const void *y, double alpha, const double *alpha_
         const int g = reduce_grid(n);
         hipLaunchKernelGGL((k_reduce<V, 2>), dim3(g), dim3(kBlock), 0, s, (V *)x, (const V *)y,
                            (V)alpha, alpha_dev, n, out, sl, skip);
-        hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, (const double *)sl.partials, (int64_t)g, out,
-                           skip);
+        if (g > 1)
+            hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, (const double *)sl.partials, (int64_t)g,
+                               out, skip);
         return hipGetLastError();
     });
 }

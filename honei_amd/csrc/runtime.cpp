@@ -34,8 +34,10 @@ Workspace *workspace_for(hipStream_t s) {
                               sizeof(double) * (size_t)Workspace::kSlotCapacity * Workspace::kSlotLanes);
     hipError_t e2 = hipMalloc((void **)&w->slots.counter, 64);
     hipError_t e3 = hipMalloc((void **)&w->scalars, sizeof(double) * Workspace::kScalars);
-    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
+    hipError_t e4 = hipHostMalloc((void **)&w->returns, sizeof(double) * Workspace::kReturns, hipHostMallocDefault);
+    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess || e4 != hipSuccess) {
         set_error("workspace allocation failed");
+        if (e4 == hipSuccess) (void)hipHostFree(w->returns);
         if (e1 == hipSuccess) (void)hipFree(w->slots.partials);
         if (e2 == hipSuccess) (void)hipFree(w->slots.counter);
         if (e3 == hipSuccess) (void)hipFree(w->scalars);
@@ -47,6 +49,7 @@ Workspace *workspace_for(hipStream_t s) {
         fill_bytes_zero(w->scalars, sizeof(double) * Workspace::kScalars, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
         set_error("workspace initialisation failed");
+        (void)hipHostFree(w->returns);
         (void)hipFree(w->slots.partials);
         (void)hipFree(w->slots.counter);
         (void)hipFree(w->scalars);
@@ -80,6 +83,7 @@ void release_workspaces() {
         (void)hipFree(kv.second->slots.partials);
         (void)hipFree(kv.second->slots.counter);
         (void)hipFree(kv.second->scalars);
+        (void)hipHostFree(kv.second->returns);
         if (kv.second->scratch) (void)hipFree(kv.second->scratch);
         delete kv.second;
     }

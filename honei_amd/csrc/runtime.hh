@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <string>
 
 #include "backend.hh"
@@ -20,6 +21,12 @@ struct Workspace {
     static constexpr int kScalars = 256;
     static constexpr int kSlotCapacity = 1 << 17;   // blocks
     static constexpr int kSlotLanes = 4;
+    // Results of reductions that return to the host: pinned, written by the
+    // reduction's last kernel itself.  A call takes the next of kReturns.
+    double *returns = nullptr;
+    std::atomic<uint32_t> next_return{0};
+    static constexpr uint32_t kReturns = 64;
+    double *take_return() { return returns + next_return.fetch_add(1, std::memory_order_relaxed) % kReturns; }
     void *scratch = nullptr;     // grows on demand, never shrinks
     size_t scratch_bytes = 0;
     // Returns a buffer of at least `bytes` (reallocating only when larger
