@@ -380,6 +380,8 @@ class BatchMG {
     SlotScalars *sc_host_ = nullptr;   // pinned
     int32_t *list_ = nullptr;          // active slots (device, b_compact)
     int32_t *bounds_ = nullptr;        // active counts below each class boundary
+    int32_t *list_u_ = nullptr;        // CG: new and verifying slots, listed after every check for the next iteration
+    int32_t *bounds_u_ = nullptr;
     std::vector<int64_t> boundaries_;  // class firsts, then nslots
 
     hipStream_t s_main_ = nullptr, s_load_ = nullptr;
@@ -409,6 +411,7 @@ class BatchMG {
     hipError_t capture();
     hipError_t capture_iterations(int iters, hipGraph_t *graph, hipGraphExec_t *exec);
     hipError_t note_batch_end();
+    hipError_t enqueue_iterations(int n, hipStream_t s);
     hipError_t enqueue_iteration(hipStream_t s);
     hipError_t enqueue_vcycle(hipStream_t s);
     BWork level_work(int64_t level) const;
@@ -428,8 +431,10 @@ hipError_t b_build(const BuildEntry *entries_dev, const BuildParams &P, int max_
 
 // Which slots a compaction lists.
 enum ListMode : int { LIST_NONIDLE = 0, LIST_ACTIVE = 1, LIST_UNSETTLED = 2 /* NEW or VERIFY */ };
+// One list, or two of different modes, in one launch.
 hipError_t b_compact(const SlotScalars *sc, int64_t nslots, const int64_t *boundaries, int nb, int32_t *list,
-                     int32_t *bounds, int mode, hipStream_t s);
+                     int32_t *bounds, int mode, hipStream_t s, int32_t *list2 = nullptr, int32_t *bounds2 = nullptr,
+                     int mode2 = 0);
 hipError_t b_ell(ValueType vt, int T, int block, int group, EllMode mode, const BMat &m, const BWork &w,
                  int64_t max_slots, void *out, const void *x, const void *rhs, const void *dinv, hipStream_t s);
 // FP64 outer work over the active slots of all classes (w: lo = 0, hi = nclass).
@@ -443,7 +448,8 @@ hipError_t b_outer(OuterOp op, const BClassTab &tab, const BWork &w, int64_t max
 // classes; max_tiles: the tiles of all slots of all classes.
 hipError_t b_dir_spmv(const BClassTab &tab, const BWork &w, int64_t max_tiles, const SlotScalars *sc, hipStream_t s,
                       bool mf);
-// One block per listed slot: reduce its partials and update its scalars.
+// One block per listed slot (FIN_CHECK_CG: per slot that is not idle): reduce
+// its partials and update its scalars.
 hipError_t b_finish(FinishOp op, const BClassTab &tab, const BWork &w, int64_t max_slots, SlotScalars *sc,
                     double tol, int32_t max_outer, hipStream_t s);
 hipError_t b_restrict(ValueType vt, const BLevel &fine, const BLevel &coarse, const BWork &w, hipStream_t s);

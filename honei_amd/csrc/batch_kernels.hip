@@ -49,8 +49,12 @@ __device__ inline void div32(int64_t a, int64_t b, int64_t &q, int64_t &r) {
 __device__ inline int64_t active_first(const BWork &w) { return w.bounds[w.lo]; }
 __device__ inline int64_t active_count(const BWork &w) { return w.bounds[w.hi] - w.bounds[w.lo]; }
 
-// list of non-idle slots (ascending) and, for each boundary k, the number of
-// them below boundaries[k]; one 1024-thread block.
+// Lists of slots (ascending) and, for each boundary k, the number of them
+// below boundaries[k]; a 1024-thread work-group each.
+struct BLists {
+    int32_t *list[2], *bounds[2];
+    int32_t mode[2];
+};
 __device__ inline bool listed(const SlotScalars &s, int mode) {
     if (mode == LIST_ACTIVE) return s.state == SLOT_ACTIVE;
     if (mode == LIST_UNSETTLED) return s.state == SLOT_NEW || s.state == SLOT_VERIFY;
@@ -58,7 +62,9 @@ __device__ inline bool listed(const SlotScalars &s, int mode) {
 }
 
 __global__ __launch_bounds__(1024) void k_b_compact(const SlotScalars *sc, int64_t nslots, BBoundaries bd,
-                                                     int32_t *list, int32_t *bounds, int mode) {
+                                                     BLists ls) {
+    int32_t *const list = blockIdx.x ? ls.list[1] : ls.list[0], *const bounds = blockIdx.x ? ls.bounds[1] : ls.bounds[0];
+    const int mode = blockIdx.x ? ls.mode[1] : ls.mode[0];
     __shared__ int32_t pre[1024];
     const int t = threadIdx.x;
     const int64_t chunk = (nslots + 1023) / 1024;
@@ -863,11 +869,15 @@ __global__ __launch_bounds__(256) void k_b_outer_elem(BClassTab tab, BWork w, co
 //   FIN_BETA: rho = r.z, beta = rho / rho_prev (0 after a (re)start);
 //   FIN_ALPHA: alpha = rho / p.Ap.
 template <int OP>
-__global__ __launch_bounds__(1024) void k_b_finish(BClassTab tab, BWork w, SlotScalars *sc, double tol,
-                                                   int32_t max_outer) {
-    const int64_t a0 = active_first(w), na = active_count(w);
+__global__ __launch_bounds__(1024) void k_b_finish(BClassTab tab, BWork w, int64_t nslots, SlotScalars *sc,
+                                                   double tol, int32_t max_outer) {
+    // the CG check looks at every slot (w is not used): no list of the
+    // non-idle ones is made for it
+    const bool all = OP == FIN_CHECK_CG;
+    const int64_t a0 = all ? 0 : active_first(w), na = all ? nslots : active_count(w);
     for (int64_t a = blockIdx.x; a < na; a += gridDim.x) {
-        const int64_t g = w.list[a0 + a];
+        const int64_t g = all ? a : w.list[a0 + a];
+        if (all && sc[g].state == SLOT_IDLE) continue;   // the same for the whole work-group
         int c = 0;
         while (c + 1 < tab.nclass && g >= tab.c[c + 1].first) ++c;
         const BClassEntry &e = tab.c[c];
@@ -1271,12 +1281,13 @@ int batch_grid(int64_t items, int block) {
 }
 
 hipError_t b_compact(const SlotScalars *sc, int64_t nslots, const int64_t *boundaries, int nb, int32_t *list,
-                     int32_t *bounds, int mode, hipStream_t s) {
+                     int32_t *bounds, int mode, hipStream_t s, int32_t *list2, int32_t *bounds2, int mode2) {
     if (nb < 1 || nb > kMaxClasses + 1 || nslots < 1) return hipErrorInvalidValue;
     BBoundaries bd{};
     bd.n = nb;
     for (int k = 0; k < nb; ++k) bd.v[k] = boundaries[k];
-    hipLaunchKernelGGL(k_b_compact, dim3(1), dim3(1024), 0, s, sc, nslots, bd, list, bounds, mode);
+    const BLists ls{{list, list2}, {bounds, bounds2}, {mode, mode2}};
+    hipLaunchKernelGGL(k_b_compact, dim3(list2 ? 2 : 1), dim3(1024), 0, s, sc, nslots, bd, ls);
     return hipGetLastError();
 }
 
@@ -1375,14 +1386,14 @@ hipError_t b_finish(FinishOp op, const BClassTab &tab, const BWork &w, int64_t m
     const dim3 grid((unsigned)(max_slots < 1024 ? max_slots : 1024)), block(1024);
     switch (op) {
         case FIN_CHECK_DC:
-            hipLaunchKernelGGL(k_b_finish<FIN_CHECK_DC>, grid, block, 0, s, tab, w, sc, tol, max_outer);
+            hipLaunchKernelGGL(k_b_finish<FIN_CHECK_DC>, grid, block, 0, s, tab, w, max_slots, sc, tol, max_outer);
             break;
         case FIN_CHECK_CG:
-            hipLaunchKernelGGL(k_b_finish<FIN_CHECK_CG>, grid, block, 0, s, tab, w, sc, tol, max_outer);
+            hipLaunchKernelGGL(k_b_finish<FIN_CHECK_CG>, grid, block, 0, s, tab, w, max_slots, sc, tol, max_outer);
             break;
-        case FIN_BETA: hipLaunchKernelGGL(k_b_finish<FIN_BETA>, grid, block, 0, s, tab, w, sc, tol, max_outer); break;
+        case FIN_BETA: hipLaunchKernelGGL(k_b_finish<FIN_BETA>, grid, block, 0, s, tab, w, max_slots, sc, tol, max_outer); break;
         case FIN_ALPHA:
-            hipLaunchKernelGGL(k_b_finish<FIN_ALPHA>, grid, block, 0, s, tab, w, sc, tol, max_outer);
+            hipLaunchKernelGGL(k_b_finish<FIN_ALPHA>, grid, block, 0, s, tab, w, max_slots, sc, tol, max_outer);
             break;
         default: return hipErrorInvalidValue;
     }
