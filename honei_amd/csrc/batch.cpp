@@ -504,6 +504,7 @@ BClassTab BatchMG::class_table() const {
         const BLevel &top = L_[(size_t)c.level];
         BClassEntry &e = t.c[k];
         e.first = c.first;
+        e.count = c.count;
         e.n = c.n;
         e.side = c.side;
         e.vld = c.vld;

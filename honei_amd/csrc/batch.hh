@@ -180,7 +180,7 @@ struct BWork {
 // Per-class data of the FP64 outer launches, which cover the active slots of
 // every class in one launch (logical block = 256 rows of one slot).
 struct BClassEntry {
-    int64_t first, n, side, vld, stride, ax_ld, bps, vld_top;
+    int64_t first, count, n, side, vld, stride, ax_ld, bps, vld_top;
     uint32_t side_magic;   // floor(2^32 / side) + 1: v / side = umulhi(v, side_magic) for v side < 2^32
     int64_t pst;   // partial stride per slot: 4 bps
     int64_t nps;   // partials per slot of the CG reductions: one per 64-row chunk
@@ -448,6 +448,9 @@ hipError_t b_outer(OuterOp op, const BClassTab &tab, const BWork &w, int64_t max
 // classes; max_tiles: the tiles of all slots of all classes.
 hipError_t b_dir_spmv(const BClassTab &tab, const BWork &w, int64_t max_tiles, const SlotScalars *sc, hipStream_t s,
                       bool mf);
+// b_dir_spmv's launch for many tiles with weights from the cells (after its
+// checks): one wavefront marching down each tile.
+hipError_t b_dir_march(const BClassTab &tab, const BWork &w, int64_t max_tiles, const SlotScalars *sc, hipStream_t s);
 // One block per listed slot (FIN_CHECK_CG: per slot that is not idle): reduce
 // its partials and update its scalars.
 hipError_t b_finish(FinishOp op, const BClassTab &tab, const BWork &w, int64_t max_slots, SlotScalars *sc,

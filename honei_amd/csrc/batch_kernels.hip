@@ -28,16 +28,26 @@ namespace hipx {
 namespace {
 
 // Launch grids hold about as many work-groups as the chip keeps resident
-// (256 CUs x 2048 threads); work-group p walks logical blocks p, p + grid,
-// p + 2 grid, ... with p = xcd_block(blockIdx.x, grid), so in each round the
-// grid covers one contiguous window of logical blocks and every XCD a
-// contiguous piece of it (few concurrent memory streams, neighbouring rows in
-// one L2).  Logical block counts stay below 2^31 (checked by the launchers),
-// so the per-block index arithmetic is 32-bit.
+// (256 CUs x 2048 threads) and walk the launch's logical blocks by XCD shares
+// (xcd_share).  Logical block counts stay below 2^31 (checked by the
+// launchers), so the per-block index arithmetic is 32-bit.
 constexpr int64_t kResidentThreads = 256 * 2048;
 constexpr int64_t kMaxLogicalBlocks = (int64_t(1) << 31) - 1;
 
-__device__ inline int64_t first_block() { return xcd_block(blockIdx.x, gridDim.x); }
+// The logical blocks of a work-group: every XCD takes one contiguous eighth
+// of the `total` there are, its work-groups side by side in it (neighbouring
+// rows meet in one L2, and no XCD is idle when a few systems run on a grid made
+// for many: the r.z of 256 systems' last iterations 8.0 -> 5.9 us).  (The grid has
+// at least 8 work-groups, so every share is walked.)
+struct Share {
+    int64_t first, end, step;
+    __device__ int64_t count() const { return first < end ? (end - 1 - first) / step + 1 : 0; }
+};
+__device__ inline Share xcd_share(int64_t total) {
+    const int64_t xcd = blockIdx.x % kXcds, each = total / kXcds, more = total % kXcds;
+    const int64_t lo = xcd * each + (xcd < more ? xcd : more);
+    return Share{lo + blockIdx.x / kXcds, lo + each + (xcd < more ? 1 : 0), (gridDim.x - 1 - xcd) / kXcds + 1};
+}
 
 // q = a / b, a - q b for 0 <= a < 2^31, 0 < b < 2^31
 __device__ inline void div32(int64_t a, int64_t b, int64_t &q, int64_t &r) {
@@ -118,7 +128,8 @@ __global__ __launch_bounds__(1024) void k_b_ell(BMat m, BWork w, void *out, cons
     typedef typename VecOf<VT>::type V;
     const int64_t a0 = active_first(w), na = active_count(w);
     const int64_t total = ((na + G - 1) / G) * m.bps;
-    for (int64_t lb = first_block(); lb < total; lb += gridDim.x) {
+    const Share sh = xcd_share(total);
+    for (int64_t lb = sh.first; lb < sh.end; lb += sh.step) {
         int64_t grp, rb_now;
         div32(lb, m.bps, grp, rb_now);
         const int64_t e0 = grp * G;
@@ -212,9 +223,11 @@ constexpr int64_t kMinTallTiles = 256;
 // The element-wise outer launches stage at most kElemSlots logical blocks'
 // slots and scalars per work-group.
 constexpr int kElemSlots = 64;
+// The least multiple of 8 work-groups whose shares of `units` logical blocks
+// (xcd_share) are at most `most` each.
+inline int share_grid(int64_t units, int most) { return (int)((units / (most - 1) / kXcds + 1) * kXcds); }
 inline int tiled_grid(int64_t units, int threads) {
-    const int64_t g = batch_grid(units, threads), need = (units + kTileSlots - 1) / kTileSlots;
-    return (int)(g > need ? g : need);
+    return std::max(batch_grid(units, threads), share_grid(units, kTileSlots));
 }
 
 // The four coarse values around fine node (R, C) of a (2 m + 1)^2 level
@@ -307,9 +320,9 @@ __global__ __launch_bounds__(kPairTileRows * kWave, 8) void k_b_pair(BMat m, BWo
     // sizes the grid so), loaded at once: one list round trip per launch
     // instead of one per tile
     __shared__ int32_t tslot[kTileSlots];
-    const int64_t lb0 = first_block();
-    const int64_t mine = lb0 < total ? (total - 1 - lb0) / gridDim.x + 1 : 0;
-    for (int64_t k = threadIdx.x; k < mine; k += blockDim.x) tslot[k] = w.list[a0 + (lb0 + k * gridDim.x) / ups];
+    const Share sh = xcd_share(total);
+    const int64_t mine = sh.count();
+    for (int64_t k = threadIdx.x; k < mine; k += blockDim.x) tslot[k] = w.list[a0 + (sh.first + k * sh.step) / ups];
     __syncthreads();
     // the staged entry beyond one per node (threads < kExtra): grid rows
     // r0 - 2 and r0 + TR - 1, columns c0 - 2 and c0 + kWave - 1
@@ -334,7 +347,7 @@ __global__ __launch_bounds__(kPairTileRows * kWave, 8) void k_b_pair(BMat m, BWo
     }
     auto on_border = [&](int a, int b) { return a == 0 || a == S - 1 || b == 0 || b == S - 1; };
     int64_t k = 0;
-    for (int64_t lb = lb0; lb < total; lb += gridDim.x, ++k) {
+    for (int64_t lb = sh.first; lb < sh.end; lb += sh.step, ++k) {
         int64_t e, rem, strip, seg;
         div32(lb, ups, e, rem);
         // strips minor: the tiles side by side in a band of rows are
@@ -553,7 +566,8 @@ __global__ __launch_bounds__(256) void k_b_outer_rows(BClassTab tab, BWork w, co
     }
     __syncthreads();
     const int64_t total = pre[tab.nclass];
-    for (int64_t lb = first_block(); lb < total; lb += gridDim.x) {
+    const Share sh = xcd_share(total);
+    for (int64_t lb = sh.first; lb < sh.end; lb += sh.step) {
         int c = 0;
         while (lb >= pre[c + 1]) ++c;
         const BClassEntry &e = tab.c[c];
@@ -644,7 +658,7 @@ __global__ __launch_bounds__(kPairTileRows * kWave, 8) void k_b_dir_spmv(BClassT
     __shared__ int32_t tslot[kTileSlots];
     __shared__ double tbeta[kTileSlots], tscale[kTileSlots];
     __shared__ uint8_t tcur[kTileSlots];
-    const int64_t lb0 = first_block();
+    const int64_t lb0 = xcd_block(blockIdx.x, gridDim.x);
     const int64_t mine = lb0 < total ? (total - 1 - lb0) / gridDim.x + 1 : 0;
     for (int64_t k = threadIdx.x; k < mine; k += blockDim.x) {
         const int64_t lb = lb0 + k * gridDim.x;
@@ -773,10 +787,10 @@ __global__ __launch_bounds__(256) void k_b_outer_elem(BClassTab tab, BWork w, co
     // first iteration)
     __shared__ int32_t tslot[kElemSlots], tflag[kElemSlots];
     __shared__ double ta[kElemSlots], tb[kElemSlots];
-    const int64_t lb0 = first_block();
-    const int64_t mine = lb0 < total ? (total - 1 - lb0) / gridDim.x + 1 : 0;
+    const Share sh = xcd_share(total);
+    const int64_t mine = sh.count();
     for (int64_t k = threadIdx.x; k < mine; k += blockDim.x) {
-        const int64_t lb = lb0 + k * gridDim.x;
+        const int64_t lb = sh.first + k * sh.step;
         int c = 0;
         while (lb >= pre[c + 1]) ++c;
         const int64_t g = w.list[w.bounds[c] + (lb - pre[c]) / ((tab.c[c].bps + R - 1) / R)];
@@ -788,7 +802,7 @@ __global__ __launch_bounds__(256) void k_b_outer_elem(BClassTab tab, BWork w, co
     }
     __syncthreads();
     int64_t kt = 0;
-    for (int64_t lb = lb0; lb < total; lb += gridDim.x, ++kt) {
+    for (int64_t lb = sh.first; lb < sh.end; lb += sh.step, ++kt) {
         int c = 0;
         while (lb >= pre[c + 1]) ++c;
         const BClassEntry &e = tab.c[c];
@@ -971,7 +985,8 @@ __global__ __launch_bounds__(1024) void k_b_finish(BClassTab tab, BWork w, int64
         const int64_t a0_ = active_first(w);                                     \
         const int64_t bpe_ = ((n) + 255) / 256;                                   \
         const int64_t total_ = active_count(w) * bpe_;                            \
-        for (int64_t lb_ = first_block(); lb_ < total_; lb_ += gridDim.x) {      \
+        const Share sh_ = xcd_share(total_);                                      \
+        for (int64_t lb_ = sh_.first; lb_ < sh_.end; lb_ += sh_.step) {          \
             int64_t s_, b_;                                                       \
             div32(lb_, bpe_, s_, b_);                                             \
             const int64_t g = w.list[a0_ + s_];                                   \
@@ -1034,7 +1049,8 @@ __global__ __launch_bounds__(256) void k_b_restrict_rows(BWork w, V *rhs_c, int6
     const int32_t nc = m + 1, nf = 2 * m + 1;
     const int64_t units = active_count(w) * (int64_t)nc * ((nc + kWave - 1) / kWave);
     const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    for (int64_t lb = first_block(); lb * 4 * U < units; lb += gridDim.x) {
+    const Share sh = xcd_share((units + 4 * U - 1) / (4 * U));
+    for (int64_t lb = sh.first; lb < sh.end; lb += sh.step) {
         const int64_t u0 = __builtin_amdgcn_readfirstlane((int32_t)((lb * 4 + wv) * U));
         V f[U][9];
         int64_t dst[U];
@@ -1103,7 +1119,8 @@ __global__ __launch_bounds__(256) void k_b_prolong_rows(BWork w, V *x_f, int64_t
     const int32_t nc = m + 1, nf = 2 * m + 1;
     const int64_t units = active_count(w) * (int64_t)nf * ((nf + kWave - 1) / kWave);
     const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    for (int64_t lb = first_block(); lb * 4 * U < units; lb += gridDim.x) {
+    const Share sh = xcd_share((units + 4 * U - 1) / (4 * U));
+    for (int64_t lb = sh.first; lb < sh.end; lb += sh.step) {
         const int64_t u0 = __builtin_amdgcn_readfirstlane((int32_t)((lb * 4 + wv) * U));
         V t[U][4], xv[U];
         int64_t id[U];
@@ -1277,7 +1294,7 @@ bool entry_fits(int64_t max_slots, int64_t n) { return max_slots * ((n + 255) / 
 
 int batch_grid(int64_t items, int block) {
     const int64_t cap = kResidentThreads / block;
-    return (int)(items < 1 ? 1 : (items > cap ? cap : items));
+    return (int)(items < kXcds ? kXcds : (items > cap ? cap : items));   // every XCD's share has a work-group
 }
 
 hipError_t b_compact(const SlotScalars *sc, int64_t nslots, const int64_t *boundaries, int nb, int32_t *list,
@@ -1306,6 +1323,8 @@ hipError_t b_ell(ValueType vt, int T, int block, int group, EllMode mode, const 
     return hipGetLastError();
 }
 
+constexpr int64_t kDirMarchTiles = 1024;
+
 // Slots per logical block of the row-sum launches, 256-row blocks per
 // logical block of the element-wise launches.
 constexpr int kOuterRowGroup = 1, kOuterElemBlocks = 4;
@@ -1318,10 +1337,10 @@ hipError_t b_outer(OuterOp op, const BClassTab &tab, const BWork &w, int64_t max
         for (int c = 0; c < tab.nclass; ++c)
             if (!tab.c[c].kappa || tab.c[c].kld < (tab.c[c].side - 1) * (tab.c[c].side - 1)) return hipErrorInvalidValue;
     constexpr int G = kOuterRowGroup, R = kOuterElemBlocks;
-    const int64_t ue = (max_blocks + R - 1) / R;
-    const int ge_min = (int)((ue + kElemSlots - 1) / kElemSlots);   // at most kElemSlots logical blocks each
+    int64_t ue = 0;
+    for (int c = 0; c < tab.nclass; ++c) ue += tab.c[c].count * ((tab.c[c].bps + R - 1) / R);
     const dim3 block(256), gr(batch_grid((max_blocks + G - 1) / G, 256)),
-        ge(std::max(batch_grid(ue, 256), ge_min));
+        ge(std::max(batch_grid(ue, 256), share_grid(ue, kElemSlots)));
     switch (op) {
         case OP_DEFECT_ALL:
             if (mf)
@@ -1364,6 +1383,10 @@ hipError_t b_dir_spmv(const BClassTab &tab, const BWork &w, int64_t max_tiles, c
             (mf && (!e.kappa || e.kld < (e.side - 1) * (e.side - 1))) || (!mf && !e.Ax))
             return hipErrorInvalidValue;
     }
+    // a wavefront per tile from one a SIMD on (tile launch / march in us: 648
+    // tiles 18.3 / 17.3, 960 16.4 / 17.0, 1350 22.5 / 19.4, 12,600 179 / 127;
+    // below, the march's 32 rows one after the other: 137 tiles 8 / 16)
+    if (mf && max_tiles >= kDirMarchTiles) return b_dir_march(tab, w, max_tiles, sc, s);
     const int threads = kPairTileRows * kWave;
     const dim3 grid(tiled_grid(max_tiles, threads)), block(threads);
     if (tab.c[0].top64) {

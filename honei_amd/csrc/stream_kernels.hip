@@ -332,7 +332,121 @@ void stream_pair(int pair, dim3 grid, hipStream_t s, const BWork &w, const Strea
         stream_launch<VT, PAIR_POST, WM, false>(grid, s, w, g, lv, out0, xin, nullptr, 0);
 }
 
+// k_b_dir_spmv with weights from the cells, a wavefront marching down each
+// tile: row r's p arrives (and is stored), then row r - 1's q = A p from the
+// last three rows.  p, q and the tile's p.q are that launch's, the p.q too:
+// the tile kernel's thread i holds rows i and i + 16 of the tile, its sixteen
+// wavefronts' sums are added as one more wavefront's lanes.  Bound by memory:
+// 36 bytes a node, 256 systems of five sizes (17.9 10^6 nodes) 179 -> 127 us
+// (5.1 TB/s): no barriers, every wavefront with three rows' loads on their way.
+template <typename Z>
+__global__ __launch_bounds__(256, 4) void k_b_dir_march(BClassTab tab, BWork w, const SlotScalars *sc) {
+    constexpr int T = kPairTileRows, TR = T * kDirNodes, D = 3;   // rows of a tile with its halo, rows in flight
+    static_assert(kDirNodes == 2 && kDirRows == TR - 2, "two rows of a tile for each of its partial sums");
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    int64_t total = 0;
+    for (int c = 0; c < tab.nclass; ++c) total += (int64_t)(w.bounds[c + 1] - w.bounds[c]) * tab.c[c].ntiles;
+    const int64_t quads = (total + 3) / 4, share = quads / kXcds, more = quads % kXcds;
+    const int64_t xcd = blockIdx.x % kXcds, step = (gridDim.x - 1 - xcd) / kXcds + 1;
+    const int64_t lo = xcd * share + (xcd < more ? xcd : more), hi = lo + share + (xcd < more ? 1 : 0);
+    for (int64_t quad = lo + blockIdx.x / kXcds; quad < hi; quad += step) {
+        int64_t q = quad * 4 + wave;
+        if (q >= total) break;
+        int c = 0;
+        int64_t here;
+        while (q >= (here = (int64_t)(w.bounds[c + 1] - w.bounds[c]) * tab.c[c].ntiles)) {
+            q -= here;
+            ++c;
+        }
+        const BClassEntry &e = tab.c[c];
+        const uint32_t si = (uint32_t)q / (uint32_t)e.ntiles, tile = (uint32_t)q - si * (uint32_t)e.ntiles;
+        const uint32_t seg = tile / (uint32_t)e.strips, strip = tile - seg * (uint32_t)e.strips;
+        const int64_t g = w.list[w.bounds[c] + (int64_t)si], ls = g - e.first;
+        const double beta = sc[g].beta, scale = sc[g].scale;
+        const int64_t cur = sc[g].pcur & 1;
+        const int S = (int)e.side;
+        const int r0 = (int)seg * kDirRows, r1 = min(S, r0 + kDirRows);
+        const int c0 = (int)strip * e.tw, c1 = min(S, c0 + e.tw);
+        const int col = c0 - 1 + lane;
+        const bool mine = lane >= 1 && col < c1;
+        const uint32_t cn = (uint32_t)min(max(col, 0), S - 1), cc = (uint32_t)min(max(col, 0), S - 2);
+        const bool side_border = cn == 0 || (int)cn == S - 1;
+        const double *pold = e.p + ls * e.vld + cur * e.palt;
+        double *pnew = e.p + ls * e.vld + (1 - cur) * e.palt, *qs = e.q + ls * e.vld;
+        const Z *zs = (const Z *)e.x_top + g * e.vld_top;
+        const double *ks = e.kappa + g * e.kld;
+        Z pz[D];
+        double po[D], pk[D];
+        auto load = [&](int r, int i) {
+            const int64_t at = (int64_t)min(max(r, 0), min(S - 1, r1)) * S;
+            pz[i] = (zs + at)[cn];
+            po[i] = (pold + at)[cn];
+            pk[i] = (ks + (int64_t)min(max(r - 1, 0), S - 2) * (S - 1))[cc];   // the cells below the row
+        };
+#pragma unroll
+        for (int i = 0; i < D; ++i) load(r0 - 1 + i, i);
+        double part[T];
+#pragma unroll
+        for (int i = 0; i < T; ++i) part[i] = 0.0;
+        double x1 = 0.0, x2 = 0.0, k1 = 0.0, across1 = 0.0;
+        CellRow<double> c2{};
+#pragma unroll
+        for (int I = 0; I < TR; ++I) {
+            const int r = r0 - 1 + I, i = I % D;
+            if (r > r1) continue;   // past a short tile's halo: the same for the whole wavefront
+            // ---- row r of p ----
+            const double z = (double)pz[i] * scale;
+            const double x0 = beta == 0.0 ? z : z + beta * po[i];
+            if (mine && r >= r0 && r < r1) (pnew + (int64_t)r * S)[cn] = x0;
+            // ---- the weights of row r - 1, as q1_cell_weights forms them ----
+            const double k0 = pk[i], kw = from_west(k0), pair0 = kw + k0;
+            CellRow<double> c1r;
+            NodeRow<double> n1;
+            c1r.corner = -div3_rn(k0);
+            c1r.across = -0.5 * div3_rn(pair0);
+            n1.east = -0.5 * div3_rn(k1 + k0);
+            n1.diag = div3_rn(2.0 * ((across1 + kw) + k0));
+            k1 = k0;
+            across1 = pair0;
+            if (I + D < TR) load(r + D, i);
+            // ---- row r - 1 of q = A p ----
+            if (I >= 2) {
+                const int a = r - 1;
+                double t = stencil(c2, n1, c1r, x2, x1, x0);
+                if (side_border || a == 0 || a == S - 1) t = 0.0 + x1;
+                if (mine && a < r1) {
+                    (qs + (int64_t)a * S)[cn] = t;
+                    part[(I - 1) % T] = part[(I - 1) % T] + x1 * t;
+                }
+            }
+            x2 = x1;
+            x1 = x0;
+            c2 = c1r;
+        }
+        double sum = 0.0;
+#pragma unroll
+        for (int i = 0; i < T; ++i) {
+            const double v = wave_sum(part[i]);
+            const int vl = __builtin_amdgcn_readfirstlane(__double2loint(v));
+            const int vh = __builtin_amdgcn_readfirstlane(__double2hiint(v));
+            sum = lane == i ? __hiloint2double(vh, vl) : sum;
+        }
+        sum = wave_sum(sum);
+        if (lane == 0) e.partials[ls * e.pst + tile] = sum;
+    }
+}
+
 }  // namespace
+
+hipError_t b_dir_march(const BClassTab &tab, const BWork &w, int64_t max_tiles, const SlotScalars *sc, hipStream_t s) {
+    const int64_t blocks = (max_tiles + 3) / 4;
+    const dim3 grid((uint32_t)(blocks < kStreamBlocks ? blocks : kStreamBlocks));
+    if (tab.c[0].top64)
+        hipLaunchKernelGGL(k_b_dir_march<double>, grid, dim3(256), 0, s, tab, w, sc);
+    else
+        hipLaunchKernelGGL(k_b_dir_march<float>, grid, dim3(256), 0, s, tab, w, sc);
+    return hipGetLastError();
+}
 
 hipError_t b_pair_stream(ValueType vt, int pair, const BLevel &lv, const BWork &w, void *out0, const void *xin,
                          hipStream_t s, int wmode, void *xc, int64_t vld_c) {

@@ -1,6 +1,7 @@
 """The paired row passes that march down column strips (large levels) against
-one launch per pass, in a batch pool: the same bits while all systems run and
-when the last few do.
+one launch per pass, and the CG direction that marches down its tiles against
+the tile launch, in a batch pool: the same bits while all systems run and when
+the last few do.
 """
 import numpy as np
 import pytest
@@ -17,17 +18,14 @@ def _init():
     yield
 
 
-# launches of many tiles on one level, on each level, and with all levels'
-# systems together; one system short of the rule on its finest level; enough
-# systems for medium and for long segments (shorter ones as systems finish)
-@pytest.mark.parametrize("levels,counts", [([7], [18]), ([7], [17]), ([8], [6]), ([9, 8, 7], [2, 4, 14]),
-                                           ([7], [130]), ([7], [230])])
-@pytest.mark.parametrize("inner", [H.F32, H.BF16, H.F64])
-def test_pairs(inner, levels, counts):
+def _same(levels, counts, **variants):
+    """Both values of the one option in `variants` give the same results."""
+    (option, values), = ((k, v) for k, v in variants.items() if isinstance(v, tuple))
+    rest = {k: v for k, v in variants.items() if k != option}
     got = []
-    for pair in (0, 1):
-        B = H.Batch(levels, counts, H.batch_config(autotune=0, inner_vtype=inner, pair_sweeps=pair, iters_per_launch=4,
-                                                   max_outer=40))
+    for value in values:
+        B = H.Batch(levels, counts, H.batch_config(autotune=0, iters_per_launch=4, max_outer=40, **rest,
+                                                   **{option: value}))
         keep, slots = [], []
         for c, lv in enumerate(levels):
             for j in range(counts[c]):
@@ -55,3 +53,21 @@ def test_pairs(inner, levels, counts):
         assert ia == ib
         assert np.array_equal(xa, xb)
         assert np.isfinite(xa).all() and xa.any()
+
+
+# launches of many tiles on one level, on each level, and with all levels'
+# systems together; one system short of the rule on its finest level; enough
+# systems for medium and for long segments (shorter ones as systems finish)
+@pytest.mark.parametrize("levels,counts", [([7], [18]), ([7], [17]), ([8], [6]), ([9, 8, 7], [2, 4, 14]),
+                                           ([7], [130]), ([7], [230])])
+@pytest.mark.parametrize("inner", [H.F32, H.BF16, H.F64])
+def test_pairs(inner, levels, counts):
+    _same(levels, counts, inner_vtype=inner, pair_sweeps=(0, 1))
+
+
+# 1024 tiles (15, 45 and 162 a system of levels 7, 8 and 9) and fewer, every
+# band of rows short of its full height among them
+@pytest.mark.parametrize("levels,counts", [([7], [69]), ([7], [68]), ([9, 8, 7], [4, 6, 8]), ([8, 5, 3], [20, 80, 60])])
+@pytest.mark.parametrize("inner", [H.F32, H.F64])
+def test_direction(inner, levels, counts):
+    _same(levels, counts, inner_vtype=inner, matrix_free=(0, 1))
