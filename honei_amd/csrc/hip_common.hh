@@ -165,10 +165,22 @@ struct ReduceSlots {
     int capacity;          // max blocks
 };
 
-// Deterministic sum of partials[b*lanes + lane] over b < nparts by one block.
+// Deterministic sum of partials[b*lanes + lane] over b < nparts by one block:
+// a thread's in ascending order, the loads of eight of them issued before the
+// first is added.
 __device__ inline double sum_partials(const double *partials, int64_t nparts, int lanes, int lane) {
+    constexpr int U = 8;
     double v = 0.0;
-    for (int64_t b = threadIdx.x; b < nparts; b += blockDim.x) v += partials[b * lanes + lane];
+    for (int64_t b = threadIdx.x; b < nparts; b += (int64_t)U * blockDim.x) {
+        double p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t at = b + u * (int64_t)blockDim.x;
+            p[u] = partials[(at < nparts ? at : b) * lanes + lane];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) v = b + u * (int64_t)blockDim.x < nparts ? v + p[u] : v;
+    }
     return block_sum(v);
 }
 
