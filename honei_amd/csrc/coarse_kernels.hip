@@ -16,12 +16,14 @@
 // the 3^2 CG run in one wavefront, without barriers; the CG's sums and products
 // are register moves between its nine lanes.
 //
-// What bounds it: FP64 arithmetic of the weights (a quarter), VALU issue of
-// the 65^2 phases (a third), and the chain of short phases below.  One system
-// of 257^2 nodes 20.9 us; 18 systems, levels 1..6, 17.8 us; 256 systems of up
-// to 513^2 nodes 20.6 us.  (With flat node numbers, five a thread, and weights
-// in LDS below 33^2: 26.5, 22.8, 26.4; an earlier launch for levels 1..4 alone:
-// 32, 28, 38.)  Distinct weights read instead of formed: 21.8, 16.1, 22.2.
+// What bounds it: FP64 arithmetic of the weights (a fifth), VALU issue of the
+// 65^2 phases (a third), and the chain of short phases below.  One system of
+// 257^2 nodes 18.9 us (constant operator 14.5); 16 bf16 systems of levels
+// 5..8 19.8; 256 systems of up to 513^2 nodes 23.7.  (With a thread's four nodes of 65^2
+// sixteen rows apart, so that they share neither cells nor staged rows: 20.5,
+// 16.1, 22.4, 25.8; with flat node numbers, five a thread, and weights in LDS
+// below 33^2: 26.5 for the first; an earlier launch for levels 1..4 alone: 32.)
+// Distinct weights read instead of formed: 21.8 against 20.9.
 //
 // Sums and roundings are those of the level-by-level launches: rows in column
 // order, boundary rows 0 + 1 x, transfers as k_b_restrict_rows /
@@ -55,16 +57,16 @@ constexpr int kTail = 160;
 __host__ __device__ constexpr int lds_elements(int top) { return (vec_at(top + 1) + kTail + 3) / 4 * 4; }
 
 // Interior nodes over threads: a wavefront takes `rows` grid rows of `cols`
-// columns (a power of two, one more than the level's interior), the
-// work-group np times `step` rows.  So a node's stencil is one address and
-// fixed offsets.
+// columns (a power of two, one more than the level's interior); a thread has
+// np nodes, one above the other (np > 1: rows = 1).  So a node's stencil is one
+// address and fixed offsets, and a thread's nodes share staged rows and cells.
 template <int L> struct Lv {
     static constexpr int side = side_at(L), n = nodes_at(L);
     static constexpr bool wave = L <= kWaveTop;
     static constexpr int cols = 1 << L < kWave ? 1 << L : kWave, rows = kWave / cols;
     static constexpr int waves = (1 << L) / rows < 1 ? 1 : ((1 << L) / rows < kWaves ? (1 << L) / rows : kWaves);
-    static constexpr int step = waves * rows, np = ((1 << L) + step - 1) / step;
-    static_assert((1 << L) <= cols, "one lane per column");
+    static constexpr int np = ((1 << L) + waves * rows - 1) / (waves * rows);
+    static_assert((1 << L) <= cols && (np == 1 || rows == 1), "one lane per column");
 };
 
 // what a thread keeps of its interior nodes: in registers; of the wavefront's
@@ -74,7 +76,7 @@ template <typename V, int NP> struct Regs {
 };
 // ... and what that is made from, as loaded (rhs used on the finest level only)
 template <typename V, int NP> struct Raw {
-    double c[NP][4];
+    double c[NP + 1][2];
     V di[NP], rh[NP];
 };
 constexpr int kKeep = 11 * kWave;   // LDS elements of one of the wavefront's levels
@@ -110,20 +112,20 @@ template <typename V> __device__ inline V lane_value(V v, int lane) {
     }
 }
 
-// Node 0 of this thread on level L: grid position and LDS index; node q is
-// q * Lv<L>::step rows further.
+// Node 0 of this thread on level L: grid position and LDS index; node q is q
+// rows further.
 template <int L> struct Pos {
     int r, c, id;
     bool mine;   // the wavefront takes part
     __device__ inline Pos(int lane_, int wv) {
         const int lane = fresh(lane_);
-        r = 1 + wv * Lv<L>::rows + lane / Lv<L>::cols;
+        r = 1 + wv * Lv<L>::rows * Lv<L>::np + lane / Lv<L>::cols;
         c = 1 + lane % Lv<L>::cols;
         id = r * Lv<L>::side + c;
         mine = wv < Lv<L>::waves;
     }
     __device__ inline bool live(int q) const {
-        return c < Lv<L>::side - 1 && r + q * Lv<L>::step < Lv<L>::side - 1;
+        return c < Lv<L>::side - 1 && r + q < Lv<L>::side - 1;
     }
 };
 
@@ -154,17 +156,19 @@ template <typename VT, bool COEF, int TOP> struct Cycle {
         if (!p.mine) return;
         const V *dinv = (const V *)cl.dinv + g * cl.vld, *rhs = (const V *)cl.rhs + g * cl.vld;
         const double *kap = cl.kappa + g * cl.kld;
+        // a lane without a node: the last interior one's
+        const int c = min(p.c, S - 2);
+        if constexpr (COEF) {
+#pragma unroll
+            for (int k = 0; k <= Lv<L>::np; ++k) {
+                const double *cs = kap + (min(p.r - 1 + k, S - 2) * (S - 1) + c - 1);
+                raw.c[k][0] = cs[0];
+                raw.c[k][1] = cs[1];
+            }
+        }
 #pragma unroll
         for (int q = 0; q < Lv<L>::np; ++q) {
-            // a lane without a node: the last interior one's
-            const int r = min(p.r + q * Lv<L>::step, S - 2), c = min(p.c, S - 2);
-            if constexpr (COEF) {
-                const double *cs = kap + ((r - 1) * (S - 1) + c - 1), *cs2 = cs + (S - 1);
-                raw.c[q][0] = cs[0];
-                raw.c[q][1] = cs[1];
-                raw.c[q][2] = cs2[0];
-                raw.c[q][3] = cs2[1];
-            }
+            const int r = min(p.r + q, S - 2);
             raw.di[q] = dinv[r * S + c];
             raw.rh[q] = rhs[r * S + c];
         }
@@ -174,14 +178,13 @@ template <typename VT, bool COEF, int TOP> struct Cycle {
     __device__ inline void settle(Regs<V, Lv<L>::np> &reg, const Raw<V, Lv<L>::np> &raw, bool top, int v) const {
         const Pos<L> p(lane, v);
         if (!p.mine) return;
+        if constexpr (COEF) q1_column_weights<VT, Lv<L>::np, V>(raw.c, reg.w);
 #pragma unroll
         for (int q = 0; q < Lv<L>::np; ++q) {
-            if constexpr (COEF)
-                q1_interior_weights_cells<VT, V>(raw.c[q][0], raw.c[q][1], raw.c[q][2], raw.c[q][3], reg.w[q]);
             reg.di[q] = raw.di[q];
             reg.rh[q] = raw.rh[q];
             if (top && p.live(q))
-                (mem + vec_at(L) + Lv<L>::n)[p.id + q * Lv<L>::step * Lv<L>::side] = raw.di[q] * raw.rh[q];
+                (mem + vec_at(L) + Lv<L>::n)[p.id + q * Lv<L>::side] = raw.di[q] * raw.rh[q];
         }
     }
 
@@ -211,20 +214,22 @@ template <typename VT, bool COEF, int TOP> struct Cycle {
         constexpr int S = Lv<L>::side;
         const Pos<L> p(lane, wv);
         if (p.mine) {
-            src += p.id;
+            src += p.id - S - 1;
+            V x[3][3], w[9];
+            if constexpr (!COEF) q1_constant_weights<VT, V>(w);
 #pragma unroll
-            for (int q = 0; q < Lv<L>::np; ++q) {
-                constexpr int Q = Lv<L>::step * S;
-                V x[9], w[9], s = V(0);
+            for (int k = 0; k < Lv<L>::np + 2; ++k) {   // staged row k: above node k - 2
 #pragma unroll
-                for (int k = 0; k < 9; ++k) x[k] = src[q * Q + (k / 3 - 1) * S + (k % 3 - 1)];
-                if constexpr (!COEF) q1_constant_weights<VT, V>(w);
+                for (int j = 0; j < 3; ++j) x[k % 3][j] = src[k * S + j];
+                if (k < 2) continue;
+                const int q = k - 2;
+                V s = V(0);
 #pragma unroll
-                for (int k = 0; k < 9; ++k) s = s + (COEF ? reg.w[q][k] : w[k]) * x[k];
+                for (int i = 0; i < 9; ++i) s = s + (COEF ? reg.w[q][i] : w[i]) * x[(q + i / 3) % 3][i % 3];
                 const V d = reg.rh[q] - s;
-                if (p.live(q)) dst[p.id + q * Q] = DEFECT ? d : x[4] + d * reg.di[q];
+                if (p.live(q)) dst[p.id + q * S] = DEFECT ? d : x[(q + 1) % 3][1] + d * reg.di[q];
             }
-            src -= p.id;
+            src -= p.id - S - 1;
         }
         if (top && bid >= 0) {
             const V x = src[bid], d = brh - (V(0) + V(1) * x);
@@ -241,8 +246,8 @@ template <typename VT, bool COEF, int TOP> struct Cycle {
         const V *f = other<C + 1>() + 2 * p.r * SF + 2 * p.c;
 #pragma unroll
         for (int q = 0; q < Lv<C>::np; ++q) {
-            const V *f0 = f + q * 2 * Lv<C>::step * SF, *fm = f0 - SF, *fp = f0 + SF;
-            const int d = p.c - (p.r + q * Lv<C>::step);
+            const V *f0 = f + q * 2 * SF, *fm = f0 - SF, *fp = f0 + SF;
+            const int d = p.c - (p.r + q);
             const V h = V(0.5), qq = V(0.25);
             const V A_ = h * fm[0], B_ = h * fp[0], C_ = h * f0[1], D_ = h * f0[-1];
             const V E_ = qq * fp[1], F_ = qq * fp[-1], G_ = qq * fm[1], H_ = qq * fm[-1];
@@ -268,7 +273,7 @@ template <typename VT, bool COEF, int TOP> struct Cycle {
         const Pos<C> p(lane, wv);
         restrict_to<C>([&](int q, V s) {
             reg.rh[q] = s;
-            if (p.live(q)) (mem + vec_at(C) + Lv<C>::n)[p.id + q * Lv<C>::step * Lv<C>::side] = reg.di[q] * s;
+            if (p.live(q)) (mem + vec_at(C) + Lv<C>::n)[p.id + q * Lv<C>::side] = reg.di[q] * s;
         });
     }
 
@@ -293,7 +298,7 @@ template <typename VT, bool COEF, int TOP> struct Cycle {
         if (p.mine) {
 #pragma unroll
             for (int q = 0; q < Lv<L>::np; ++q) {
-                const int r = p.r + q * Lv<L>::step, c = p.c, id = p.id + q * Lv<L>::step * Lv<L>::side;
+                const int r = p.r + q, c = p.c, id = p.id + q * Lv<L>::side;
                 const V *c0 = xc + (r >> 1) * nc + (c >> 1), *c1 = xc + ((r + 1) >> 1) * nc + (c >> 1);
                 const int dc = c & 1;
                 const V t0 = c0[0], t1 = c0[dc], t2 = c1[0], t3 = c1[dc];

@@ -62,6 +62,42 @@ __device__ inline float bf16_round(float v) {
     return __uint_as_float((u >> 16) << 16);
 }
 
+// q1_interior_weights_cells of NP nodes, one above the other, from the rows of
+// two cells around them (c[k] = cells west and east of cell row k, row 0 below
+// the lowest node): what neighbouring nodes share -- their common cells and
+// the pairs of them -- formed once, by the same expressions.
+template <typename VT, int NP, typename A>
+__device__ inline void q1_column_weights(const double (&c)[NP + 1][2], A (&w)[NP][9]) {
+    auto put = [](double v) {
+        A a = (A)v;
+        if constexpr (sizeof(VT) == 2) a = bf16_round(a);
+        return a;
+    };
+    double below = 0.0;
+    A west = A(0), across = A(0), east = A(0);
+#pragma unroll
+    for (int k = 0; k <= NP; ++k) {
+        const double row = c[k][0] + c[k][1];
+        const A wk = put(-div3_rn(c[k][0])), ak = put(-0.5 * div3_rn(row)), ek = put(-div3_rn(c[k][1]));
+        if (k) {
+            A *u = w[k - 1];
+            u[0] = west;
+            u[1] = across;
+            u[2] = east;
+            u[3] = put(-0.5 * div3_rn(c[k - 1][0] + c[k][0]));
+            u[4] = put(div3_rn(2.0 * (below + c[k][0] + c[k][1])));
+            u[5] = put(-0.5 * div3_rn(c[k - 1][1] + c[k][1]));
+            u[6] = wk;
+            u[7] = ak;
+            u[8] = ek;
+        }
+        below = row;
+        west = wk;
+        across = ak;
+        east = ek;
+    }
+}
+
 // The nine weights of an interior row of the constant operator as a kernel
 // reading the stored matrix of value type VT sees them.
 template <typename VT, typename A>
