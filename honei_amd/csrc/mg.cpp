@@ -557,10 +557,17 @@ hipError_t MGHierarchy::solve_pcg_q1(const double *b, double *x, hipStream_t s, 
     };
     int64_t chunk = 4;
     for (int64_t k = 0;;) {
+        const int64_t first = k;
         for (int64_t e = k + chunk; k < e; ++k) {
-            HX(mg_pcg_rhs(inner, top.rhs, r, o.n, sc, s));
+            // an iteration's check with the next one's right-hand side, the
+            // chunk's last by itself
+            const bool late = mg_pcg_late_check(o.n);
+            if (late && k > first)
+                HX(mg_pcg_check_rhs(inner, top.rhs, r, o.n, sc, slots_, s));
+            else
+                HX(mg_pcg_rhs(inner, top.rhs, r, o.n, sc, s));
             HX(q1_vcycle(max_level, &sc->work, s));
-            HX(mg_pcg_outer(inner, o, top.x, x, r, p[k & 1], p[(k + 1) & 1], q64_, sc, slots_, s));
+            HX(mg_pcg_outer(inner, o, top.x, x, r, p[k & 1], p[(k + 1) & 1], q64_, sc, slots_, !late || k + 1 == e, s));
         }
         HX(mg_pcg_defect(false, o, b, x, r, sc, slots_, cfg.tolerance, cap, s));
         HX(read_back());

@@ -199,21 +199,32 @@ __global__ __launch_bounds__(kRows) void k_mg_update(double *x, const double *p,
     });
 }
 
-// after the update: the iteration's decision (one work-group)
+// after the update: the iteration's decision from the partials of ||r||^2, the
+// same in every thread that has r2; whether the solve goes on, and its norm
+__device__ inline bool pcg_goes_on(const MgPcgScalars *sc, double r2, double &nrm, bool &verify) {
+    nrm = sqrt(r2);
+    verify = nrm < sc->tol * sc->initial;
+    return !verify && sc->iters < sc->cap && isfinite(nrm);
+}
+__device__ inline void pcg_decide(MgPcgScalars &c, double r2, double nrm, bool verify, bool on) {
+    c.r2 = r2;
+    c.nrm = nrm;
+    c.rho_prev = c.rz;
+    if (verify)
+        c.verify = 1;
+    else if (!on)
+        c.done = 1;
+    c.halt = c.verify | c.done;
+    c.work.end = c.halt ? 0 : 1;
+}
 __global__ __launch_bounds__(1024) void k_mg_check(MgPcgScalars *sc, const double *pr2, int64_t nparts) {
     if (block_uniform_flag(&sc->halt)) return;
     const double r2 = sum_partials(pr2, nparts, 1, 0);
     if (threadIdx.x != 0) return;
-    MgPcgScalars &c = *sc;
-    c.r2 = r2;
-    c.nrm = sqrt(r2);
-    c.rho_prev = c.rz;
-    if (c.nrm < c.tol * c.initial)
-        c.verify = 1;
-    else if (!(c.iters < c.cap) || !isfinite(c.nrm))
-        c.done = 1;
-    c.halt = c.verify | c.done;
-    c.work.end = c.halt ? 0 : 1;
+    double nrm;
+    bool verify;
+    const bool on = pcg_goes_on(sc, r2, nrm, verify);
+    pcg_decide(*sc, r2, nrm, verify, on);
 }
 
 // INIT after the first defect, CONFIRM after the gated true defect (one
@@ -247,6 +258,26 @@ __global__ __launch_bounds__(256) void k_mg_rhs(V *rhs, const double *d, int64_t
                                                 const double *nrm, const int *halt) {
     if (*halt) return;
     const double f = inv ? *inv : 1.0 / *nrm;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        rhs[i] = (V)(d[i] * f);
+}
+
+// the decision of the iteration before and this one's right-hand side, up to
+// kSplitRows rows: every work-group sums the (at most 256) partials and comes
+// to the same decision, the first writes it (the others read nothing that it
+// changes, but for a halt, which they come to themselves); 257^2 nodes 2.0 and
+// 3.9 us in two launches
+template <typename V>
+__global__ __launch_bounds__(256) void k_mg_check_rhs(V *rhs, const double *d, int64_t n, MgPcgScalars *sc,
+                                                      const double *pr2, int64_t nparts) {
+    if (block_uniform_flag(&sc->halt)) return;
+    const double r2 = sum_partials(pr2, nparts, 1, 0);
+    double nrm;
+    bool verify;
+    const bool on = pcg_goes_on(sc, r2, nrm, verify);
+    if (blockIdx.x == 0 && threadIdx.x == 0) pcg_decide(*sc, r2, nrm, verify, on);
+    if (!on) return;
+    const double f = 1.0 / nrm;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         rhs[i] = (V)(d[i] * f);
 }
@@ -331,6 +362,20 @@ hipError_t mg_pcg_defect(bool init, const Q1Outer &o, const double *b, const dou
     return hipGetLastError();
 }
 
+bool mg_pcg_late_check(int64_t n) { return n <= kSplitRows; }
+
+hipError_t mg_pcg_check_rhs(ValueType inner, void *rhs, const double *r, int64_t n, MgPcgScalars *sc,
+                            const ReduceSlots &sl, hipStream_t s) {
+    const double *pr2 = parts(sl, 2);
+    if (inner == VT_F64)
+        hipLaunchKernelGGL(k_mg_check_rhs<double>, dim3(stream_groups(n)), dim3(256), 0, s, (double *)rhs, r, n, sc, pr2,
+                           dot_groups(n));
+    else
+        hipLaunchKernelGGL(k_mg_check_rhs<float>, dim3(stream_groups(n)), dim3(256), 0, s, (float *)rhs, r, n, sc, pr2,
+                           dot_groups(n));
+    return hipGetLastError();
+}
+
 hipError_t mg_pcg_rhs(ValueType inner, void *rhs, const double *r, int64_t n, const MgPcgScalars *sc, hipStream_t s) {
     if (inner == VT_F64)
         hipLaunchKernelGGL(k_mg_rhs<double>, dim3(stream_groups(n)), dim3(256), 0, s, (double *)rhs, r, n,
@@ -342,7 +387,8 @@ hipError_t mg_pcg_rhs(ValueType inner, void *rhs, const double *r, int64_t n, co
 }
 
 hipError_t mg_pcg_outer(ValueType inner, const Q1Outer &o, const void *x_top, double *x, double *r, const double *pold,
-                        double *pnew, double *q, MgPcgScalars *sc, const ReduceSlots &sl, hipStream_t s) {
+                        double *pnew, double *q, MgPcgScalars *sc, const ReduceSlots &sl, bool check,
+                        hipStream_t s) {
     const int64_t g = dot_groups(o.n);
     const dim3 grid((unsigned)g), blk(kRows);
     double *prz = parts(sl, 0), *ppq = parts(sl, 1), *pr2 = parts(sl, 2);
@@ -377,7 +423,7 @@ hipError_t mg_pcg_outer(ValueType inner, const Q1Outer &o, const void *x_top, do
                            (const MgPcgScalars *)sc, ppq);
     hipLaunchKernelGGL(k_mg_update, grid, blk, 0, s, x, (const double *)pnew, r, (const double *)q, o.n, sc,
                        (const double *)ppq, g, pr2);
-    hipLaunchKernelGGL(k_mg_check, dim3(1), dim3(1024), 0, s, sc, (const double *)pr2, g);
+    if (check) hipLaunchKernelGGL(k_mg_check, dim3(1), dim3(1024), 0, s, sc, (const double *)pr2, g);
     return hipGetLastError();
 }
 

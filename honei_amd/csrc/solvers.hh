@@ -92,10 +92,16 @@ hipError_t mg_mixed_rhs(float *rhs, const double *d, int64_t n, const MgMixedSca
 hipError_t mg_pcg_defect(bool init, const Q1Outer &o, const double *b, const double *x, double *r, MgPcgScalars *sc,
                          const ReduceSlots &sl, double tol, int cap, hipStream_t s);
 hipError_t mg_pcg_rhs(ValueType inner, void *rhs, const double *r, int64_t n, const MgPcgScalars *sc, hipStream_t s);
+// The same after the check of the iteration before, in one launch, for systems
+// with mg_pcg_late_check() (that iteration's mg_pcg_outer without its check).
+bool mg_pcg_late_check(int64_t n);
+hipError_t mg_pcg_check_rhs(ValueType inner, void *rhs, const double *r, int64_t n, MgPcgScalars *sc,
+                            const ReduceSlots &sl, hipStream_t s);
 // One iteration after its V-cycle (result x_top): r.z, direction and q = A p,
-// update, check.
+// update, and the check.
 hipError_t mg_pcg_outer(ValueType inner, const Q1Outer &o, const void *x_top, double *x, double *r, const double *pold,
-                        double *pnew, double *q, MgPcgScalars *sc, const ReduceSlots &sl, hipStream_t s);
+                        double *pnew, double *q, MgPcgScalars *sc, const ReduceSlots &sl, bool check,
+                        hipStream_t s);
 
 // Host side of CGSolver (solvers_capi.cpp), shared by honei_hip_cg_solve and
 // its allocation-free variant: argument checks (HONEI status code), the
