@@ -502,79 +502,56 @@ def serving_requests(seconds, rate=SERVE_RATE, seed=SERVE_SEED):
     return patterns.serving_requests(seconds, rate, seed, SERVE_LEVELS)
 
 
-def q1_nnz(side):
-    """Stored entries of the Q1 operator: 9 per interior row, 1 per Dirichlet row."""
-    return 9 * (side - 2) ** 2 + 4 * (side - 1)
-
-
-def slot_solve_bytes(L, iters, vs=4, fused=4, pair_from=5, mf=True):
+def slot_solve_bytes(L, iters, coarse=6):
     """Algorithmic bytes of every launch one slot of finest level L takes
-    part in during a batched step with `iters` outer (CG) iterations, each
-    launch counted by its own compulsory traffic (SURVEY-style: values and
-    vectors once per launch, index streams only where a launch reads one).
-    mf (the pool's default, matrix_free 1): the paired passes and the FP64
-    row sums read the cell coefficients (8 bytes per cell) instead of
-    stored values, and those values are never built.
+    part in during a batched step with `iters` outer (CG) iterations, in the
+    pool's default form (FP32 vectors, matrix_free 1), each launch counted by
+    its own compulsory traffic (vectors once per launch, weights as the cell
+    coefficients, 8 bytes per cell; no values or indices are read or stored):
 
       build    : coefficient read from its source and written, every coarser
-                 coefficient from four finer cells, every stored level's
-                 values (vs bytes each) and every level's dinv, the FP64
-                 operator (not with mf), b copied, x0;
+                 coefficient from four finer cells, every level's dinv, b
+                 copied, x0;
       settle   : r = b - A x in FP64 at the start and at the verification
-                 (nnz*8 + 24n each, mf: 8 per cell + 24n; neighbours from
-                 the grid, no indices), each followed by r/|r| -> FP32
-                 (12n);
+                 (8 per cell + 24n each; neighbours from the grid), each
+                 followed by r/|r| -> FP32 (12n);
       per iteration, on the finest level n = n_L:
                  r.z (12n), p = z + beta p with q = A p and p.q in one
-                 launch (nnz*8 + 28n, mf: 8 per cell + 28n: z and p read,
-                 the new p and q written), x, r update with |r|^2 and the
-                 next cycle's FP32 right-hand side (52n);
-      per iteration, per level l (n_l, nnz_l):
-                 l >= pair_from: paired Jacobi0 + defect and paired two
-                 sweeps (nnz_l*vs + 16 n_l each, mf: 8 per cell + 16 n_l),
-                 restriction (4 n_l + 4 n_{l-1}), the prolongation fused
-                 into the paired sweeps (4 n_{l-1} more: the coarse result
-                 read, the fine x read in place of the corrected vector);
-                 2 <= l <= fused: the fused coarse launch's passes, each
-                 with its index stream: Jacobi0, one Jacobi sweep, the
-                 defect, two post sweeps (nnz_l*(vs+4) + 16 n_l, the defect
-                 12 n_l), restriction and prolongation as above;
-                 level 1 (3x3, coarse CG): not counted."""
+                 launch (8 per cell + 28n: z and p read, the new p and q
+                 written), x, r update with |r|^2 and the next cycle's FP32
+                 right-hand side (52n);
+      per iteration, per level l (n_l):
+                 l > coarse: down, Jacobi0 + defect + restriction (8 per
+                 cell + 12 n_l + 4 n_{l-1}: the defect is not stored); up,
+                 prolongation and two sweeps (8 per cell + 16 n_l +
+                 4 n_{l-1});
+                 l <= coarse: one launch for all of them, cells and dinv of
+                 each once, the finest one's right-hand side and result."""
     def n_(l):
         return (2 ** l + 1) ** 2
-
-    def nnz_(l):
-        return q1_nnz(2 ** l + 1)
 
     def cells(l):
         return 4 ** l
 
-    n, nnz = n_(L), nnz_(L)
-    op64 = 8 * cells(L) if mf else nnz * 8     # bytes of the FP64 operator a row sum reads
-    build = 16 * cells(L) + 24 * n + (0 if mf else nnz * 8)
+    n, op64 = n_(L), 8 * cells(L)
+    build = 16 * cells(L) + 24 * n
     for l in range(1, L + 1):
-        stored = not (mf and l >= pair_from)
-        build += 8 * cells(l) + (nnz_(l) * vs if stored else 0) + 4 * n_(l)
+        build += 8 * cells(l) + 4 * n_(l)
         if l < L:
             build += 8 * cells(l + 1) + 8 * cells(l)
     settle = 2 * (op64 + 24 * n + 12 * n)
-    it = 12 * n + (op64 + 28 * n) + 52 * n
-    for l in range(2, L + 1):
-        nl, zl, nc = n_(l), nnz_(l), n_(l - 1)
-        transfers = (4 * nl + 4 * nc) + (8 * nl + 4 * nc)
-        if l >= pair_from:
-            it += 2 * ((8 * cells(l) if mf else zl * vs) + 16 * nl) + (4 * nl + 4 * nc) + 4 * nc
-        elif l <= fused:
-            sweep = zl * (vs + 4) + 16 * nl
-            it += 4 * sweep + (zl * (vs + 4) + 12 * nl) + transfers
+    top = min(L, coarse)
+    it = 12 * n + (op64 + 28 * n) + 52 * n + 8 * n_(top)
+    for l in range(1, L + 1):
+        it += 8 * cells(l) + 4 * n_(l) if l <= coarse else 16 * cells(l) + 28 * n_(l) + 8 * n_(l - 1)
     return build + settle + iters * it
 
 
-def step_roofline(levels, iters, seconds, vs=4):
+def step_roofline(levels, iters, seconds):
     """Step-level roofline: the algorithmic bytes of every launch of one
     batched step (slot_solve_bytes summed over the systems with their own
     iteration counts) over the step's wall time, against 8 TB/s."""
-    total = sum(slot_solve_bytes(L, int(k), vs) for L, k in zip(levels, iters))
+    total = sum(slot_solve_bytes(L, int(k)) for L, k in zip(levels, iters))
     gbs = total / seconds / 1e9
     return {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs / PEAK_GBS, 4), "bytes_per_step": int(total),
@@ -647,7 +624,7 @@ def level_launch_rates(B, levels, level, reps=20):
         # z (4) and p (8) read, the new p and q (8 each) written, 8 per cell
         nb = sum(8 * 4 ** L + 28 * (2 ** L + 1) ** 2 for L in levels)
         g = nb / (spmv * 1e-6) / 1e9
-        out["outer_spmv_dot"] = {"kernel": ("k_b_dir_spmv<weights from cells, float>: FP64 p = z + beta p, q = A p, "
+        out["outer_spmv_dot"] = {"kernel": ("k_b_dir_march / k_b_dir_spmv, weights from cells: FP64 p = z + beta p, q = A p, "
                                             "p.q, every slot"),
                                  "us": round(spmv, 2),
                                  "algorithmic_bytes": int(nb), "achieved_gbs": round(g, 1),
@@ -859,18 +836,21 @@ def batch_kernel_roofline(B, level):
                          "achieved_gbs": round(gbs, 1), "frac": round(gbs / PEAK_GBS, 4),
                          "bytes_rule": "slots*(nnz*4 + n*16) + nnz*4 + n*4: the column indices are shared by all "
                                        "slots",
-                         "note": "one pass per launch; levels from 33^2 up run the paired launches below"}}
+                         "note": "one pass per launch; levels from 129^2 up run the paired launches below"}}
     pre, post = B.pair_timing(level)   # the pool's weight source: the cell coefficients
-    pbytes = ns * (8 * (side - 1) ** 2 + n * 16)
-    for name, t, what in (("paired_pre", pre, "k_b_pair<float,PRE,weights from cells>: Jacobi0 then the defect"),
-                          ("paired_post", post, "k_b_pair<float,POST,weights from cells>: two Jacobi sweeps")):
+    nc = ((side - 1) // 2 + 1) ** 2
+    for name, t, nb, what, rule in (
+            ("paired_pre", pre, 8 * (side - 1) ** 2 + n * 12 + nc * 4, "Jacobi0, the defect and its restriction",
+             "slots*(8*cells + n*12 + nc*4): the cell coefficients once for all passes, rhs, dinv, the output, the "
+             "coarse right-hand side; no index or value stream"),
+            ("paired_post", post, 8 * (side - 1) ** 2 + n * 16, "two Jacobi sweeps",
+             "slots*(8*cells + n*16): the cell coefficients once for both passes, rhs, dinv, the input, the output; "
+             "no index or value stream")):
         if t > 0:
-            g = pbytes / (t * 1e-6) / 1e9
-            out[name] = {"kernel": f"{what}, level {level} ({side}^2)", "slots": ns, "us": round(t, 2),
-                         "algorithmic_bytes": int(pbytes), "achieved_gbs": round(g, 1),
-                         "frac": round(g / PEAK_GBS, 4),
-                         "bytes_rule": "slots*(8*cells + n*16): the cell coefficients once for both passes, rhs, "
-                                       "dinv, the input or first output, the output; no index or value stream"}
+            g = ns * nb / (t * 1e-6) / 1e9
+            out[name] = {"kernel": f"paired launch, weights from cells: {what}, level {level} ({side}^2)", "slots": ns,
+                         "us": round(t, 2), "algorithmic_bytes": int(ns * nb), "achieved_gbs": round(g, 1),
+                         "frac": round(g / PEAK_GBS, 4), "bytes_rule": rule}
     return out
 
 
