@@ -89,12 +89,12 @@ int reduce_to_host(double *out, void *stream, hipError_t (*launch)(double *, con
     // the result goes to pinned memory from the last kernel (a Jacobi step, a
     // defect and its norm at 33^2: 34.1 us with a copy launch and a finishing
     // launch of one partial, 23.1 without)
-    volatile double *v = w->take_return();
-    int st = check(launch((double *)v, w->slots, ctx), "reduction");
+    const ReturnSlot v(*w);
+    int st = check(launch(v.get(), w->slots, ctx), "reduction");
     if (st) return st;
     st = check(hipStreamSynchronize(S(stream)), "reduction sync");
     if (st) return st;
-    *out = *v;
+    *out = *(volatile double *)v.get();
     return HONEI_HIP_SUCCESS;
 }
 

@@ -77,6 +77,20 @@ void *Workspace::ensure_scratch(size_t bytes) {
     return scratch;
 }
 
+ReturnSlot::ReturnSlot(Workspace &w) : w_(w) {
+    std::unique_lock<std::mutex> lock(w.returns_mutex);
+    w.returned.wait(lock, [&] { return w.returns_free != 0; });
+    k_ = __builtin_ctzll(w.returns_free);
+    w.returns_free &= w.returns_free - 1;
+}
+ReturnSlot::~ReturnSlot() {
+    {
+        std::lock_guard<std::mutex> lock(w_.returns_mutex);
+        w_.returns_free |= uint64_t(1) << k_;
+    }
+    w_.returned.notify_one();
+}
+
 void release_workspaces() {
     std::lock_guard<std::mutex> lock(g_mutex);
     for (auto &kv : g_ws) {

@@ -3,7 +3,9 @@
 
 #include <hip/hip_runtime.h>
 
-#include <atomic>
+#include <condition_variable>
+#include <cstdint>
+#include <mutex>
 #include <string>
 
 #include "backend.hh"
@@ -21,17 +23,34 @@ struct Workspace {
     static constexpr int kScalars = 256;
     static constexpr int kSlotCapacity = 1 << 17;   // blocks
     static constexpr int kSlotLanes = 4;
-    // Results of reductions that return to the host: pinned, written by the
-    // reduction's last kernel itself.  A call takes the next of kReturns.
+    // Results of reductions that return to the host (ReturnSlot): pinned,
+    // written by the reduction's last kernel itself.
+    static constexpr int kReturns = 64;
     double *returns = nullptr;
-    std::atomic<uint32_t> next_return{0};
-    static constexpr uint32_t kReturns = 64;
-    double *take_return() { return returns + next_return.fetch_add(1, std::memory_order_relaxed) % kReturns; }
+    uint64_t returns_free = ~uint64_t(0);   // bit k: returns[k] has no owner
+    std::mutex returns_mutex;
+    std::condition_variable returned;
     void *scratch = nullptr;     // grows on demand, never shrinks
     size_t scratch_bytes = 0;
     // Returns a buffer of at least `bytes` (reallocating only when larger
     // than any earlier request), or nullptr on allocation failure.
     void *ensure_scratch(size_t bytes);
+};
+
+// One of a workspace's results, owned by a call from before its launches until
+// it has read the value; a call that finds none free waits for another's (an
+// owner waits for its launches only).
+class ReturnSlot {
+  public:
+    explicit ReturnSlot(Workspace &w);
+    ~ReturnSlot();
+    ReturnSlot(const ReturnSlot &) = delete;
+    ReturnSlot &operator=(const ReturnSlot &) = delete;
+    double *get() const { return w_.returns + k_; }
+
+  private:
+    Workspace &w_;
+    int k_;
 };
 
 // Returns nullptr (and records the error) when allocation fails.
