@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -78,6 +79,8 @@ int ell_call(ValueType vt, EllArgs a, const void *Aj, const void *Ax, const void
     if (!w) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
     a.block = (int)blocksize;
     EllView A = make_view(Aj, Ax, Arl, (size_t)a.row_end, ncpr, stride, threads, vt, index_words);
+    std::unique_lock<std::mutex> use(w->use, std::defer_lock);
+    if (a.norm2) use.lock();   // the only launches here with partials
     return check(ell_apply(A, a, w->slots, S(stream)), what);
 }
 
@@ -90,7 +93,11 @@ int reduce_to_host(double *out, void *stream, hipError_t (*launch)(double *, con
     // defect and its norm at 33^2: 34.1 us with a copy launch and a finishing
     // launch of one partial, 23.1 without)
     const ReturnSlot v(*w);
-    int st = check(launch(v.get(), w->slots, ctx), "reduction");
+    int st;
+    {
+        std::lock_guard<std::mutex> use(w->use);
+        st = check(launch(v.get(), w->slots, ctx), "reduction");
+    }
     if (st) return st;
     st = check(hipStreamSynchronize(S(stream)), "reduction sync");
     if (st) return st;
@@ -476,6 +483,7 @@ int honei_hip_narrow_indices(void *dst, const void *src, size_t n, uint64_t boun
     if (n > (size_t)INT64_MAX / 8) return fail(HONEI_HIP_ERROR_INVALID_ARGUMENT, "n too large");
     Workspace *w = workspace_for(S(stream));
     if (!w) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
+    std::lock_guard<std::mutex> use(w->use);
     const uint64_t lim = bound < (uint64_t(1) << 32) ? bound : (uint64_t(1) << 32);
     unsigned int *bad = (unsigned int *)(w->scalars + Workspace::kScalars - 1);
     int st = check(fill_bytes_zero(bad, sizeof(unsigned int), S(stream)), "narrow_indices clear");
@@ -638,6 +646,7 @@ int honei_hip_dot_product_dev(int vt, double *out, const void *x, const void *y,
     if (!out || (n && (!x || !y))) return fail(HONEI_HIP_ERROR_INVALID_ARGUMENT, "null pointer");
     Workspace *w = workspace_for(S(stream));
     if (!w) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
+    std::lock_guard<std::mutex> use(w->use);
     return check(dot(x, y, (int64_t)n, (ValueType)vt, out, w->slots, S(stream)), "dot");
 }
 int honei_hip_norm_l2_dev(int vt, double *out, const void *x, size_t n, void *stream) {
@@ -645,6 +654,7 @@ int honei_hip_norm_l2_dev(int vt, double *out, const void *x, size_t n, void *st
     if (!out || (n && !x)) return fail(HONEI_HIP_ERROR_INVALID_ARGUMENT, "null pointer");
     Workspace *w = workspace_for(S(stream));
     if (!w) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
+    std::lock_guard<std::mutex> use(w->use);
     return check(norm2(x, (int64_t)n, (ValueType)vt, out, w->slots, S(stream)), "norm");
 }
 int honei_hip_axpy_norm_dev(int vt, void *x, const void *y, double alpha, double *out, size_t n, void *stream) {
@@ -652,6 +662,7 @@ int honei_hip_axpy_norm_dev(int vt, void *x, const void *y, double alpha, double
     if (!out || (n && (!x || !y))) return fail(HONEI_HIP_ERROR_INVALID_ARGUMENT, "null pointer");
     Workspace *w = workspace_for(S(stream));
     if (!w) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
+    std::lock_guard<std::mutex> use(w->use);
     return check(axpy_norm2(x, y, alpha, nullptr, (int64_t)n, (ValueType)vt, out, w->slots, S(stream)), "axpy_norm");
 }
 

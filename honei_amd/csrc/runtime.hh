@@ -18,6 +18,10 @@ namespace hipx {
 // on first use with hipMalloc, kept until honei_hip_shutdown(); no per-call
 // allocation on any path.
 struct Workspace {
+    // Held by a call while it enqueues launches that use the slots or scalars
+    // (another thread's on the same stream then follow all of them), and by a
+    // solve, which also reads back between them, until it returns.
+    std::mutex use;
     ReduceSlots slots;
     double *scalars = nullptr;   // kScalars doubles
     static constexpr int kScalars = 256;

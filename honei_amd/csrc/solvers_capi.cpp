@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -178,6 +179,7 @@ int honei_hip_cg_solve(int vtype, const void *Aj, const void *Ax, const void *Ar
     if (st) return st;
     Workspace *w = workspace_for(S(stream));
     if (!w) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
+    std::lock_guard<std::mutex> use(w->use);
     const size_t vbytes = cg_vector_bytes((ValueType)vtype, rows);
     const EllView A = cg_view(vtype, Aj, Ax, Arl, rows, num_cols_per_row, stride, threads);
     const bool fits = cg_resident_fits(A);
@@ -201,6 +203,7 @@ int honei_hip_pcg_jacobi(int vtype, const void *Aj, const void *Ax, const void *
     if (max_iters > 0x7fffffff) max_iters = 0x7fffffff;
     Workspace *w = workspace_for(S(stream));
     if (!w) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
+    std::lock_guard<std::mutex> use(w->use);
     const ValueType vt = (ValueType)vtype;
     const size_t es = vec_size(vt);
     const size_t vbytes = ((rows * es + 255) / 256) * 256;
@@ -255,6 +258,7 @@ int honei_hip_cg_konv(int vtype, const void *Aj, const void *Ax, const void *Arl
     if (max_iters > 0x7fffffff) max_iters = 0x7fffffff;
     Workspace *w = workspace_for(S(stream));
     if (!w) return HONEI_HIP_ERROR_OUT_OF_MEMORY;
+    std::lock_guard<std::mutex> use(w->use);
     const size_t es = vec_size((ValueType)vtype);
     const size_t vbytes = ((rows * es + 255) / 256) * 256;
     char *base = (char *)w->ensure_scratch(3 * vbytes + 256);

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import honei_amd as H
+import oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -71,9 +72,10 @@ def test_more_waiting_calls_than_kept_results():
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("kind", ["dot", "norm"])
-@pytest.mark.parametrize("n", [1, 2048])
+@pytest.mark.parametrize("n", [1, 2048, 2049, 100003])
 def test_sums_that_return(n, kind, dtype):
-    """Sums of one work-group; the results of the same calls one after another."""
+    """One work-group's sum and sums over partials; the results of the same
+    calls one after another."""
     rng = np.random.default_rng(n)
     arrays = [H.DeviceArray.from_host(rng.standard_normal(n).astype(dtype)) for _ in range(6)]
     want = [_reduce(kind, a, arrays[0]) for a in arrays]
@@ -87,3 +89,74 @@ def test_sums_that_return(n, kind, dtype):
 
     assert not _run(6, work)
     assert not bad, (len(bad), bad[:4], want)
+
+
+def test_sums_left_on_the_device():
+    """The same for sums that stay on the device, a defect's norm among them."""
+    n, side, rounds = 60001, 257, 60
+    rng = np.random.default_rng(5)
+    xs = [H.DeviceArray.from_host(rng.standard_normal(n)) for _ in range(2)]
+    D = H.DeviceEll.from_oracle(oracle.q1_matrix(side))
+    x, b, r = (H.DeviceArray.from_host(rng.standard_normal(side * side)) for _ in range(3))
+
+    def call(k, out, j):
+        at = H._p(out.ptr + 8 * j)
+        if k == 0:
+            H.call("honei_hip_dot_product_dev", H.F64, at, xs[0].ptr, xs[1].ptr, n, None)
+        elif k == 1:
+            H.call("honei_hip_norm_l2_dev", H.F64, at, xs[1].ptr, n, None)
+        else:
+            H.call("honei_hip_defect_norm_smell_dv", D.vtype, b.ptr, r.ptr, D.Aj.ptr, D.Ax.ptr, D.Arl.ptr, x.ptr, D.rows,
+                   D.ncpr, D.stride, D.threads, at, None)
+
+    outs = [H.DeviceArray(rounds + 1, np.float64) for _ in range(3)]
+    for k in range(3):
+        call(k, outs[k], rounds)
+
+    def work(k):
+        for j in range(rounds):
+            call(k, outs[k], j)
+
+    assert not _run(3, work)
+    H.call("honei_hip_synchronize", None)
+    for k in range(3):
+        got = outs[k].get()
+        assert (got == got[rounds]).all(), k
+
+
+def test_solves_and_sums():
+    """CG and PCG-Jacobi solves (of more and more rows: the scratch grows), and
+    sums beside them: the results of the same calls one after another."""
+    n, sides = 50021, [33, 65, 129, 257]
+    rng = np.random.default_rng(9)
+    x = H.DeviceArray.from_host(rng.standard_normal(n))
+    systems = []
+    for side in sides:
+        b = rng.standard_normal((side, side))
+        b[0] = b[-1] = b[:, 0] = b[:, -1] = 0
+        systems.append((H.DeviceEll.from_oracle(oracle.q1_matrix(side)), H.DeviceArray.from_host(b.ravel()),
+                        H.DeviceArray.from_host(np.full(side * side, 0.375))))
+
+    def solve(pcg, i):
+        D, b, dinv = systems[i]
+        u = H.DeviceArray.from_host(np.zeros(b.n))
+        r = (H.pcg_jacobi(D, b, u, dinv, 400, 1e-9, check=False) if pcg else
+             H.cg_solve(D, b, u, 400, 1e-9, check=False))
+        return r, u.get().tobytes()
+
+    sums = _reduce("dot", x, x)
+    want = {(pcg, i): solve(pcg, i) for pcg in (0, 1) for i in range(len(sides))}
+    bad = []
+
+    def work(k):
+        if k < 3:
+            for i in range(len(sides)):
+                if solve(k % 2, i) != want[k % 2, i]:
+                    bad.append((k, i))
+        else:
+            for j in range(200):
+                if _reduce("dot", x, x) != sums:
+                    bad.append((k, j))
+
+    assert not _run(5, work)
+    assert not bad, bad[:5]
