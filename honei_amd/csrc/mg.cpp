@@ -362,7 +362,8 @@ hipError_t MGHierarchy::run_kernel(hipStream_t s, int64_t *inner_iters, double *
     const bool lean = mixed_inner_ && !cfg.convergence_check;
     const bool q1 = q1_cycle();
     const bool need_initial = !(lean && cfg.n_max_iter == 1);
-    // d[max] = rhs when the start vector is zero (no matvec), else rhs - A x
+    // d[max] = rhs when the start vector is zero (no matvec), else rhs - A x;
+    // from the second cycle on the defect that the cycle before ends with
     const void *top_d = top.d;
     if (cfg.initial_zero) {
         top_d = top.rhs;
@@ -381,6 +382,7 @@ hipError_t MGHierarchy::run_kernel(hipStream_t s, int64_t *inner_iters, double *
         for (iter = 1; iter <= cfg.n_max_iter; ++iter) {
             const bool skip_final = lean && iter == cfg.n_max_iter;
             int64_t l = maxl;
+            if (iter > 1) top_d = top.d;
             if (q1 && maxl > coarse_top(inner)) {
                 // the top level's down-leg on x, the rest as one-slot launches
                 HX(smooth_from_zero(maxl, top_d, top.c, top.x, s));
