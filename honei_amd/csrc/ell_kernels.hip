@@ -18,6 +18,7 @@
 
 #include "backend.hh"
 #include "ell_device.hh"
+#include "row_slot.hh"
 
 #pragma clang fp contract(off)
 
@@ -305,10 +306,10 @@ constexpr int kRowsBlock = 512;
 constexpr int kRowsWindow = 9216;   // entries of x: 36 KiB, four work-groups a CU
 constexpr int64_t kRowsMin = 98304;
 
-template <int NC>
+// Stored widths LEAST .. NC.
+template <int LEAST, int NC>
 __global__ __launch_bounds__(kRowsBlock, 6) void k_product_rows(KArgs a) {
     constexpr int P = 8, U = 8;   // entries looked at first; entries a step
-    constexpr uint32_t kOutside = 0x80000000u;
     __shared__ float win[kRowsWindow];
     __shared__ int32_t red[4][kRowsBlock / kWave];
     const float *__restrict__ x = (const float *)a.x;
@@ -318,11 +319,12 @@ __global__ __launch_bounds__(kRowsBlock, 6) void k_product_rows(KArgs a) {
     const uint32_t oj = (uint32_t)row * 4u, stride = (uint32_t)a.stride;
     int32_t j[NC];
     auto index = [&](int k) {
-        j[k] = BufLoad<int32_t>::template load<kBufNT>(rAj, (uint32_t)k < len ? oj : kOutside, (uint32_t)k * stride * 4u);
+        const RowSlot e = row_slot((uint32_t)row, (uint32_t)k, len, stride, a.aj_bytes, LEAST);
+        j[k] = BufLoad<int32_t>::template load<kBufNT>(rAj, e.lane, e.wave);
     };
     auto value = [&](int k) {
-        return BufLoad<float>::template load<kBufNT>(rAx, (uint32_t)k < len ? oj : kOutside,
-                                                  (uint32_t)k * stride * 4u);
+        const RowSlot e = row_slot((uint32_t)row, (uint32_t)k, len, stride, a.ax_bytes, LEAST);
+        return BufLoad<float>::template load<kBufNT>(rAx, e.lane, e.wave);
     };
 #pragma unroll
     for (int k = 0; k < P; ++k) index(k);
@@ -534,7 +536,7 @@ hipError_t ell_apply(const EllView &A, const EllArgs &e, const ReduceSlots &slot
     k.ax_bytes = (uint32_t)(slots_total * vsz);
     if (e.mode == ELL_PRODUCT && A.vtype == VT_F32 && T == 1 && iw == 1 && !e.gate && e.block <= 0 && A.ncpr > 16 &&
         A.ncpr <= 28 && nrows >= kRowsMin && slots_total * 4 < (int64_t(1) << 31)) {
-        fn = A.ncpr <= 24 ? k_product_rows<24> : k_product_rows<28>;
+        fn = A.ncpr <= 24 ? k_product_rows<17, 24> : k_product_rows<25, 28>;
         hipLaunchKernelGGL(fn, dim3((unsigned)((nrows + kRowsBlock - 1) / kRowsBlock)), dim3(kRowsBlock), 0, s, k);
         return hipGetLastError();
     }
