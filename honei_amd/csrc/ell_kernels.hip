@@ -331,7 +331,7 @@ __global__ __launch_bounds__(kRowsBlock, 6) void k_product_rows(KArgs a) {
     // scattered: most entries of neighbouring rows (four of a row looked at)
     // lie further apart than a cache line of 32 entries
     const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
-    const uint32_t wlen = lane ? (uint32_t)__shfl_up((int)len, 1) : 0u;
+    const uint32_t before = (uint32_t)__shfl_up((int)len, 1), wlen = lane ? before : 0u;
     int far = 0, pairs = 0;
 #pragma unroll
     for (int k = 0; k < P; k += 2) {

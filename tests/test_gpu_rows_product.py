@@ -67,3 +67,17 @@ def test_product(width, n, pattern):
         part = H.DeviceArray(last - first, np.float32)
         D.product(part, dx, row_start=first, row_end=last)
         assert np.array_equal(part.get(), want[first:last], equal_nan=True)
+
+
+@pytest.mark.parametrize("pattern", [700, "everywhere", "band"])
+def test_first_two_rows_of_a_wavefront(pattern):
+    """Only lanes 0 and 1 have entries: what the work-group decides on is the
+    one pair of neighbouring rows a wavefront has."""
+    n, width = MIN_ROWS + 64, 27
+    A, x = _matrix(n, n + 3, width, pattern)
+    length = A.Arl.copy()
+    length[np.arange(n) % 64 > 1] = 0
+    A = oracle.Ell(n, n + 3, A.stride, width, 1, A.Aj, A.Ax, length)
+    dx, dy = H.DeviceArray.from_host(x), H.DeviceArray(n, np.float32)
+    H.DeviceEll.from_oracle(A).product(dy, dx)
+    assert np.array_equal(dy.get(), oracle.product(A, x), equal_nan=True)
