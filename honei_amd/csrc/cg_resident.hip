@@ -30,11 +30,17 @@
 // its grid-stride elements and block_sum, sum_partials' tree), so x, the
 // iteration count and the defect do not depend on the path.
 //
-// Waits are bounded: a work-group that sees no progress for kWaitTicks sets
-// sc->aborted and leaves; x is written to scratch and copied to the caller's
-// vector only when no work-group did, so the caller can run the launches
-// instead.  A lease bounds the work-groups of all such launches on a device
-// by its compute units, so concurrent solves cannot keep each other out.
+// Waits are bounded: a work-group that sees no progress for too long sets
+// sc->aborted and leaves, the others follow; x is written to scratch and
+// copied to the caller's vector only when no work-group did, so the caller can
+// run the launches instead.  A lease bounds the work-groups of all such
+// launches of a process on a device by its compute units, so its own solves
+// cannot keep each other out.  Other processes' can: each then holds part of
+// the chip and waits for the rest of its own.  So the first exchange of a
+// launch, after which every work-group is known to be on the chip, waits
+// kArriveTicks only.  Four processes with twelve solves each on 522,729 rows
+// (5.5 ms a solve alone): 0.3 to 0.4 s, launches only 0.4 to 0.5; the long wait there
+// too: 5.4 s.
 
 #include <atomic>
 
@@ -55,7 +61,9 @@ constexpr int kGroupChunks = 8;        // chunks of one update partial (2048 row
 constexpr int kWidth = 9;              // stored entries per row at most
 constexpr int64_t kMaxChunks = 2048;   // partials two rounds of 1024 threads sum
 constexpr int64_t kFourRows = 65536, kTwoRows = 262144;   // four / two work-groups per group up to here
-constexpr uint64_t kWaitTicks = 100000000ull;   // wall_clock64 ticks (100 MHz): 1 s
+// wall_clock64 ticks (100 MHz): 2 ms for the work-groups of a launch to arrive
+// (some 50 us where nothing is in their way), 1 s for any other wait
+constexpr uint64_t kArriveTicks = 200000ull, kWaitTicks = 100000000ull;
 
 // What crosses work-groups is empty (a signalling NaN, which no addition or
 // product returns; results that are NaN travel as quiet ones) until its owner
@@ -99,16 +107,17 @@ __device__ inline void agent_store_bits(V *base, uint32_t byte_off, typename Emp
 __device__ inline void post(uint64_t *w, double v) { agent_store(w, __builtin_bit_cast(uint64_t, v)); }
 
 // t0: 0 at the first call of a wait
-__device__ inline bool in_time(uint64_t &t0) {
+__device__ inline bool in_time(uint64_t &t0, uint64_t ticks) {
     const uint64_t now = wall_clock64();
     if (t0 == 0) t0 = now;
-    return now - t0 <= kWaitTicks;
+    return now - t0 <= ticks;
 }
 
 // The N words w[0], w[step], ... once all are posted; false when the wait
 // runs out.  Neighbouring lanes read neighbouring words: a poll of a
 // wavefront is N requests of 512 bytes.
-template <int N> __device__ inline bool take(const uint64_t *w, int step, double (&v)[N]) {
+template <int N>
+__device__ inline bool take(const uint64_t *w, int step, double (&v)[N], uint64_t ticks) {
     uint64_t t0 = 0, q[N];
     for (uint32_t spin = 0;; ++spin) {
         bool all = true;
@@ -117,7 +126,7 @@ template <int N> __device__ inline bool take(const uint64_t *w, int step, double
 #pragma unroll
         for (int i = 0; i < N; ++i) all = all && q[i] != kEmpty;
         if (all) break;
-        if ((spin & 255u) == 255u && !in_time(t0)) return false;
+        if ((spin & 255u) == 255u && !in_time(t0, ticks)) return false;
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) v[i] = __builtin_bit_cast(double, q[i]);
@@ -164,7 +173,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_resident(EllView A, const typen
                                                           typename VecOf<VT>::type *pub0,
                                                           typename VecOf<VT>::type *pub1, CGScalars *sc,
                                                           uint64_t *words, int nchunks, int g2, int it_begin,
-                                                          int it_end) {
+                                                          int it_end, uint64_t arrive) {
     typedef typename VecOf<VT>::type V;
     typedef typename EmptyOf<V>::Bits Bits;
     constexpr int Q = 4 / R, NRED = PCG ? 2 : 1;
@@ -173,7 +182,8 @@ __global__ __launch_bounds__(kThreads) void k_cg_resident(EllView A, const typen
     __shared__ double red_a[16], red_b[NRED][16], sq[NRED][kGroupChunks][64 * R], wsum[kGroupChunks][R],
         bsum[NRED][R];
     __shared__ int bad;
-    if (sc->done || sc->aborted) return;
+    // another work-group may set aborted meanwhile: read it once
+    if (sc->done || block_uniform_flag(&sc->aborted)) return;
     const int tid = threadIdx.x, lane = tid % kWave, w = tid / kWave;
     const int b = blockIdx.x / Q, h = blockIdx.x % Q;
     const VT *Ax = (const VT *)A.Ax;
@@ -223,7 +233,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_resident(EllView A, const typen
     const V initial = (V)sc->initial, eps_rel = (V)sc->eps_rel;
     const int max_iters = sc->max_iters;
     V alpha = (V)sc->alpha, factor = V(0), current = V(0);   // alpha: |r|^2 (CG), r.z (PCG)
-    bool stop = false, conv = false, ok = true;
+    bool stop = false, conv = false, ok = arrive != 0;   // 0: give up at the first wait
     int it = it_begin;
     __syncthreads();
     while (true) {
@@ -257,7 +267,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_resident(EllView A, const typen
                 double q[Q];
 #pragma unroll
                 for (int u = 0; u < Q; ++u) q[u] = 0.0;
-                if (ok) ok = take(word_a(it, 0) + i, nchunks, q);
+                if (ok) ok = take(word_a(it, 0) + i, nchunks, q, it == it_begin ? arrive : kWaitTicks);
                 acc += combine(q);
             }
             acc = wave_sum(acc);
@@ -357,7 +367,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_resident(EllView A, const typen
 #pragma unroll
                     for (int i = 0; i < NRED * Q; ++i) need = need || q[i] == kEmpty;
                 }
-                if ((spin & 255u) == 255u) ok = in_time(t0);
+                if ((spin & 255u) == 255u) ok = in_time(t0, kWaitTicks) && !agent_load(&sc->aborted);
             }
             if (w * kWave < g2) {
 #pragma unroll
@@ -454,12 +464,13 @@ __global__ __launch_bounds__(256) void k_empty_words(uint64_t *w, int n) {
 
 template <typename VT, bool PCG>
 hipError_t launch(const EllView &A, const void *dinv, const void *xin, void *x, void *xs, void *p, void *r, void *pub0,
-                  void *pub1, CGScalars *sc, uint64_t *words, int it_begin, int it_end, hipStream_t s) {
+                  void *pub1, CGScalars *sc, uint64_t *words, int it_begin, int it_end, uint64_t arrive, hipStream_t s) {
     typedef typename VecOf<VT>::type V;
     const int nchunks = (int)((A.rows + kChunk - 1) / kChunk), g2 = groups(A.rows);
 #define RUN(R)                                                                                                  \
     hipLaunchKernelGGL((k_cg_resident<VT, PCG, R>), dim3(g2 * (4 / R)), dim3(kThreads), 0, s, A, (const V *)dinv, \
-                       (const V *)xin, (V *)xs, (V *)p, (V *)r, (V *)pub0, (V *)pub1, sc, words, nchunks, g2, it_begin, it_end)
+                       (const V *)xin, (V *)xs, (V *)p, (V *)r, (V *)pub0, (V *)pub1, sc, words, nchunks, g2, it_begin, it_end, \
+                       arrive)
     switch (split(A.rows)) {
         case 4: RUN(1); break;
         case 2: RUN(2); break;
@@ -500,13 +511,14 @@ ResidentLease::~ResidentLease() {
 
 hipError_t cg_resident(const EllView &A, const void *dinv, const void *xin, void *x, void *xs, void *p, void *r,
                        void *pub0, void *pub1, CGScalars *sc, const ReduceSlots &sl, int it_begin, int it_end,
-                       hipStream_t s) {
+                       bool give_up, hipStream_t s) {
+    const uint64_t arrive = give_up ? 0 : kArriveTicks;
     uint64_t *words = (uint64_t *)sl.partials;
     if (it_begin == 0)
         hipLaunchKernelGGL(k_empty_words, dim3((kWords + 255) / 256), dim3(256), 0, s, words, (int)kWords);
 #define RES(VT)                                                                                              \
-    return dinv ? launch<VT, true>(A, dinv, xin, x, xs, p, r, pub0, pub1, sc, words, it_begin, it_end, s)             \
-                : launch<VT, false>(A, dinv, xin, x, xs, p, r, pub0, pub1, sc, words, it_begin, it_end, s)
+    return dinv ? launch<VT, true>(A, dinv, xin, x, xs, p, r, pub0, pub1, sc, words, it_begin, it_end, arrive, s)             \
+                : launch<VT, false>(A, dinv, xin, x, xs, p, r, pub0, pub1, sc, words, it_begin, it_end, arrive, s)
     switch (A.vtype) {
         case VT_F32: RES(float);
         case VT_F64: RES(double);

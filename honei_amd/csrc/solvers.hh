@@ -135,7 +135,8 @@ hipError_t pcg_iteration(const EllView &A, void *x, void *d, void *r, void *t0, 
 // first iteration above expects in p, r and sc; xin is x (first launch) or
 // xs, pub0 and pub1 vectors of scratch.  x receives the result once the
 // solve is over.  sc->aborted set: x is untouched and the launches above have
-// to run, from the start.  Same bits as cg_iteration / pcg_iteration.
+// to run, from the start; give_up: every work-group does so at its first wait.
+// Same bits as cg_iteration / pcg_iteration.
 // The lease (held while its launches run) says whether A fits and bounds the
 // resident work-groups per device; without one the launches above run.
 constexpr int kResidentIters = 4096;   // iterations per launch at most
@@ -153,7 +154,7 @@ class ResidentLease {
 };
 hipError_t cg_resident(const EllView &A, const void *dinv, const void *xin, void *x, void *xs, void *p, void *r,
                        void *pub0, void *pub1, CGScalars *sc, const ReduceSlots &sl, int it_begin, int it_end,
-                       hipStream_t s);
+                       bool give_up, hipStream_t s);
 hipError_t coarse_cg(const EllView &A, const void *rhs, void *x, void *g, void *u, void *en, double konv,
                      int max_iters, int *iters_dev, hipStream_t s);
 hipError_t boundary_guess(double *guess, const double *b, int64_t n, int64_t side, hipStream_t s);

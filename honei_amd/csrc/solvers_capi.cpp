@@ -56,6 +56,10 @@ int upload_ell(DevEll &M, ValueType vt, size_t rows, size_t cols, size_t stride,
     return check(hipMemcpy(M.Ax, Ax, size * vt_size(vt), hipMemcpyHostToDevice), "ELL value upload");
 }
 
+// The resident launch (0: the first) in which the calling thread's solves give
+// up; negative: none (honei_hip_resident_give_up)
+thread_local int32_t t_give_up = -1;
+
 // The iteration loop of CG and PCG-Jacobi: resident launches where the
 // system fits and the device has room for them, else (or when one gave up
 // waiting) single iterations enqueued in chunks with one flag read per chunk.
@@ -73,7 +77,8 @@ int run_iterations(const EllView &A, bool may_stay, const ReduceSlots &slots, CG
         if (lease) {
             for (size_t it = 0; it < max_iters; it += kResidentIters) {
                 const size_t end = std::min(max_iters, it + (size_t)kResidentIters);
-                if (int st = resident((int)it, (int)end)) return st;
+                const bool give_up = t_give_up >= 0 && it / kResidentIters == (size_t)t_give_up;
+                if (int st = resident((int)it, (int)end, give_up)) return st;
                 if (int st = read_back()) return st;
                 if (h.done || h.aborted) break;
             }
@@ -151,9 +156,9 @@ int cg_solve_on(const EllView &A, const void *b, void *x, size_t max_iters, doub
     auto iterate = [&](int it) {
         return check(cg_iteration(A, x, p, r, v, sc, slots, it, s), "cg iteration");
     };
-    auto resident = [&](int begin, int end) {
+    auto resident = [&](int begin, int end, bool give_up) {
         return check(cg_resident(A, nullptr, begin ? v : x, x, v, p, r, pub, (char *)pub + cg_vector_bytes(A.vtype, rows),
-                                 sc, slots, begin, end, s),
+                                 sc, slots, begin, end, give_up, s),
                      "cg resident");
     };
     if (int st = run_iterations(A, pub != nullptr, slots, sc, max_iters, s, start, iterate, resident, h)) return st;
@@ -189,6 +194,11 @@ int honei_hip_cg_solve(int vtype, const void *Aj, const void *Ax, const void *Ar
     return cg_solve_on(A, b, x, max_iters, eps_relative, used_iters, final_defect, S(stream), w->slots, base,
                        base + vbytes, base + 2 * vbytes, fits ? base + 3 * vbytes : nullptr,
                        (CGScalars *)(base + vectors * vbytes));
+}
+
+int honei_hip_resident_give_up(int32_t launch) {
+    t_give_up = launch;
+    return HONEI_HIP_SUCCESS;
 }
 
 int honei_hip_pcg_jacobi(int vtype, const void *Aj, const void *Ax, const void *Arl, size_t rows,
@@ -235,9 +245,9 @@ int honei_hip_pcg_jacobi(int vtype, const void *Aj, const void *Ax, const void *
     auto iterate = [&](int it) {
         return check(pcg_iteration(A, x, d, r, t0, dd_inverted, sc, w->slots, it, s), "pcg iteration");
     };
-    auto resident = [&](int begin, int end) {
+    auto resident = [&](int begin, int end, bool give_up) {
         return check(cg_resident(A, dd_inverted, begin ? t0 : x, x, t0, d, r, pub, pub + vbytes, sc, w->slots, begin,
-                                 end, s),
+                                 end, give_up, s),
                      "pcg resident");
     };
     if (int st = run_iterations(A, fits, w->slots, sc, max_iters, s, start, iterate, resident, h)) return st;

@@ -351,6 +351,14 @@ int honei_hip_pcg_jacobi(int vtype, const void *Aj, const void *Ax, const void *
                          const void *dd_inverted_dev, size_t max_iters, double eps_relative, size_t *used_iters,
                          double *final_defect, void *stream);
 
+/* For tests of what CG and PCG-Jacobi solves do when their resident launches
+ * cannot have the chip to themselves (systems of up to 524,288 rows; other
+ * processes' work may keep part of their work-groups off it): the calling
+ * thread's solves behave so in resident launch number `launch` (0: the first;
+ * 4096 iterations each) and go on launch by launch, with the same results.
+ * Negative (the default): only when it happens.                            */
+int honei_hip_resident_give_up(int32_t launch);
+
 /* ConjugateGradients<Tag, methods::NONE>::value(A, b, x, konv_rad)
  * (math/conjugate_gradients.hh:154-201, 587-623), the multigrid coarse
  * solver: x = 0, iterate until ||x||^2 grows by no more than konv_rad.

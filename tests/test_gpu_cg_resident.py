@@ -135,3 +135,18 @@ def test_threads_and_streams():
     assert not errors, errors
     for (x1, u1, f1), (x2, u2, f2) in zip(want, got):
         assert u1 == u2 and f1 == f2 and np.array_equal(x1.view(np.uint8), x2.view(np.uint8))
+
+
+@pytest.mark.parametrize("launch,max_iters,eps", [(0, 300, 1e-9), (1, 4500, 0.0)])
+@pytest.mark.parametrize("pcg", [False, True])
+@pytest.mark.parametrize("side,vtype", [(33, H.F64), (129, H.F32), (259, H.F64), (515, H.BF16)])
+def test_given_up(side, vtype, pcg, launch, max_iters, eps):
+    """A resident launch whose work-groups give up waiting -- the first, or one
+    that continues from another's state -- leaves the launch-by-launch result.
+    Sides: four, two and one work-groups per group of rows."""
+    H.call("honei_hip_resident_give_up", launch)
+    try:
+        used = _same(_grid(side), vtype, pcg, eps, max_iters)
+    finally:
+        H.call("honei_hip_resident_give_up", -1)
+    assert launch == 0 or used == max_iters
