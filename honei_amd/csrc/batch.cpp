@@ -145,7 +145,11 @@ hipError_t BatchMG::tune_level(BLevel &lv) {
     hipError_t err = hipSuccess;
     const size_t vs = vt_size(vt), es = inner_vector_bytes();
     for (int T : {1, 2, 4}) {
-        if (T > 1 && lv.level <= kMaxCoarseTop) break;   // the coarse launch sums rows as T = 1
+        // the coarse launch sums rows as T = 1; so do the levels it can take when
+        // they run level by level (fused_levels 0 and 1), for the same results.
+        // Where these were tuned too, T = 4 was chosen for some 9^2 levels and
+        // gained nothing: 512 FP32 systems of 33^2 and 17^2 4.66 ms, now 4.52
+        if (T > 1 && lv.level <= coarse_top(vt)) break;
         const Level0 g = level_geometry(lv.level, T, 256);
         void *Aj = nullptr, *Arl = nullptr, *Ax = nullptr, *vec = nullptr, *scd = nullptr, *lst = nullptr;
         const size_t vbytes = (size_t)(ns * g.vld) * es;
