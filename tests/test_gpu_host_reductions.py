@@ -69,3 +69,18 @@ def test_threads():
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("partials", [1, 1024, 1025, 4096, 4097, 8193])
+def test_sums_of_partials(partials):
+    """A defect's norm from one partial per 256 rows, on both sides of the rule
+    for loading them one by one or eight at a time: integers, so exact."""
+    n = 256 * (partials - 1) + 17
+    stride = 32 * ((n + 31) // 32)
+    b = np.random.default_rng(partials).integers(-8, 9, n).astype(np.float64)
+    D = H.DeviceEll(n, n, stride, 1, 1, np.zeros(stride, np.uint64), np.zeros(stride), np.zeros(n, np.uint64), H.F64)
+    db, x, r, out = (H.DeviceArray.from_host(b), H.DeviceArray.from_host(b), H.DeviceArray(n, np.float64),
+                     H.DeviceArray(1, np.float64))
+    D.defect_norm(r, db, x, out)
+    assert out.get()[0] == (b * b).sum()
+    assert np.array_equal(r.get(), b)
