@@ -492,6 +492,13 @@ bool cg_resident_fits(const EllView &A) {
            A.rows <= kMaxChunks * kChunk;
 }
 
+// Iterations from which a resident launch pays for bringing the rows in: up to
+// one (two / three) launch by launch against resident, us a call, FP64: 65^2
+// rows 66 / 69 (82 / 72), 385^2 75 / 80 (97 / 85), 513^2 79 / 95 (104 / 106),
+// 720^2 92 / 100 (128 / 114); bf16: 513^2 72 / 98 (94 / 108; 115 / 118), 720^2
+// 76 / 105 (102 / 116; 128 / 127).
+size_t cg_resident_from(const EllView &A) { return A.rows > kTwoRows && A.vtype != VT_F64 ? 3 : 2; }
+
 ResidentLease::ResidentLease(const EllView &A, const ReduceSlots &slots) {
     if (!cg_resident_fits(A) || (int64_t)slots.capacity * 4 < kWords) return;
     int dev = 0, cus = 0;

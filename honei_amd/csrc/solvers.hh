@@ -140,7 +140,8 @@ hipError_t pcg_iteration(const EllView &A, void *x, void *d, void *r, void *t0, 
 // The lease (held while its launches run) says whether A fits and bounds the
 // resident work-groups per device; without one the launches above run.
 constexpr int kResidentIters = 4096;   // iterations per launch at most
-bool cg_resident_fits(const EllView &A);   // by layout and size
+bool cg_resident_fits(const EllView &A);     // by layout and size
+size_t cg_resident_from(const EllView &A);   // fewest iterations a caller may allow
 class ResidentLease {
   public:
     ResidentLease(const EllView &A, const ReduceSlots &slots);

@@ -72,7 +72,7 @@ int run_iterations(const EllView &A, bool may_stay, const ReduceSlots &slots, CG
         return check(hipStreamSynchronize(s), "cg sync");
     };
     if (int st = start()) return st;
-    if (may_stay && max_iters > 0) {
+    if (may_stay && max_iters >= cg_resident_from(A)) {
         const ResidentLease lease(A, slots);
         if (lease) {
             for (size_t it = 0; it < max_iters; it += kResidentIters) {

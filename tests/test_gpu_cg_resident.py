@@ -150,3 +150,11 @@ def test_given_up(side, vtype, pcg, launch, max_iters, eps):
     finally:
         H.call("honei_hip_resident_give_up", -1)
     assert launch == 0 or used == max_iters
+
+
+@pytest.mark.parametrize("max_iters", [1, 2, 3])
+@pytest.mark.parametrize("pcg", [False, True])
+@pytest.mark.parametrize("side,vtype", [(65, H.F32), (515, H.F64), (515, H.F32)])
+def test_few_iterations(side, vtype, pcg, max_iters):
+    """On both sides of the iteration count from which solves stay resident."""
+    assert _same(_grid(side), vtype, pcg, 1e-9, max_iters) == max_iters
