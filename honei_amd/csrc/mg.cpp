@@ -160,9 +160,7 @@ hipError_t MGHierarchy::build_q1_coeff(double omega, const double *coeff, int av
     for (int64_t l = max_level; l >= min_level && err == hipSuccess; --l) {
         const int64_t cells = (1ll << l);
         double *&k = L[(size_t)l].kappa;
-        if (k) (void)hipFree(k);
-        k = nullptr;
-        err = hipMalloc((void **)&k, sizeof(double) * (size_t)(cells * cells));
+        if (!k) err = hipMalloc((void **)&k, sizeof(double) * (size_t)(cells * cells));   // a level's size is fixed
         if (err != hipSuccess) break;
         if (l == max_level)
             err = vcopy(k, coeff, cells * cells, VT_F64, s);

@@ -114,3 +114,29 @@ def test_degenerate_right_hand_sides(b):
         dx.zero()
         iters, rd = mg.solve_pcg(H.DeviceArray.from_host(rhs), dx, check=False)
         assert iters == 0 and rd == 0.0, (stored, iters, rd)
+
+
+def test_rebuilt_with_other_coefficients():
+    """A handle built again, with other coefficients or none in between, solves
+    as a fresh one."""
+    level, side = 7, 129
+    b = H.DeviceArray.from_host(uniform_pm1(5, side * side))
+    kappas = [H.DeviceArray.from_host(lognormal_cells(s, (side - 1) ** 2), np.float64) for s in (11, 12)]
+
+    def solve(builds):
+        mg = H.Multigrid(H.F32, 1, level)
+        mg.configure(H.mg_config(tolerance=1e-9, max_outer=60))
+        for k in builds:
+            if k is None:
+                mg.build_q1(0.7)
+            else:
+                mg.build_q1_coeff(kappas[k], 0.8, 1)
+            x = H.DeviceArray(side * side, np.float64)
+            x.zero()
+            r = mg.solve_pcg(b, x, check=False)
+        return r, x.get().tobytes()
+
+    for last in (0, 1, None):
+        fresh = solve([last])
+        for before in ([0], [1], [None], [0, None], [1, 0]):
+            assert solve(before + [last]) == fresh, (before, last)
