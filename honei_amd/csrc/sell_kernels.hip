@@ -21,6 +21,8 @@
 #include "ell_device.hh"
 #include "hip_common.hh"
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 namespace honei {
@@ -31,7 +33,7 @@ constexpr int kSellC = 64;          // rows per slice
 constexpr int kSellWindow = 2048;   // rows sorted together
 constexpr int kSellKeys = 64;       // sort keys: lengths 0..62 and 63+ (longer rows share the last key)
 constexpr int kSellChunks = kSellWindow / kSellC;
-constexpr int kSellStaged = 512;    // threads of the staged product
+constexpr int kSellStaged = 1024;   // threads of the staged product
 
 // perm / len of window blockIdx.x: rows by key descending, ties by row index
 // (a counting sort; ranks from wavefront ballots, so the order is fixed).
@@ -209,24 +211,27 @@ __global__ __launch_bounds__(1024) void k_sell_ranges(const int32_t *__restrict_
     }
 }
 
-// y = A x with x staged in LDS: one 512-thread work-group per sort window (32
-// slices, four per wavefront: one of each eight, so that every wavefront has
-// long and short ones).  The window's column range of x is copied into LDS
-// once (coalesced); each wavefront streams its slices one after the other,
-// the next eight slots' index and value loads issued before this eight's sums
-// (into the next slice, too), and gathers x from LDS.  Slots past a slice's
-// width are asked for outside its buffer (no memory access).  The terms and
-// their order are k_sell_spmv's, so y has the same bits; a window wider than
-// `cap` entries, or a row with an entry outside the recorded range, sums that
-// row from global x instead.
-// Bound by memory once the loads run ahead: a work-group waits four times (its
-// slices' widths, x's range, x, the first slots) before it streams, so two of
-// them share a CU (2 x 80 KiB of doubles at +-4096 columns) and eight slots of
-// each lane are always on their way.  Rows of 1 .. 27 entries within +-4096
-// columns, 2 10^6: FP64 88 -> 77 us (4.8 TB/s), FP32 70 -> 50; 100,003: 23.8 ->
-// 15.9, 21.8 -> 12.8, where two slices per wavefront of 1024 threads waited
-// for every eight or four slots.  Both slices side by side with sixteen slots
-// on their way took 94 (one work-group a CU); twelve slots took 78.
+// y = A x with x staged in LDS: one 1024-thread work-group per sort window (32
+// slices, two per wavefront: one of each sixteen, so that every wavefront has a
+// long and a short one).  The window's column range of x is copied into LDS
+// once (coalesced); each wavefront streams its slices one after the other, the
+// next four slots' index and value loads issued before this four's sums (into
+// the next slice, too), and gathers x from LDS.  Slots past a slice's width are
+// asked for outside its buffer (no memory access), and at most one of them is
+// summed over.  The terms and their order are k_sell_spmv's, so y has the same
+// bits; a window wider than `cap` entries, or a row with an entry outside the
+// recorded range, sums that row from global x instead, with nothing loaded
+// ahead.
+// Bound by memory once the loads run ahead; before that a work-group waits
+// three times (its slices' widths with the window's range, x with the first
+// slots, the sums), which few windows do not hide.  Rows of 1 .. 27 entries
+// within +-4096 columns, 2 10^6: FP64 86 -> 74 us (5.0 TB/s), FP32 70 -> 48;
+// 100,003: 24.1 -> 14.5, 21.7 -> 10.3, where slices of eight (FP64 four) slots
+// a step each waited for its own loads.  Rows of nine entries, FP64: 2 10^6
+// 52.9 -> 48.2, 2001 (one window) 6.5 and 6.5.  Eight slots a step (70 and more
+// registers: fewer wavefronts, more slots past a narrow slice's width): 78 and
+// 56 at 2 10^6, 8.1 at 2001; work-groups of 512 threads with four slices a
+// wavefront, eight slots: 76, 53.6, 8.7; four slots: 75, 48.7, 7.7.
 template <typename VT>
 __global__ __launch_bounds__(kSellStaged, 4) void k_sell_spmv_staged(
     const int32_t *__restrict__ sAj, const VT *__restrict__ sAx, const int32_t *__restrict__ perm,
@@ -235,10 +240,12 @@ __global__ __launch_bounds__(kSellStaged, 4) void k_sell_spmv_staged(
     int64_t cap) {
     extern __shared__ unsigned char sell_stage_raw[];
     VT *win = reinterpret_cast<VT *>(sell_stage_raw);
-    constexpr int W = kSellStaged / kWave, N = kSellChunks / W, U = 8;   // wavefronts, slices of each, slots a step
+    constexpr int W = kSellStaged / kWave, N = kSellChunks / W, U = 4;   // wavefronts, slices of each, slots a step
     constexpr int kWidest = 1 << 20;                                     // 32-bit offsets into a slice
     const int64_t wdw = xcd_block(blockIdx.x, gridDim.x);                // neighbouring windows on one XCD
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int32_t lo = ranges[2 * wdw], hi = ranges[2 * wdw + 1];
+    const int64_t wn = (int64_t)hi - (int64_t)lo + 1;
     int64_t sl[N], b[N];
     int w[N];
     uint32_t l[N];
@@ -268,40 +275,61 @@ __global__ __launch_bounds__(kSellStaged, 4) void k_sell_spmv_staged(
     };
     int32_t j[U], jn[U];
     VT v[U], vn[U];
-    load(0, 0, j, v);
-    const int32_t lo = ranges[2 * wdw], hi = ranges[2 * wdw + 1];
-    const int64_t wn = (int64_t)hi - (int64_t)lo + 1;
-    const bool staged = hi >= lo && wn <= cap;
-    if (staged) {
-        constexpr int C = 10;   // loads of the copy in flight
-        for (int i0 = threadIdx.x; i0 < (int)wn; i0 += C * kSellStaged) {
+    const bool copied = hi >= lo && wn <= cap;   // the same for the work-group
+    const bool staged = copied && narrow;        // for the wavefront
+    if (staged) load(0, 0, j, v);
+    if (copied) {
+        // `count` entries of the copy in flight; the last of them may be past the end
+        auto copy = [&](int i0, auto count) {
+            constexpr int C = decltype(count)::value;
             VT c[C];
 #pragma unroll
-            for (int i = 0; i < C; ++i) c[i] = x[lo + min(i0 + i * kSellStaged, (int)wn - 1)];
+            for (int i = 0; i < C; ++i) c[i] = x[lo + min(i0 + i * kSellStaged + (int)threadIdx.x, (int)wn - 1)];
 #pragma unroll
-            for (int i = 0; i < C; ++i)
-                if (i0 + i * kSellStaged < (int)wn) win[i0 + i * kSellStaged] = c[i];
+            for (int i = 0; i < C; ++i) {
+                const int at = i0 + i * kSellStaged + (int)threadIdx.x;
+                if (at < (int)wn) win[at] = c[i];
+            }
+            return i0 + C * kSellStaged;
+        };
+        for (int i0 = 0; i0 < (int)wn;) {
+            const int left = ((int)wn - i0 + kSellStaged - 1) / kSellStaged;
+            if (left > 4)
+                i0 = copy(i0, std::integral_constant<int, 10>());
+            else if (left > 2)
+                i0 = copy(i0, std::integral_constant<int, 4>());
+            else
+                i0 = copy(i0, std::integral_constant<int, 2>());
         }
     }
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < N; ++h) {
         VT acc = VT(0);
-        bool outside = !staged || !narrow;
-        if (staged && narrow) {
+        bool outside = !staged;
+        if (staged) {
             for (int k0 = 0;;) {
                 const bool last = k0 + U >= w[h];
                 if (!last)
                     load(h, k0 + U, jn, vn);
                 else if (h + 1 < N)
                     load(h + 1 < N ? h + 1 : h, 0, jn, vn);
+                auto add = [&](auto count) {
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const uint32_t o = (uint32_t)(j[u] - lo);
-                    const bool in = o < (uint32_t)wn, use = (uint32_t)(k0 + u) < l[h];
-                    outside |= use && !in;
-                    acc = use ? acc + v[u] * win[in ? o : 0u] : acc;
-                }
+                    for (int u = 0; u < decltype(count)::value; ++u) {
+                        const uint32_t o = (uint32_t)(j[u] - lo);
+                        const bool in = o < (uint32_t)wn, use = (uint32_t)(k0 + u) < l[h];
+                        outside |= use && !in;
+                        acc = use ? acc + v[u] * win[in ? o : 0u] : acc;
+                    }
+                };
+                const int left = w[h] - k0;   // the same for the wavefront
+                if (left > U / 2)
+                    add(std::integral_constant<int, U>());
+                else if (left > U / 4)
+                    add(std::integral_constant<int, U / 2>());
+                else
+                    add(std::integral_constant<int, U / 4>());
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     j[u] = jn[u];
