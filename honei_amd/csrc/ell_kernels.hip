@@ -287,21 +287,31 @@ __global__ __launch_bounds__(1024) void k_product_staged(const int32_t *__restri
 // columns are scattered, ell_row_kernel is bound by its gathers: each takes a
 // cache line of its own from L2, and four of them at a time wait for the
 // indices before them.  Here a work-group looks at the first entries of its
-// rows.  Scattered: the whole row's indices go to registers, the column window
-// of the work-group follows from them, x is copied into LDS once (coalesced)
-// and gathered from there; a window too wide for it is gathered from global
-// memory.  Not scattered: rows in steps of eight entries, the next step's
-// indices loaded ahead.  Entries past a row's end are asked for outside the
-// buffer (no memory access), so no load sits behind a branch.  The sum is
-// ell_lane_sum's, term for term.
-// Rows of 1 .. 27 entries within +-4096 columns: 10^6 rows 90 -> 50 us (216 MB
-// of padded streams, 4.3 TB/s), 120,000 12.1 -> 9.8.  27-point stencil of
-// 100^3: 37.5 -> 35.6; 25 points of 1000^2: 33.7 -> 34.0.
+// rows.  Scattered, and more than eight entries a row: the whole row's indices
+// go to registers, the column window of the work-group follows from them, x is
+// copied into LDS once (coalesced) and gathered from there; a window too wide
+// for it is gathered from global memory.  Else: rows in steps of eight entries,
+// the next step's indices loaded ahead, lanes past their row's end gathering a
+// column that the wavefront has anyway.  Entries past a row's end are asked for
+// outside the buffer (no memory access), so no load sits behind a branch.  The
+// sum is ell_lane_sum's, term for term.
+// Rows of 1 .. 27 entries within +-4096 columns: 10^6 rows 90 -> 49 us (216 MB
+// of padded streams, 4.4 TB/s), 120,000 12.1 -> 9.8.  27-point stencil of
+// 100^3: 37.5 -> 35.6; 25 points of 1000^2: 33.8 -> 33.0.  Against
+// ell_row_kernel over widths 17 to 28, 98,305 to 10^6 rows: all rows full,
+// scattered 0.49 to 0.92 of its time, else 0.7 to 1.1; slower where the width
+// says little about the rows: none of more than three entries 1.0 to 1.28, one
+// in a hundred 0.9 to 1.25, 1 .. width consecutive columns 0.85 to 1.25 (10^6
+// rows 1.0).  (Without the rule of eight entries rows of up to three scattered
+// entries took 2.0, the copy of x being most of the work; with a line for each
+// idle lane 1.8; with idle lanes switched off instead, full rows 1.1.)
 // Doubles stay with ell_row_kernel: the window and the row leave four
 // wavefronts a SIMD, which took 121 -> 69 us on scattered rows but 62 -> 68 on
-// the 27-point stencil; so do rows of more than 28 entries (regular ones 14.0
-// -> 15.2 at 300,000 rows), of 16 and fewer (nothing gained where regular),
-// and fewer rows than kRowsMin (65,537: 4.6 -> 6.3, too few work-groups).
+// the 27-point stencil; so do bf16 values (25 points of 1000^2 27.3 -> 28.9),
+// rows of more than 28 entries (regular ones 14.0 -> 15.2 at 300,000 rows), of
+// 16 and fewer (nothing gained where regular), and fewer rows than kRowsMin
+// (65,537: 4.6 -> 6.3, too few work-groups).  Scattered rows of those widths
+// and types have not been measured but for the doubles.
 constexpr int kRowsBlock = 512;
 constexpr int kRowsWindow = 9216;   // entries of x: 36 KiB, four work-groups a CU
 constexpr int64_t kRowsMin = 98304;
@@ -311,7 +321,7 @@ template <int LEAST, int NC>
 __global__ __launch_bounds__(kRowsBlock, 6) void k_product_rows(KArgs a) {
     constexpr int P = 8, U = 8;   // entries looked at first; entries a step
     __shared__ float win[kRowsWindow];
-    __shared__ int32_t red[4][kRowsBlock / kWave];
+    __shared__ int32_t red[3][kRowsBlock / kWave];
     const float *__restrict__ x = (const float *)a.x;
     const int64_t row = a.row_start + xcd_block(blockIdx.x, gridDim.x) * kRowsBlock + threadIdx.x;
     const uint32_t len = row < a.row_end ? a.Arl[row] : 0u;
@@ -340,19 +350,20 @@ __global__ __launch_bounds__(kRowsBlock, 6) void k_product_rows(KArgs a) {
         pairs += __popcll(__ballot(both));
         far += __popcll(__ballot(both && (d > 32 || d < -32)));
     }
-    if (lane == 0) {
-        red[0][wv] = far;
-        red[1][wv] = pairs;
-    }
-    __syncthreads();
-    far = pairs = 0;
+    // the wavefront's vote, and the entries of its rows, in eights
+    int eights = 0;
 #pragma unroll
-    for (int w = 0; w < kRowsBlock / kWave; ++w) {
-        far += red[0][w];
-        pairs += red[1][w];
-    }
+    for (int k = P / 2; k < NC; k += P) eights += __popcll(__ballot((uint32_t)k < len));
+    if (lane == 0) red[0][wv] = eights + (2 * far > pairs ? 1 << 16 : 0);
+    __syncthreads();
+    int32_t votes = 0;
+#pragma unroll
+    for (int w = 0; w < kRowsBlock / kWave; ++w) votes += red[0][w];
+    votes = __builtin_amdgcn_readfirstlane(votes);
     float s = 0.0f;
-    if (2 * far > pairs) {   // the same for the whole work-group
+    // the same for the whole work-group: half of its wavefronts are scattered,
+    // and its rows have more than the eight entries that are here already
+    if ((votes >> 16) * 2 * kWave >= kRowsBlock && (votes & 0xffff) > kRowsBlock) {
 #pragma unroll
         for (int k = P; k < NC; ++k) index(k);
         int32_t lo = INT32_MAX, hi = INT32_MIN;
@@ -367,15 +378,17 @@ __global__ __launch_bounds__(kRowsBlock, 6) void k_product_rows(KArgs a) {
             hi = oh > hi ? oh : hi;
         }
         if (lane == 0) {
-            red[2][wv] = lo;
-            red[3][wv] = hi;
+            red[1][wv] = lo;
+            red[2][wv] = hi;
         }
         __syncthreads();
 #pragma unroll
         for (int w = 0; w < kRowsBlock / kWave; ++w) {
-            lo = red[2][w] < lo ? red[2][w] : lo;
-            hi = red[3][w] > hi ? red[3][w] : hi;
+            lo = red[1][w] < lo ? red[1][w] : lo;
+            hi = red[2][w] > hi ? red[2][w] : hi;
         }
+        lo = __builtin_amdgcn_readfirstlane(lo);   // the same in every lane
+        hi = __builtin_amdgcn_readfirstlane(hi);
         const int64_t width = (int64_t)hi - lo + 1;
         const bool staged = width <= kRowsWindow;
         if (staged) {
@@ -413,10 +426,13 @@ __global__ __launch_bounds__(kRowsBlock, 6) void k_product_rows(KArgs a) {
             for (int u = 0; u < U && k0 + u < NC; ++u) s = (uint32_t)(k0 + u) < len ? s + av[u] * xv[u] : s;
         }
     } else {
+        // lanes past their row's end gather one column of the wavefront's: a
+        // line, not one each
+        const uint64_t rows = __ballot(len > 0);
+        const int32_t some = __builtin_amdgcn_readlane(j[0], rows ? __builtin_ctzll(rows) : 0);
         int32_t jj[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) jj[u] = j[u];
-        const int32_t some = j[0];   // a column of the row
         for (uint32_t k0 = 0; k0 < len; k0 += U) {
             float av[U], xv[U];
 #pragma unroll

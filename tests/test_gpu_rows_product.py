@@ -81,3 +81,58 @@ def test_first_two_rows_of_a_wavefront(pattern):
     dx, dy = H.DeviceArray.from_host(x), H.DeviceArray(n, np.float32)
     H.DeviceEll.from_oracle(A).product(dy, dx)
     assert np.array_equal(dy.get(), oracle.product(A, x), equal_nan=True)
+
+
+def test_columns_beyond_a_buffer():
+    """Columns on both sides of 2^29 and 2^30 (x of 4 GiB and more): byte
+    offsets of more than 31 and 32 bits."""
+    n, width = MIN_ROWS + 70, 18
+    starts = [0, 2 ** 29 - 2048, 2 ** 30 - 2048, 2 ** 30 + 4096]
+    cols = starts[-1] + 4096
+    stride = 32 * ((n + 31) // 32)
+    r = np.arange(n)
+    first = np.array(starts)[r // 256 % 4] + r % 3000
+    col = first + np.arange(width)[:, None]
+    rng = np.random.default_rng(1)
+    length = rng.integers(width - 3, width + 1, n)
+    used = np.arange(width)[:, None] < length
+    Aj, Ax = np.zeros((width, stride), np.uint64), np.zeros((width, stride), np.float32)
+    Aj[:, :n] = np.where(used, col, 0)
+    Ax[:, :n] = np.where(used, rng.standard_normal((width, n)), 0).astype(np.float32)
+    dx, dy = H.DeviceArray(cols, np.float32), H.DeviceArray(n, np.float32)
+    dx.zero()
+    want = np.zeros(n, np.float32)
+    pieces = [rng.standard_normal(4096).astype(np.float32) for _ in starts]
+    for c0, p in zip(starts, pieces):
+        H.call("honei_hip_upload", H._p(dx.ptr + 4 * c0), p.ctypes.data_as(H._p), p.nbytes, None)
+    xv = np.array(pieces)[r // 256 % 4, (r % 3000) + np.arange(width)[:, None]]
+    for k in range(width):
+        want = np.where(k < length, want + Ax[k, :n] * xv[k], want)
+    D = H.DeviceEll(n, cols, stride, width, 1, Aj.reshape(-1), Ax.reshape(-1), length.astype(np.uint64), H.F32)
+    D.product(dy, dx)
+    assert np.array_equal(dy.get(), want)
+
+
+@pytest.mark.parametrize("entries", [8, 9])
+@pytest.mark.parametrize("scattered", [3, 4, 8])
+def test_mixed_work_groups(scattered, entries):
+    """Work-groups in which some of the eight wavefronts are scattered, with
+    rows on either side of the length from which x is copied; lengths differ
+    within a wavefront (0 .. 2 entries, as many of as many more)."""
+    n, width = MIN_ROWS + 300, 20
+    rng = np.random.default_rng(scattered * 10 + entries)
+    stride = 32 * ((n + 31) // 32)
+    r = np.arange(n)
+    length = np.where(r % 2 == 0, entries, np.where(r % 4 == 1, rng.integers(0, 3, n), 2 * entries))
+    wave = r // 64 % 8 < scattered
+    col = np.where(wave, rng.integers(0, 6000, (width, n)), r % 3000 + np.arange(width)[:, None])
+    used = np.arange(width)[:, None] < length
+    Aj, Ax = np.zeros((width, stride), np.uint64), np.zeros((width, stride), np.float32)
+    Aj[:, :n] = np.where(used, col, 6000)
+    Ax[:, :n] = np.where(used, rng.standard_normal((width, n)), 0).astype(np.float32)
+    A = oracle.Ell(n, 6001, stride, width, 1, Aj.reshape(-1), Ax.reshape(-1), length.astype(np.uint64))
+    x = rng.standard_normal(6001).astype(np.float32)
+    x[6000] = np.nan   # padding only
+    dx, dy = H.DeviceArray.from_host(x), H.DeviceArray(n, np.float32)
+    H.DeviceEll.from_oracle(A).product(dy, dx)
+    assert np.array_equal(dy.get(), oracle.product(A, x))
