@@ -1384,7 +1384,7 @@ hipError_t b_dir_spmv(const BClassTab &tab, const BWork &w, int64_t max_tiles, c
             return hipErrorInvalidValue;
     }
     // a wavefront per tile from one a SIMD on (tile launch / march in us: 648
-    // tiles 18.3 / 17.3, 960 16.4 / 17.0, 1350 22.5 / 19.4, 12,600 179 / 127;
+    // tiles 18.3 / 17.3, 960 16.4 / 17.0, 1350 22.5 / 19.4, 12,600, in an iteration, 179 / 127;
     // below, the march's 32 rows one after the other: 137 tiles 8 / 16)
     if (mf && max_tiles >= kDirMarchTiles) return b_dir_march(tab, w, max_tiles, sc, s);
     const int threads = kPairTileRows * kWave;

@@ -156,9 +156,11 @@ __device__ inline int block_uniform_flag(const int *flag) {
 
 // Cross-block reduction slots.  A reducing kernel stores one partial per
 // block with a plain store; a one-block finisher launched behind it sums the
-// partials in a fixed order.  (A last-block-arrives scheme would need an
-// agent-scope release per block, which on MI355X writes back the XCD's L2 --
-// far more expensive than the extra launch.)
+// partials in a fixed order.  (A last-block-arrives scheme over plain stores
+// would need an agent-scope release per block, which on MI355X writes back the
+// XCD's L2 -- far more expensive than the extra launch.  Relaxed agent-scope
+// words, as cg_resident.hip posts its partials, need no release; that has not
+// been tried here.)
 struct ReduceSlots {
     double *partials;      // [capacity][lanes]
     unsigned int *counter; // unused by the partial/finisher scheme; kept zero

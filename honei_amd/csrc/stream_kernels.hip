@@ -338,7 +338,9 @@ void stream_pair(int pair, dim3 grid, hipStream_t s, const BWork &w, const Strea
 // the tile kernel's thread i holds rows i and i + 16 of the tile, its sixteen
 // wavefronts' sums are added as one more wavefront's lanes.  Bound by memory:
 // 36 bytes a node, 256 systems of five sizes (17.9 10^6 nodes) 179 -> 127 us
-// (5.1 TB/s): no barriers, every wavefront with three rows' loads on their way.
+// (5.1 TB/s; 127 to 135 over a solve): no barriers, every wavefront with three
+// rows' loads on their way.  That is in an iteration, where the launches before
+// leave z and p in the memory-side cache; repeated by itself 151 to 162.
 template <typename Z>
 __global__ __launch_bounds__(256, 4) void k_b_dir_march(BClassTab tab, BWork w, const SlotScalars *sc) {
     constexpr int T = kPairTileRows, TR = T * kDirNodes, D = 3;   // rows of a tile with its halo, rows in flight

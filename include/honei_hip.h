@@ -446,8 +446,9 @@ int honei_hip_fill_lognormal(double *dst_dev, size_t n, double sigma, uint64_t s
  * iters_per_launch outer iterations of every active slot; slots retire on
  * the device when ||b - A x|| < tolerance * ||b - A x0||, where x0 is zero
  * with the first row, last row and first column of the grid set to b.
- * autotune: threads-per-row T in {1,2,4} and block size per level picked by
- * timing (cached for the process); 0 uses T = 1, block 256, which with
+ * autotune: threads-per-row T in {1,2,4} (1 on levels that the coarse launch
+ * can take) and block size per level picked by timing (cached for the
+ * process); 0 uses T = 1, block 256, which with
  * outer_method 0 makes each slot bit-identical to honei_hip_mg_solve_mixed
  * with n_max_iter 1, initial_zero, zero_inner_start and post sweeps = pre
  * sweeps.  The batch
@@ -472,9 +473,10 @@ typedef struct {
     int32_t use_graphs;        /* 1 (default): a step is one hipGraph launch; 0: the same kernels
                                   enqueued directly at every step (same results; for profilers
                                   that cannot follow graph launches) */
-    int32_t pair_sweeps;       /* 1 (default): on levels of 33^2 nodes and up, Jacobi0 + defect and
-                                  the two post-smoothing sweeps each run as one launch that reads
-                                  the matrix once (n_pre == 2, n_post == 2; same results) */
+    int32_t pair_sweeps;       /* 1 (default): on levels of 33^2 nodes and up that the coarse launch
+                                  does not take, Jacobi0 + defect and the two post-smoothing sweeps
+                                  each run as one launch that reads the matrix once (n_pre == 2,
+                                  n_post == 2; same results) */
     int32_t matrix_free;       /* where those paired launches and the FP64 outer row sums take
                                   each row's weights (same results in every form): 0 the nine
                                   stored values; 1 (default) formed from the slot's cell
@@ -538,8 +540,8 @@ int honei_hip_batch_run(void *batch, int64_t *launches);
  * batch (microseconds, else 0) and that batch's slot count.                */
 int honei_hip_batch_shape(void *batch, int32_t level, int32_t *threads, int32_t *block, int32_t *group,
                           double *sweep_us, int64_t *tune_slots);
-/* Levels that run the paired launches (pair_sweeps, levels of 33^2 nodes and
- * up): the autotuner's measured time of one paired Jacobi0 + defect launch
+/* Levels of 33^2 nodes and up with pair_sweeps (those that the coarse launch
+ * takes among them: what the paired launches would take there): the autotuner's measured time of one paired Jacobi0 + defect launch
  * (matrix_free 1: with the restriction in it) and of one paired two-sweep
  * launch over the same tuning batch (microseconds; 0 when the level is not
  * paired or not tuned).                                                    */
